@@ -452,12 +452,31 @@ __device__ __forceinline__ StepOut particle_step(const MeshDev& mesh, const Step
   o.Fy = Fy;
   o.Sx = Sx;
   o.Sy = Sy;
-  double px = xn, py = yn, dth = 0.0;
+  double px = xn, py = yn;
   const bool finite = isfinite(xn) && isfinite(yn) && isfinite(thn);
   if (!finite) o.fl |= kFlagNonfinite;
-  else if (!seam_wrap_group<LANES, WAVE>(me.x, me.y, px, py, dth, prm.max_crossings, lane, &o.q)) o.fl |= kFlagTiling;
+  const bool leaves = finite && !inside_unit(px, py);
+  bool folded = false;
+  if (leaves) folded = seam_fold(me.x, me.y, px, py, thn, prm.max_crossings, &o.q);
+  const bool loop = leaves && !folded;  // rare: the closed form does not settle the move
+  double dth = 0.0;
+  if constexpr (WAVE) {  // every lane of the wave goes along, so that all 64 can take the last flight
+    if (__builtin_amdgcn_ballot_w64(loop) != 0) {
+      double lx = loop ? px : 0.5, ly = loop ? py : 0.5;
+      int q = 0;
+      const bool good = seam_wrap_group<LANES, true>(me.x, me.y, lx, ly, dth, prm.max_crossings, lane, &q);
+      if (loop) {
+        px = lx;
+        py = ly;
+        o.q = q;
+        if (!good) o.fl |= kFlagTiling;
+      }
+    }
+  } else if (loop) {
+    if (!seam_wrap_group<LANES, false>(me.x, me.y, px, py, dth, prm.max_crossings, lane, &o.q)) o.fl |= kFlagTiling;
+  }
+  if (finite && !folded) thn = wrap_heading(thn + dth);
   if (finite && !inside_unit(px, py)) o.fl |= kFlagLost;
-  if (finite) thn = wrap_heading(thn + dth);
   o.xo = (float)px;
   o.yo = (float)py;
   o.to = (float)thn;

@@ -506,6 +506,52 @@ __device__ inline bool seam_wrap_group(double ax, double ay, double& px, double&
 // heading kept in [-pi, pi)
 __host__ __device__ inline double wrap_heading(double t) { return t - 2.0 * kPi * floor((t + kPi) / (2.0 * kPi)); }
 
+// The same result in closed form. Every crossing maps the end point by a quarter turn about (0, 0)
+// (left, down, and the fall-through) or about (1, 1) (right, up), so the end point never leaves its
+// orbit under the group those turns generate: the translations by 2 along each axis and the quarter
+// turns about the corners (the wallpaper group p4), of which the open unit square is a fundamental
+// domain. The loop stops inside the square, so it stops at the orbit's one point there and with
+// the one rotation that leads there, whatever borders it crossed and however the snapping of exit
+// points bent its path: fold the point into [0, 2)^2 and apply the map of the quadrant it lies in.
+// What does depend on the path is the rounding of the end point's images (a few ulps of its largest
+// coordinate) and of the heading's running sum (up to half an ulp of the sum per crossing, so about
+// the square of the crossings). Both are far below the FP32 resolution of the step's state, so the
+// fold is taken exactly when the FP32 position and heading are the same anywhere within those
+// bounds; otherwise (false; px, py and heading untouched) the caller runs the loop. Also refused:
+// images within 1e-9 of the square's border, where the representative is not unique, and flights
+// that might exceed the crossing bound: over 1.08e9 random flights on and off edges and corners the
+// loop took at most 3.5 (|dx| + |dy| + 4) crossings, and its results lay within 0.12 of the position
+// bound and 0.45 of the heading bound (the latter sets how often a flight is refused, a few in 10,000
+// at 200 crossings).
+// A crossing of the loop costs about 0.6 us of a wave's time, one after the other, and the longest
+// flight of a step bounds the step; the closed form is some 60 instructions for any length (MI355X, per
+// step: 2,000 particles 18.7 -> 12.6 us, 100,000 particles with flights of up to 500 crossings
+// 277 -> 161 us, 256 replicas of 100 to 4,000 particles 212 -> 189 us).
+// heading: theta' before the wrap, in: unwrapped, out: rotated and kept in [-pi, pi).
+__host__ __device__ inline bool seam_fold(double ax, double ay, double& px, double& py, double& heading,
+                                          int max_crossings, int* quarter_out) {
+  const double len = fabs(px - ax) + fabs(py - ay) + 16.0;
+  const double X = px - 2.0 * floor(0.5 * px), Y = py - 2.0 * floor(0.5 * py);
+  const bool right = X > 1.0, up = Y > 1.0;
+  const double u = right ? 2.0 - X : X, v = up ? 2.0 - Y : Y;
+  const bool odd = right != up;  // a quarter turn: the coordinates change places
+  const double x = odd ? (up ? v : Y) : u, y = odd ? (up ? X : u) : v;
+  const int quarter = odd ? (up ? 1 : 3) : (right ? 2 : 0);
+  const double t = wrap_heading(heading + (odd ? (up ? 0.5 * kPi : -0.5 * kPi) : (right ? kPi : 0.0)));
+  const double far = fmax(fmax(fabs(px), fabs(py)), 2.0);
+  const double bp = 0x1p-50 * far;                                        // of the position
+  const double bt = 3e-16 * (len * len) + 0x1p-49 * fabs(heading);        // of the heading
+  const int inside = (int)(x > 1e-9) & (int)(x < 1.0 - 1e-9) & (int)(y > 1e-9) & (int)(y < 1.0 - 1e-9);
+  const int sure = (int)((float)(x - bp) == (float)(x + bp)) & (int)((float)(y - bp) == (float)(y + bp)) &
+                   (int)((float)(t - bt) == (float)(t + bt)) & (int)(t - bt >= -kPi) & (int)(t + bt < kPi);
+  if (!(inside & sure & (int)(4.0 * len <= (double)max_crossings))) return false;
+  px = x;
+  py = y;
+  heading = t;
+  *quarter_out = quarter;
+  return true;
+}
+
 // ------------------------------------------------------------------ point location
 
 template <class T>

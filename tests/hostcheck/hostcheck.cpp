@@ -100,6 +100,17 @@ void hc_seam_wrap_passes_many(int n, const double* a, const double* p, int max_c
   }
 }
 
+// the closed form of the seam wrap (seam_fold): settled[i] = 1 and p, heading (in and out), quarter
+// where it settles the move, 0 and everything untouched where it leaves it to the loop
+void hc_seam_fold_many(int n, const double* a, double* p, double* heading, int max_crossings, int* settled,
+                       int* quarter) {
+  for (int i = 0; i < n; ++i)
+    settled[i] = tdev::seam_fold(a[2 * i], a[2 * i + 1], p[2 * i], p[2 * i + 1], heading[i], max_crossings, quarter + i)
+                     ? 1 : 0;
+}
+
+double hc_wrap_heading(double t) { return tdev::wrap_heading(t); }
+
 void hc_seam_wrap_quarter_many(int n, const double* a, const double* p, int max_crossings, int* quarter) {
   for (int i = 0; i < n; ++i) {
     double px = p[2 * i], py = p[2 * i + 1], dt = 0.0;
