@@ -159,7 +159,8 @@ static_assert(32 % kScanChunk == 0, "scan chunks must tile the 32-entry window")
 // buckets' occupancy mask is staged in LDS by the workgroup: the table walk tests occupancy there
 // and touches a bucket in global memory only when its vertex holds particles; without it the walk
 // reads each entry's bucket count. Both visit the same buckets in the same order.
-template <bool OCC>
+// SORTED: the buckets are known to be sorted (the kernels of crowded systems).
+template <bool OCC, bool SORTED = false>
 struct GlobalSource {
   static constexpr bool kOcc = OCC;
   BucketsIn b;
@@ -178,6 +179,7 @@ struct GlobalSource {
     return h;
   }
   __device__ __forceinline__ int count(int w) const { return b.count[w]; }
+  // the particles of bucket w in ascending id order, without (each) and with (each_pos) their state
   template <class F>
   __device__ __forceinline__ void each(int w, const Head& h, F&& f) const {
     if (h.c == 0) return;
@@ -189,6 +191,45 @@ struct GlobalSource {
       return;
     }
     for_bucket(b, w, f);
+  }
+  template <class F>
+  __device__ __forceinline__ void each_pos(int w, const Head& h, F&& f) const {
+    if constexpr (!SORTED) {
+      each(w, h, [&](int j) { f(j, pos(j)); });
+    } else {
+      const int c = h.c;
+      if (c == 0) return;
+      if (c <= 2) {  // ids in the head
+        const int j1 = c == 2 ? h.s1 : h.s0;
+        const float4 q0 = pos(h.s0), q1 = pos(j1);
+        f(h.s0, q0);
+        if (c == 2) f(j1, q1);
+        return;
+      }
+      // kBatch particles at a time: the next ids and all of a batch's states are in flight together.
+      // One at a time, two dependent loads per particle, a lane with a few crowded vertices (up to
+      // 60 particles each) walked 100 us by itself and bounded the 100,000-particle step.
+      constexpr int kBatch = 8;
+      const int* ids = c <= kSlots ? b.slot + (size_t)w * kSlots : b.big + h.s0;
+      int id[kBatch];
+#pragma unroll
+      for (int k = 0; k < kBatch; ++k) id[k] = ids[k < c ? k : c - 1];
+      for (int q0 = 0; q0 < c; q0 += kBatch) {
+        float4 q[kBatch];
+        int nx[kBatch];
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k) q[k] = pos(id[k]);
+        if (q0 + kBatch < c) {
+#pragma unroll
+          for (int k = 0; k < kBatch; ++k) nx[k] = ids[q0 + kBatch + k < c ? q0 + kBatch + k : c - 1];
+        }
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k)
+          if (q0 + k < c) f(id[k], q[k]);
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k) id[k] = nx[k];
+      }
+    }
   }
   __device__ __forceinline__ float4 pos(int j) const { return xycs[j]; }
   __device__ __forceinline__ float theta(int j) const { return th[j]; }
@@ -233,6 +274,10 @@ struct LdsSource {
       prev = best;
     }
   }
+  template <class F>
+  __device__ __forceinline__ void each_pos(int w, const Head& h, F&& f) const {
+    each(w, h, [&](int j) { f(j, pos(j)); });
+  }
   __device__ __forceinline__ float4 pos(int j) const { return xycs[j]; }
   __device__ __forceinline__ float theta(int j) const { return th[j]; }
 };
@@ -262,8 +307,7 @@ __device__ __forceinline__ StepOut particle_step(const MeshDev& mesh, const Step
     const double dd = d == 0.0f ? 0.001 : (double)d;
     const double g64 = (kc64 * (dd - prm.two_sigma64)) / dd;
     const bool counted = d != 0.0f;
-    src.each(w, h, [&](int j) {
-      const float4 q = src.pos(j);
+    src.each_pos(w, h, [&](int j, const float4& q) __attribute__((always_inline)) {
       if (j != i) {
         Fx64 += g64 * ((double)me.x - (double)q.x);
         Fy64 += g64 * ((double)me.y - (double)q.y);

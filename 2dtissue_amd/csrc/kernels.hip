@@ -116,7 +116,7 @@ __global__ void __launch_bounds__(kStepMaxBlock) k_step_tiled(MeshDev mesh, cons
         if constexpr (VISITS) io.visit[g] = make_int2(-1, 0);
       }
     } else {
-      const GlobalSource<OCC> src{replica_in(bin, r, nv, rep.off), io.xycs_in, io.th_in, s_occ};
+      const GlobalSource<OCC, WAVE> src{replica_in(bin, r, nv, rep.off), io.xycs_in, io.th_in, s_occ};
       const StepOut o = particle_step<LANES, WAVE>(mesh, rep.prm, src, g, me, th, v, eta, lane);
       if (lane == 0) {
         io.xycs_out[g] = make_float4(o.xo, o.yo, o.co, o.so);
