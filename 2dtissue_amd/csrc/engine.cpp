@@ -241,7 +241,6 @@ void Engine::alloc_bucket_set(BucketSet& b) {
   b.slot = dalloc<int>(cells * tdev::kSlots);
   b.ovf_n = dalloc<int>(R);
   b.ovf = dalloc<int2>(ntot);
-  b.multi_n = dalloc<int>(R);
   b.multi = dalloc<int>(ntot);
   b.big_n = dalloc<int>(R);
   b.big = dalloc<int>(ntot);
@@ -249,12 +248,12 @@ void Engine::alloc_bucket_set(BucketSet& b) {
 
 void Engine::free_bucket_set(BucketSet& b) {
   dfree(b.occ); dfree(b.count); dfree(b.slot); dfree(b.ovf_n); dfree(b.ovf);
-  dfree(b.multi_n); dfree(b.multi); dfree(b.big_n); dfree(b.big);
+  dfree(b.multi); dfree(b.big_n); dfree(b.big);
 }
 
 size_t Engine::bucket_set_bytes() const {
   return (size_t)R * md.nv * (1 + tdev::kSlots) * sizeof(int) + (size_t)ntot * (sizeof(int2) + 2 * sizeof(int)) +
-         3 * (size_t)R * sizeof(int) + (size_t)R * tdev::occ_words(md.nv) * sizeof(unsigned);
+         2 * (size_t)R * sizeof(int) + (size_t)R * tdev::occ_words(md.nv) * sizeof(unsigned);
 }
 
 // outside any capture: clear set b (count and list lengths), on stream st (null: the engine's)
@@ -263,7 +262,6 @@ void Engine::clear_bucket_set(BucketSet& b, hipStream_t st) {
   HIP_OK(hipMemsetAsync(b.count, 0, (size_t)R * md.nv * sizeof(int), st));
   HIP_OK(hipMemsetAsync(b.occ, 0, (size_t)R * tdev::occ_words(md.nv) * sizeof(unsigned), st));
   HIP_OK(hipMemsetAsync(b.ovf_n, 0, R * sizeof(int), st));
-  HIP_OK(hipMemsetAsync(b.multi_n, 0, R * sizeof(int), st));
   HIP_OK(hipMemsetAsync(b.big_n, 0, R * sizeof(int), st));
 }
 
@@ -296,7 +294,6 @@ void Engine::rebuild_buckets() {
     HIP_OK(hipMemsetAsync(bs[k].count, 0, cells * sizeof(int), stream));
     HIP_OK(hipMemsetAsync(bs[k].occ, 0, (size_t)R * tdev::occ_words(md.nv) * sizeof(unsigned), stream));
     HIP_OK(hipMemsetAsync(bs[k].ovf_n, 0, R * sizeof(int), stream));
-    HIP_OK(hipMemsetAsync(bs[k].multi_n, 0, R * sizeof(int), stream));
     HIP_OK(hipMemsetAsync(bs[k].big_n, 0, R * sizeof(int), stream));
   }
   bucket_state(vid[sphase], bphase);

@@ -30,12 +30,12 @@ __device__ __forceinline__ void bucket_insert(const BucketsOut& b, int v, int i)
     const int o = atomicAdd(b.ovf_n, 1);
     b.ovf[o] = make_int2(v, i);
   }
-  if (old == 1 && b.multi) b.multi[atomicAdd(b.multi_n, 1)] = v;  // the bucket needs sorting
+  if (b.multi) b.multi[i] = old == 1 ? v : -1;  // the second arrival has the bucket sorted
 }
 
 __device__ __forceinline__ BucketsOut replica_out(const BucketSet& s, int r, int nv, int off) {
-  return {s.count + (size_t)r * nv, s.slot + (size_t)r * nv * kSlots, s.ovf_n + r, s.ovf + off, s.multi_n + r,
-          s.multi ? s.multi + off : nullptr, s.occ + (size_t)r * occ_words(nv)};
+  return {s.count + (size_t)r * nv, s.slot + (size_t)r * nv * kSlots, s.ovf_n + r, s.ovf + off, s.multi,
+          s.occ + (size_t)r * occ_words(nv)};
 }
 
 // orders the LDS / global accesses of one wave (its lanes exchange data through memory)
@@ -97,7 +97,6 @@ __global__ void __launch_bounds__(kStepMaxBlock) k_step_tiled(MeshDev mesh, cons
   const unsigned halt = io.halt_in[r];
   if (tile.q == 0 && tid == 0) {
     bclr.ovf_n[r] = 0;
-    bclr.multi_n[r] = 0;
     bclr.big_n[r] = 0;
     io.halt_clr[r] = 0u;
     if (halt) atomicOr(&io.halt_out[r], halt);
@@ -152,16 +151,18 @@ __global__ void __launch_bounds__(kStepMaxBlock) k_step_tiled(MeshDev mesh, cons
 // crowded buckets up to this many particles are sorted in LDS (larger ones in global memory)
 constexpr int kSortCap = 512;
 
-// Sort every bucket of set bs that holds two or more particles (listed in multi by the insertion).
-// One thread per listed bucket: up to kSlots ids are sorted in place with the register network.
+// Sort every bucket of set bs that holds two or more particles. One thread per particle: the
+// bucket's second arrival (the insertion left the vertex in its entry of multi, -1 in the others)
+// sorts it, up to kSlots ids in place with the register network. (A compact list of such buckets
+// needs a counter, and a returning atomic on one address is served every 12 ns: with 25,000 shared
+// vertices it cost the bucketing of 100,000 particles 300 us by itself.)
 // A crowded bucket (more than kSlots) is then taken by its whole wave: its slots and its entries
 // of the overflow list are gathered (ballot compaction), ranked, and written in ascending order to
 // a fresh range of the replica's big area, whose offset replaces the bucket's first slot.
-// The kernel is a chain of dependent loads, so independent ones are issued together: the list
-// length, the overflow count and the thread's list entry (read speculatively within the
-// replica's range), then a bucket's count and all of its slots, and for a crowded bucket the
-// big-area reservation with the overflow scan. single_n > 0: one replica of single_n particles,
-// whose tiles need not be read (block b covers list entries b * blockDim.x ...).
+// The kernel is a chain of dependent loads, so independent ones are issued together: the overflow
+// count and the particle's entry, then a bucket's count and all of its slots, and for a crowded
+// bucket the big-area reservation with the overflow scan. single_n > 0: one replica of single_n
+// particles, whose tiles need not be read (block b covers particles b * blockDim.x ...).
 __global__ void __launch_bounds__(kStepMaxBlock) k_bucket_finalize(const ReplicaDesc* reps, const TileDesc* tiles,
                                                                    int nv, int single_n, BucketSet bs) {
   __shared__ __align__(16) int lds[kStepMaxBlock / 64][kSortCap];
@@ -175,14 +176,12 @@ __global__ void __launch_bounds__(kStepMaxBlock) k_bucket_finalize(const Replica
     cap = reps[r].n;
     k = tile.q * (int)blockDim.x + tid;
   }
-  const int n_multi = bs.multi_n[r];
   const int novf = bs.ovf_n[r];
-  const int v_listed = k < cap ? bs.multi[off + k] : -1;
+  const int v = k < cap ? bs.multi[off + k] : -1;
   int* slot = bs.slot + (size_t)r * nv * kSlots;
-  int v = -1, c = 0;
+  int c = 0;
   int4 s0 = make_int4(0, 0, 0, 0), s1 = s0;
-  if (k < n_multi) {
-    v = v_listed;
+  if (v >= 0) {
     int* sl = slot + (size_t)v * kSlots;
     s0 = reinterpret_cast<const int4*>(sl)[0];
     s1 = reinterpret_cast<const int4*>(sl)[1];
@@ -529,6 +528,7 @@ hipError_t launch_step_tiled(int lanes, int block, bool tape, bool wave, const M
 
 hipError_t launch_bucket_finalize(int block, const ReplicaDesc* reps, const TileDesc* tiles, int n_tiles, int nv,
                                   int single_n, const BucketSet& bs, hipStream_t st) {
+  if (single_n > 0) n_tiles = cdiv(single_n, block);
   hipLaunchKernelGGL(k_bucket_finalize, dim3(n_tiles), dim3(block), 0, st, reps, tiles, nv, single_n, bs);
   return hipGetLastError();
 }

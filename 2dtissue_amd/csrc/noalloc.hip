@@ -41,7 +41,7 @@ struct Layout {
   static constexpr size_t vid = xycs_out + al(sizeof(float4) * kMaxParticles);
   static constexpr size_t rid = vid + al(sizeof(int) * kMaxParticles);
   // one bucket set: occupancy mask, count[V], slot[V * kSlots], ovf[N] (int2), multi[N], big[N],
-  // counters[3]
+  // counters[2]
   static constexpr size_t set_occ = 0;
   static constexpr size_t set_count = set_occ + al(sizeof(unsigned) * tdev::occ_words(kMaxVertices));
   static constexpr size_t set_slot = set_count + al(sizeof(int) * kMaxVertices);
@@ -49,7 +49,7 @@ struct Layout {
   static constexpr size_t set_multi = set_ovf + al(sizeof(int2) * kMaxParticles);
   static constexpr size_t set_big = set_multi + al(sizeof(int) * kMaxParticles);
   static constexpr size_t set_ctr = set_big + al(sizeof(int) * kMaxParticles);
-  static constexpr size_t set_bytes = set_ctr + al(sizeof(int) * 3);
+  static constexpr size_t set_bytes = set_ctr + al(sizeof(int) * 2);
   static constexpr size_t sets = rid + al(sizeof(int) * kMaxParticles);
   static constexpr size_t partial = sets + 3 * set_bytes;
   static constexpr size_t tiles = partial + al(sizeof(OrderPartial) * kMaxTiles * (tissue::kStepMaxBlock / 64));
@@ -92,8 +92,7 @@ BucketSet set_at(unsigned char* base, int k, int sorted) {
   b.multi = (int*)(s + Layout::set_multi);
   b.big = (int*)(s + Layout::set_big);
   b.ovf_n = ctr;
-  b.multi_n = ctr + 1;
-  b.big_n = ctr + 2;
+  b.big_n = ctr + 1;
   b.sorted = sorted;
   return b;
 }
@@ -149,7 +148,6 @@ __global__ void k_noalloc_setup(SetupArgs a) {
   if (t < 3) {
     a.ctrs[t][0] = 0;
     a.ctrs[t][1] = 0;
-    a.ctrs[t][2] = 0;
     a.rows[t] = 0u;
   }
   if (t == 0) {
