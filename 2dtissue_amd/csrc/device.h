@@ -50,8 +50,8 @@ struct BucketsIn {
 // slots, later ones go to the (vertex, id) overflow list; the second arrival at a vertex also
 // leaves the vertex in its particle's entry of multi (the buckets the finalize pass must sort, -1 in
 // the entries of the other particles; null when no finalize pass
-// follows); the first arrival sets the vertex's bit in the occupancy mask occ (bit v % 32 of word
-// v / 32).
+// follows); where the step's kernels read the occupancy mask occ, the first arrival sets the vertex's
+// bit in it (bit v % 32 of word v / 32).
 struct BucketsOut { int* count; int* slot; int* ovf_n; int2* ovf; int* multi; unsigned* occ; };
 
 // words of a vertex-occupancy mask over nv vertices

@@ -572,6 +572,9 @@ int32_t Engine::run_once(const Shape& s, int n_steps, const float* nz, size_t st
       partial = dalloc<OrderPartial>(need);
       partial_cap = need;
     }
+    const bool occ = stage_occupancy(md.nv, s.block, s.lanes);
+    if (occ && !occ_kept) buckets_stale = true;  // the sets were filled without the masks this shape reads
+    occ_kept = occ;
     if (buckets_stale) rebuild_buckets();
   }
   const auto key = std::make_tuple(n_steps, nz, stride, s.key(), sphase, bphase);

@@ -117,6 +117,7 @@ struct Engine {
   BucketSet bs[3] = {};
   int bphase = 0;  // bucket set holding the current state's buckets
   bool buckets_ready = false, buckets_stale = true;
+  bool occ_kept = false;  // the last run's steps kept the buckets' occupancy masks (stage_occupancy)
   TileDesc* d_tiles = nullptr;
   int* d_tile_begin = nullptr;
   int n_phys = 0, n_logical = 0;

@@ -21,9 +21,10 @@ namespace tissue {
 
 namespace {
 
+template <bool OCC>
 __device__ __forceinline__ void bucket_insert(const BucketsOut& b, int v, int i) {
   const int old = atomicAdd(&b.count[v], 1);
-  if (old == 0) atomicOr(&b.occ[v >> 5], 1u << (v & 31));
+  if (OCC && old == 0) atomicOr(&b.occ[v >> 5], 1u << (v & 31));
   if (old < kSlots) {
     b.slot[(size_t)v * kSlots + old] = i;
   } else {
@@ -89,8 +90,10 @@ __global__ void __launch_bounds__(kStepMaxBlock) k_step_tiled(MeshDev mesh, cons
   // clear this replica's bucket set consumed two steps ago (it is next step's output)
   int* clr = bclr.count + (size_t)r * nv;
   for (int w = tile.q * (int)blockDim.x + tid; w < nv; w += tile.nq * (int)blockDim.x) clr[w] = 0;
-  unsigned* clr_occ = bclr.occ + (size_t)r * nw;
-  for (int k = tile.q * (int)blockDim.x + tid; k < nw; k += tile.nq * (int)blockDim.x) clr_occ[k] = 0u;
+  if constexpr (OCC) {
+    unsigned* clr_occ = bclr.occ + (size_t)r * nw;
+    for (int k = tile.q * (int)blockDim.x + tid; k < nw; k += tile.nq * (int)blockDim.x) clr_occ[k] = 0u;
+  }
   __syncthreads();
   // a replica flagged before this step passes its state through unchanged (the reference stops
   // at the first failure); the flag rows rotate like the bucket sets
@@ -111,7 +114,7 @@ __global__ void __launch_bounds__(kStepMaxBlock) k_step_tiled(MeshDev mesh, cons
         io.xycs_out[g] = me;
         io.th_out[g] = th;
         io.vid_out[g] = v;
-        bucket_insert(bo, v, g);
+        bucket_insert<OCC>(bo, v, g);
         if constexpr (VISITS) io.visit[g] = make_int2(-1, 0);
       }
     } else {
@@ -128,7 +131,7 @@ __global__ void __launch_bounds__(kStepMaxBlock) k_step_tiled(MeshDev mesh, cons
         io.r3z[g] = (float)o.L.Z;
         io.face[g] = o.L.face;
         io.nbr[g] = o.nb;  // count_particle_neighbors (2DTissue.cpp:254-268)
-        bucket_insert(bo, o.L.vid, g);
+        bucket_insert<OCC>(bo, o.L.vid, g);
         if (o.fl) {
           atomicOr(&io.halt_out[r], o.fl);
           atomicMin(&io.first_bad[r], io.step);
@@ -439,7 +442,7 @@ __global__ void k_insert(int ntot, const int* vid, const int* rid, const Replica
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= ntot) return;
   const int r = rid[g];
-  bucket_insert(replica_out(bs, r, nv, reps[r].off), vid[g], g);
+  bucket_insert<true>(replica_out(bs, r, nv, reps[r].off), vid[g], g);
 }
 
 __global__ void k_neighbor_lists(MeshDev mesh, const ReplicaDesc* reps, const int* rid, int ntot, BucketSet bs,

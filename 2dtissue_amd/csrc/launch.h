@@ -119,7 +119,9 @@ constexpr int kStepMaxBlock = 512;
 // loads the whole mask (one word per 32 vertices) before its first particle, which pays when the
 // workgroup holds enough particles per word (measured on MI355X: 256 replicas, 64 particles per
 // workgroup and 324 words, 7 % faster; 2,000 particles at 8 per workgroup, 6 % slower; 100,000
-// particles at 64 per workgroup and 3,134 words, 1 % slower). Results are the same either way.
+// particles at 64 per workgroup and 3,134 words, 1 % slower). Results are the same either way. Only
+// such launches keep the mask up to date: for the others it would be one more memory-side atomic per
+// occupied vertex (63,000 of them in a step of 100,000 particles).
 constexpr int kOccWordsPerParticle = 8;
 inline bool stage_occupancy(int nv, int block, int lanes) {
   return tdev::occ_words(nv) <= kOccWordsPerParticle * (block / lanes);
