@@ -110,11 +110,16 @@ __device__ __forceinline__ float pair_coef(float d, const StepParams& p) {
   return fij / dd;
 }
 
-template <int LANES, class T>
+// sum over the group, in the order of a butterfly from LANES / 2 down; every lane gets it
+template <int LANES, int OFF = LANES / 2, class T>
 __device__ __forceinline__ T group_sum(T v) {
-#pragma unroll
-  for (int off = LANES / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, LANES);
-  return v;
+  if constexpr (OFF >= 1) {
+    T a, b;
+    butterfly<OFF, LANES>(v, a, b);
+    return group_sum<LANES, OFF / 2>(a + b);
+  } else {
+    return v;
+  }
 }
 
 constexpr unsigned kFlagLost = 1u, kFlagNonfinite = 2u, kFlagTiling = 4u;

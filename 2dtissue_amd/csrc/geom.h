@@ -703,14 +703,82 @@ __host__ __device__ inline void merge_best(float& b1, int& f1, float& b2, float 
   }
 }
 
-template <int LANES, class T>
-__host__ __device__ inline T lane_xor(T v, int off) {
+// One level of a butterfly over the LANES lanes of a group: on return lane l holds, in a and b, the
+// values of lanes l and l ^ OFF (which of the two is in a depends on the lane: the level must combine
+// them by a symmetric operation). The levels run from OFF = LANES / 2 down to 1. On the device the
+// values move through the vector unit: DPP within a row of 16 lanes (a rotation by 4 stands for
+// l ^ 4, the level before having made lanes l and l ^ 8 equal), row and half swaps above; a shuffle
+// through the LDS crossbar costs a lone wave about 100 cycles a level, these cost about 10.
+template <int OFF, int LANES>
+__host__ __device__ inline void butterfly_word(uint32_t v, uint32_t& a, uint32_t& b) {
+  static_assert(OFF >= 1 && 2 * OFF <= LANES && LANES <= 64, "level within the group");
+  a = v;
+  b = v;
 #if defined(__HIP_DEVICE_COMPILE__)
-  return __shfl_xor(v, off, LANES);
-#else
-  (void)off;
-  return v;
+  if constexpr (OFF == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    a = r[0];
+    b = r[1];
+  } else if constexpr (OFF == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    a = r[0];
+    b = r[1];
+  } else if constexpr (OFF == 8) {
+    b = __builtin_amdgcn_update_dpp(v, v, 0x128, 0xf, 0xf, false);  // row_ror:8
+  } else if constexpr (OFF == 4 && LANES >= 16) {
+    b = __builtin_amdgcn_update_dpp(v, v, 0x124, 0xf, 0xf, false);  // row_ror:4
+  } else if constexpr (OFF == 4) {  // lanes 0-3 of each 8 take 4-7 (row_shl:4), the others 0-3 (row_shr:4)
+    b = __builtin_amdgcn_update_dpp(v, v, 0x104, 0xf, 0x5, false);
+    b = __builtin_amdgcn_update_dpp(b, v, 0x114, 0xf, 0xa, false);
+  } else if constexpr (OFF == 2) {
+    b = __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xf, 0xf, false);  // quad_perm [2,3,0,1]
+  } else {
+    b = __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xf, 0xf, false);  // quad_perm [1,0,3,2]
+  }
 #endif
+}
+
+template <int OFF, int LANES, class T>
+__host__ __device__ inline void butterfly(T v, T& a, T& b) {
+  static_assert(sizeof(T) == 4 || sizeof(T) == 8, "one or two words");
+  constexpr int W = sizeof(T) / 4;
+  uint32_t w[W], wa[W], wb[W];
+  __builtin_memcpy(w, &v, sizeof v);
+#pragma unroll
+  for (int k = 0; k < W; ++k) butterfly_word<OFF, LANES>(w[k], wa[k], wb[k]);
+  __builtin_memcpy(&a, wa, sizeof a);
+  __builtin_memcpy(&b, wb, sizeof b);
+}
+
+// the lexicographic minimum over the group, and with it the least of the other distances
+template <int OFF, int LANES>
+__host__ __device__ inline void group_merge_best(float& b1, int& f1, float& b2) {
+  if constexpr (OFF >= 1) {
+    float a1, o1, a2, o2;
+    int af, of;
+    butterfly<OFF, LANES>(b1, a1, o1);
+    butterfly<OFF, LANES>(f1, af, of);
+    butterfly<OFF, LANES>(b2, a2, o2);
+    merge_best(a1, af, a2, o1, of, o2);
+    b1 = a1;
+    f1 = af;
+    b2 = a2;
+    group_merge_best<OFF / 2, LANES>(b1, f1, b2);
+  }
+}
+
+template <int OFF, int LANES>
+__host__ __device__ inline void group_lex_min(double& d, int& f) {
+  if constexpr (OFF >= 1) {
+    double a, o;
+    int af, of;
+    butterfly<OFF, LANES>(d, a, o);
+    butterfly<OFF, LANES>(f, af, of);
+    const bool less = lex_less(o, of, a, af);
+    d = less ? o : a;
+    f = less ? of : af;
+    group_lex_min<OFF / 2, LANES>(d, f);
+  }
 }
 
 // CellHelper::calculate_barycentric_3D_coord (CellHelper.cpp:104-160) with the candidate faces
@@ -747,14 +815,7 @@ __host__ __device__ inline Located locate(const MeshDev& m, double px, double py
         merge_best(b1, f1, b2, d2, float_bits(e1[k].z), __builtin_inff());
       }
   }
-  if constexpr (LANES > 1) {
-#pragma unroll
-    for (int off = LANES / 2; off > 0; off >>= 1) {
-      const float o1 = lane_xor<LANES>(b1, off), o2 = lane_xor<LANES>(b2, off);
-      const int of1 = lane_xor<LANES>(f1, off);
-      merge_best(b1, f1, b2, o1, of1, o2);
-    }
-  }
+  group_merge_best<LANES / 2, LANES>(b1, f1, b2);
   int best_f = f1;
   if (!(sqrtf(b2) - sqrtf(b1) > kLocateMargin)) {  // close call (or non-finite input): rank in FP64
     r.fp64 |= 1;
@@ -766,14 +827,7 @@ __host__ __device__ inline Located locate(const MeshDev& m, double px, double py
       const double d = point_triangle_distance<double>(px, py, e0.x, e0.y, e0.z, e0.w, e1.x, e1.y);
       if (lex_less(d, f, bd, bf)) { bd = d; bf = f; }
     }
-    if constexpr (LANES > 1) {
-#pragma unroll
-      for (int off = LANES / 2; off > 0; off >>= 1) {
-        const double od = lane_xor<LANES>(bd, off);
-        const int of = lane_xor<LANES>(bf, off);
-        if (lex_less(od, of, bd, bf)) { bd = od; bf = of; }
-      }
-    }
+    group_lex_min<LANES / 2, LANES>(bd, bf);
     best_f = bf;
   }
   if (best_f == 0x7fffffff) best_f = 0;  // non-finite point: any valid face keeps indices in range

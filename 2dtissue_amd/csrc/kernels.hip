@@ -45,16 +45,26 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
-// the wave's sums of (sgn, cs, sn) in fixed point, written by its lane 0 to out: each wave keeps
-// its own partial (no workgroup barrier, so a finished wave leaves at once); integer sums make the
-// result independent of their order
-__device__ __forceinline__ void wave_order_partial(int sgn, long long cs, long long sn, OrderPartial* out) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    sgn += __shfl_xor(sgn, off, 64);
-    cs += __shfl_xor(cs, off, 64);
-    sn += __shfl_xor(sn, off, 64);
+// the sum over the lanes 0, STRIDE, 2 STRIDE, .. of the wave (integers, so the order is free)
+template <int STRIDE, int OFF = 32, class T>
+__device__ __forceinline__ T strided_wave_sum(T v) {
+  if constexpr (OFF >= STRIDE) {
+    T a, b;
+    butterfly<OFF, 64>(v, a, b);
+    return strided_wave_sum<STRIDE, OFF / 2>(a + b);
+  } else {
+    return v;
   }
+}
+
+// the wave's sums of (sgn, cs, sn) in fixed point over the first lane of each group, written by its
+// lane 0 to out: each wave keeps its own partial (no workgroup barrier, so a finished wave leaves at
+// once); integer sums make the result independent of their order
+template <int LANES>
+__device__ __forceinline__ void wave_order_partial(int sgn, long long cs, long long sn, OrderPartial* out) {
+  sgn = strided_wave_sum<LANES>(sgn);
+  cs = strided_wave_sum<LANES>(cs);
+  sn = strided_wave_sum<LANES>(sn);
   if ((threadIdx.x & 63) == 0) *out = OrderPartial{cs, sn, sgn, 0};
 }
 
@@ -86,15 +96,8 @@ __global__ void __launch_bounds__(kStepMaxBlock) k_step_tiled(MeshDev mesh, cons
   if constexpr (OCC) {  // stage this replica's occupancy mask of the input buckets in LDS
     const unsigned* occ_in = bin.occ + (size_t)r * nw;
     for (int k = tid; k < nw; k += (int)blockDim.x) s_occ[k] = occ_in[k];
+    __syncthreads();
   }
-  // clear this replica's bucket set consumed two steps ago (it is next step's output)
-  int* clr = bclr.count + (size_t)r * nv;
-  for (int w = tile.q * (int)blockDim.x + tid; w < nv; w += tile.nq * (int)blockDim.x) clr[w] = 0;
-  if constexpr (OCC) {
-    unsigned* clr_occ = bclr.occ + (size_t)r * nw;
-    for (int k = tile.q * (int)blockDim.x + tid; k < nw; k += tile.nq * (int)blockDim.x) clr_occ[k] = 0u;
-  }
-  __syncthreads();
   // a replica flagged before this step passes its state through unchanged (the reference stops
   // at the first failure); the flag rows rotate like the bucket sets
   const unsigned halt = io.halt_in[r];
@@ -147,8 +150,16 @@ __global__ void __launch_bounds__(kStepMaxBlock) k_step_tiled(MeshDev mesh, cons
       }
     }
   }
+  // clear this replica's bucket set consumed two steps ago (it is next step's output); last, so that
+  // no load of the step waits behind these stores
+  int* clr = bclr.count + (size_t)r * nv;
+  for (int w = tile.q * (int)blockDim.x + tid; w < nv; w += tile.nq * (int)blockDim.x) clr[w] = 0;
+  if constexpr (OCC) {
+    unsigned* clr_occ = bclr.occ + (size_t)r * nw;
+    for (int k = tile.q * (int)blockDim.x + tid; k < nw; k += tile.nq * (int)blockDim.x) clr_occ[k] = 0u;
+  }
   const int wpb = (int)blockDim.x >> 6;
-  wave_order_partial(sgn, pcs, psn, io.partial + (size_t)tile.logical * wpb + (tid >> 6));
+  wave_order_partial<LANES>(sgn, pcs, psn, io.partial + (size_t)tile.logical * wpb + (tid >> 6));
 }
 
 // crowded buckets up to this many particles are sorted in LDS (larger ones in global memory)
