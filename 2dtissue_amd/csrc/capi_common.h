@@ -113,6 +113,7 @@ inline tdev::StepParams make_step_params(const tissue_params& p) {
   s.mu64 = p.mu;
   s.dt64 = p.dt;
   s.rate64 = p.dt / p.tau;
+  s.kc64 = s.k64 / s.two_sigma64;
   return s;
 }
 

@@ -27,6 +27,7 @@ struct StepParams {
   float two_sigma, k, v0, mu, dt, rate;  // rate = dt / tau
   int32_t max_crossings, pad;
   double two_sigma64, k64, v064, mu64, dt64, rate64;  // the same parameters for the FP64 paths
+  double kc64;  // k64 / two_sigma64: Fij / d = kc (d - 2 sigma) / d, to a few ulps
 };
 
 // displacement (UV units) above which the force, speed and Euler update are redone in FP64:
@@ -56,6 +57,14 @@ struct BucketsOut { int* count; int* slot; int* ovf_n; int2* ovf; int* multi; un
 
 // words of a vertex-occupancy mask over nv vertices
 __host__ __device__ constexpr int occ_words(int nv) { return (nv + 31) >> 5; }
+
+// base[i] for a uniform base and 0 <= i * sizeof(T) < 2^32: the address is the scalar base plus a
+// 32-bit lane offset, two or three instructions fewer than a 64-bit one (the step's arrays are below
+// 4 GiB each: 2^27 particles, 2^26 vertices, 2^28 table entries)
+template <class T>
+__device__ __forceinline__ T load_at(const T* base, int i) {
+  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + (uint32_t)i * (uint32_t)sizeof(T));
+}
 
 // ------------------------------------------------------------------ neighbour traversal
 
@@ -169,6 +178,7 @@ static_assert(32 % kScanChunk == 0, "scan chunks must tile the 32-entry window")
 template <bool OCC, bool SORTED = false>
 struct GlobalSource {
   static constexpr bool kOcc = OCC;
+  static constexpr bool kCoop = true;
   BucketsIn b;
   const float4* xycs;
   const float* th;
@@ -179,12 +189,19 @@ struct GlobalSource {
   // whatever the count)
   __device__ __forceinline__ Head head(int w) const {
     Head h;
-    h.c = b.count[w];
-    h.s0 = b.slot[(size_t)w * kSlots];
-    h.s1 = b.slot[(size_t)w * kSlots + 1];
+    h.c = load_at(b.count, w);
+    const int2 s = load_at(reinterpret_cast<const int2*>(b.slot), w * (kSlots / 2));
+    h.s0 = s.x;
+    h.s1 = s.y;
     return h;
   }
-  __device__ __forceinline__ int count(int w) const { return b.count[w]; }
+  __device__ __forceinline__ int count(int w) const { return load_at(b.count, w); }
+  __device__ __forceinline__ void slots(int w, int (&a)[kSlots]) const {
+    const int4 s0 = load_at(reinterpret_cast<const int4*>(b.slot), 2 * w),
+               s1 = load_at(reinterpret_cast<const int4*>(b.slot), 2 * w + 1);
+    a[0] = s0.x; a[1] = s0.y; a[2] = s0.z; a[3] = s0.w;
+    a[4] = s1.x; a[5] = s1.y; a[6] = s1.z; a[7] = s1.w;
+  }
   // the particles of bucket w in ascending id order, without (each) and with (each_pos) their state
   template <class F>
   __device__ __forceinline__ void each(int w, const Head& h, F&& f) const {
@@ -215,7 +232,7 @@ struct GlobalSource {
       // kBatch particles at a time: the next ids and all of a batch's states are in flight together.
       // One at a time, two dependent loads per particle, a lane with a few crowded vertices (up to
       // 60 particles each) walked 100 us by itself and bounded the 100,000-particle step.
-      constexpr int kBatch = 8;
+      constexpr int kBatch = 4;
       const int* ids = c <= kSlots ? b.slot + (size_t)w * kSlots : b.big + h.s0;
       int id[kBatch];
 #pragma unroll
@@ -237,8 +254,8 @@ struct GlobalSource {
       }
     }
   }
-  __device__ __forceinline__ float4 pos(int j) const { return xycs[j]; }
-  __device__ __forceinline__ float theta(int j) const { return th[j]; }
+  __device__ __forceinline__ float4 pos(int j) const { return load_at(xycs, j); }
+  __device__ __forceinline__ float theta(int j) const { return load_at(th, j); }
 };
 
 // LDS-resident neighbour source of the persistent kernel: vertex buckets as a CSR over the
@@ -257,6 +274,7 @@ struct LdsSource {
     return h;
   }
   static constexpr bool kOcc = false;  // counts are LDS reads already
+  static constexpr bool kCoop = false;
   __device__ __forceinline__ int count(int w) const { return (int)begin[w + 1] - (int)begin[w]; }
   __device__ __forceinline__ bool occupied(int w) const { return begin[w + 1] != begin[w]; }
   template <class F>
@@ -288,7 +306,57 @@ struct LdsSource {
   __device__ __forceinline__ float theta(int j) const { return th[j]; }
 };
 
-// One particle's update (U1-U6 of the reference step) by a group of LANES lanes.
+// orders the LDS / global accesses of one wave (its lanes exchange data through memory)
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// inclusive sum over the lanes of a wave (all active)
+__device__ __forceinline__ int wave_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1, 2, 4, 8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
+  return v;
+}
+
+// ---- neighbour walk of a whole wave (narrow groups)
+//
+// With one to four lanes per particle a lane owns several table entries, few of which are occupied,
+// by one particle or by several: walked lane by lane, a wave pays for its unluckiest lane in every
+// loop, and each visit is a chain of three dependent loads. Here the wave's occupied entries are
+// compacted into LDS, its 64 lanes take one entry each (bucket head, pair coefficient) and then the
+// entries' particles, leaving each pair's terms in LDS, and every lane adds the terms of its own
+// entries in its own order: the sums are those of the lane-by-lane walk, bit for bit. Particles of a
+// crowded bucket (more than kSlots) are added by the owner lane itself, in their place. Lanes without
+// work load a fixed address instead of branching around the load: a load under a branch is waited
+// for before the next is issued. Area per wave:
+constexpr int kWaveEntries = 256;  // entries compacted at a time (more: entry by entry of the lanes)
+constexpr int kWavePairs = 192;    // pairs of a round (a round takes as many entries as fit)
+// whether P physical lanes per particle walk this way for sums laid out over LANES lanes (crowded:
+// sorted buckets; with as many lanes as the layout the lane-by-lane walk is 2-3 % faster there, 65,000
+// and 100,000 particles)
+constexpr bool coop_walk(int lanes, int p, bool crowded) { return p != lanes || (lanes <= 4 && !crowded); }
+// table entries per lane taken together, by physical lanes
+constexpr int coop_chunk(int p) { return p >= 16 ? 2 : (p == 8 ? 4 : 8); }
+struct WaveWalk {
+  double2 F[kWavePairs];        // force terms
+  float2 S[kWavePairs];         // alignment terms
+  int2 ent[kWaveEntries + 64];  // (vertex | owner lane << 26, float bits of the distance); then a slot
+                                //   per lane for what is not kept
+  int pp[64 + 4];               // before each entry of the round: pairs, and << 16 particles counted
+  unsigned vh[kWavePairs];      // visit_mix of the pair's particle (visit check only)
+};
+constexpr int kOwnerShift = 26;  // vertex ids below 2^26 (checked by the launcher)
+
+// One particle's update (U1-U6 of the reference step) by a group of P lanes. The sums over the
+// neighbours are laid out over LANES lanes: lane l of LANES adds the entries l, l + LANES, .. of the
+// particle's table row in order, and a butterfly adds the lanes. That layout fixes the results to the
+// bit; P >= LANES, the lanes that do the work, is free (the whole-wave walk): more than LANES where
+// waves are few and the longest chain counts (phys_lanes).
 //   me = (x, y, cos theta, sin theta) of particle i, th its heading, v its vertex id.
 // Neighbours: particles bucketed on the vertices w of row v of the geodesic table; pair
 // distance d = D[v, w]. Force and alignment for d < 2 sigma (ForceHelper.cpp:34-73,
@@ -296,18 +364,22 @@ struct LdsSource {
 // (2DTissue.cpp:254-268). The force is summed in FP64 (its FP32 rounding feeds the FP32 speed
 // and Euler step; the FP64 value the large-displacement path); the alignment sums are FP32, redone
 // in FP64 when they nearly cancel.
-// WAVE selects the seam-wrap loop of crowded systems (seam_wrap_group). Always inlined: as an
+// active: false for the lanes past the last particle, which only help the wave (their own result
+// is not used); ww: the wave's LDS area (whole-wave walk: all lanes of the wave present; else
+// null). WAVE selects the seam-wrap loop of crowded systems (seam_wrap_group). Always inlined: as an
 // out-of-line call (which the inliner picks once two kernels share an instantiation) its result
 // and live state go through scratch memory.
-template <int LANES, bool WAVE = false, class Src>
+template <int LANES, int P, bool WAVE = false, bool VISITS = false, class Src>
 __device__ __forceinline__ StepOut particle_step(const MeshDev& mesh, const StepParams& prm, const Src& src, int i, float4 me,
-                                        float th, int v, float eta, int lane) {
+                                        float th, int v, float eta, int lane, bool active = true,
+                                        WaveWalk* ww = nullptr) {
+  // a lane's sums: those of strand lane % LANES of the layout (its copies on the lanes above LANES equal it)
   float Sx = 0.f, Sy = 0.f;
   double Fx64 = 0.0, Fy64 = 0.0;  // the force, summed in FP64 (its FP32 rounding drives the FP32 path)
-  const double kc64 = prm.k64 / prm.two_sigma64;  // Fij / d = kc (d - 2 sigma) / d, to a few ulps
-  int na = 0, nb = 0;
+  const double kc64 = prm.kc64;
+  int na = 0, nb = 0, nb_only = 0;  // nb_only: counted without a pair by the whole-wave scan
   unsigned vh = 0u;
-  const int rs = mesh.row_ptr[v], re = mesh.row_ptr[v + 1];
+  const int rs = load_at(mesh.row_ptr, v), re = active ? load_at(mesh.row_ptr, v + 1) : rs;
   // pair set-up of a near entry (vertex w at distance d, bucket head h) and its particles
   auto visit = [&](int w, float d, const typename Src::Head& h) __attribute__((always_inline)) {
     const double dd = d == 0.0f ? 0.001 : (double)d;
@@ -326,7 +398,7 @@ __device__ __forceinline__ StepOut particle_step(const MeshDev& mesh, const Step
     });
   };
   // Each lane walks its entries rs + lane + m * LANES, m = 0, 1, .., in order.
-  if constexpr (LANES >= kHeadScanLanes) {
+  if constexpr (LANES >= kHeadScanLanes && P == LANES) {
     // At most a few entries per lane: the scan loads each near entry's bucket head (count and
     // first slots) together with the entries' counts, and the lane visits its occupied entries
     // from registers: table entry -> bucket head -> particles, no reload of marked entries.
@@ -336,7 +408,8 @@ __device__ __forceinline__ StepOut particle_step(const MeshDev& mesh, const Step
 #pragma unroll
       for (int k = 0; k < kHeadChunk; ++k) {
         const int e = base + k * LANES;
-        ent[k] = e < re ? mesh.nbr[e] : make_int2(0, 0x7f800000);  // +inf ends the walk
+        ent[k] = load_at(mesh.nbr, min(e, re - 1));
+        if (e >= re) ent[k].y = 0x7f800000;  // +inf ends the walk
       }
       bool oc[kHeadChunk];
 #pragma unroll
@@ -344,9 +417,8 @@ __device__ __forceinline__ StepOut particle_step(const MeshDev& mesh, const Step
         oc[k] = __int_as_float(ent[k].y) <= prm.t_count && (!Src::kOcc || src.occupied(ent[k].x));
 #pragma unroll
       for (int k = 0; k < kHeadChunk; ++k) {
-        const float d = __int_as_float(ent[k].y);
-        if (oc[k] && d <= prm.t_near) hd[k] = src.head(ent[k].x);
-        else if (oc[k]) hd[k].c = src.count(ent[k].x);
+        hd[k] = src.head(oc[k] ? ent[k].x : 0);
+        if (!oc[k]) hd[k].c = 0;
       }
       bool stop = false;
 #pragma unroll
@@ -360,6 +432,187 @@ __device__ __forceinline__ StepOut particle_step(const MeshDev& mesh, const Step
         else if (hd[k].c > 0) visit(ent[k].x, d, hd[k]);
       }
       if (stop) break;
+    }
+  } else if constexpr (Src::kCoop && coop_walk(LANES, P, WAVE)) {
+    constexpr int kChunk = coop_chunk(P);
+    const int wl = (int)__lane_id();
+    bool done = false;
+    for (int wbase = rs + lane;; wbase += kChunk * P) {
+      const bool more = !done && wbase < re;
+      if (__builtin_amdgcn_ballot_w64(more) == 0) break;
+      // the lane's next kChunk entries, the occupied ones marked (with the mask in LDS: counted-only
+      // entries too, their count comes with the head; else their count is added here)
+      int2 ent[kChunk];
+      unsigned mark = 0u;
+#pragma unroll
+      for (int k = 0; k < kChunk; ++k) {
+        const int e = wbase + k * P;
+        ent[k] = load_at(mesh.nbr, max(min(e, re - 1), 0));
+        if (!more || e >= re) ent[k].y = 0x7f800000;
+      }
+      if constexpr (Src::kOcc) {
+#pragma unroll
+        for (int k = 0; k < kChunk; ++k)
+          mark |= __int_as_float(ent[k].y) <= prm.t_count && src.occupied(ent[k].x) ? 1u << k : 0u;
+      } else {
+        int cnt[kChunk];
+#pragma unroll
+        for (int k = 0; k < kChunk; ++k) cnt[k] = src.count(__int_as_float(ent[k].y) <= prm.t_count ? ent[k].x : 0);
+#pragma unroll
+        for (int k = 0; k < kChunk; ++k) {
+          const float d = __int_as_float(ent[k].y);
+          nb_only += d > prm.t_near && d <= prm.t_count ? cnt[k] : 0;
+          mark |= d <= prm.t_near && cnt[k] > 0 ? 1u << k : 0u;
+        }
+      }
+      done = __int_as_float(ent[kChunk - 1].y) > prm.t_count;  // rows ascend in distance
+      // (hardly ever more marks than the list holds: then one entry of each lane at a time)
+      const bool split = 64 * kChunk > kWaveEntries &&
+                         __builtin_amdgcn_readlane(wave_scan(__builtin_popcount(mark)), 63) > kWaveEntries;
+      for (unsigned all = split ? 1u : ~0u; all != 0u; all = split ? (all << 1) & ((1u << kChunk) - 1u) : 0u) {
+        // places in the list: by particle, then by strand, then in the row's order; [first, last) of
+        // the lane's strand
+        int first, last, at[kChunk], total = 0;
+        const unsigned kept = mark & all;
+        if constexpr (P == LANES) {
+          const int mine = __builtin_popcount(kept), upto = wave_scan(mine);
+          total = __builtin_amdgcn_readlane(upto, 63);
+          last = first = upto - mine;
+#pragma unroll
+          for (int k = 0; k < kChunk; ++k) {
+            at[k] = last;
+            last += (kept >> k) & 1u;
+          }
+        } else {
+          // lanes v, v + LANES, .. of the group share strand v = lane % LANES
+          constexpr unsigned kEvery = LANES == 1 ? ~0u : (LANES == 2 ? 0x55555555u : (LANES == 4 ? 0x11111111u : 0x01010101u));
+          constexpr unsigned kGroup = P >= 32 ? ~0u : (1u << P) - 1u;
+          const int v = lane & (LANES - 1), gbase = wl & ~(P - 1);
+          const unsigned same = kEvery << v & kGroup;                // the strand's lanes
+          const unsigned less = kEvery * ((1u << v) - 1u) & kGroup;  // the lanes of the strands before
+          const unsigned below = same & ((1u << lane) - 1u);
+          int p = 0, in_strand = 0;
+#pragma unroll
+          for (int k = 0; k < kChunk; ++k) {
+            const uint64_t b = __builtin_amdgcn_ballot_w64(((kept >> k) & 1u) != 0u);
+            const unsigned g = (unsigned)(b >> gbase) & kGroup;
+            p += __builtin_popcountll(b & ((1ull << gbase) - 1ull)) + __builtin_popcount(g & less);
+            at[k] = in_strand + __builtin_popcount(g & below);
+            in_strand += __builtin_popcount(g & same);
+            total += __builtin_popcountll(b);
+          }
+#pragma unroll
+          for (int k = 0; k < kChunk; ++k) at[k] += p;
+          first = p;
+          last = p + in_strand;
+        }
+        if (total == 0) continue;
+#pragma unroll
+        for (int k = 0; k < kChunk; ++k)
+          ww->ent[(kept >> k) & 1u ? at[k] : kWaveEntries + wl] =
+              make_int2((int)((unsigned)ent[k].x | ((unsigned)wl << kOwnerShift)), ent[k].y);
+        wave_sync();
+        for (int r0 = 0; r0 < total;) {
+          // one entry per lane: its bucket and pair coefficient
+          const bool has = r0 + wl < total;
+          const int2 en = ww->ent[has ? r0 + wl : r0];
+          const int w = en.x & ((1 << kOwnerShift) - 1), owner = (int)((unsigned)en.x >> kOwnerShift);
+          const float d = __int_as_float(en.y);
+          const int count = src.count(has ? w : 0);
+          int a[kSlots];  // the slots are in bounds whatever the count
+          src.slots(has ? w : 0, a);
+          const float ox = __shfl(me.x, owner, 64), oy = __shfl(me.y, owner, 64);
+          const int oi = __shfl(i, owner, 64);
+          const double dd = d == 0.0f ? 0.001 : (double)d;
+          const double g64 = (kc64 * (dd - prm.two_sigma64)) / dd;
+          const int c = has ? count : 0;
+          const bool is_near = !Src::kOcc || d <= prm.t_near;
+          const int np = c > kSlots || !is_near ? 0 : c;  // pairs left in LDS
+          const int pk = c > kSlots ? 0 : (np | (d != 0.0f ? c << 16 : 0));
+          const int sum = wave_scan(pk), before = sum - pk;
+          const uint64_t fits = __builtin_amdgcn_ballot_w64((sum & 0xffff) <= kWavePairs);
+          const int taken = min(fits == ~0ull ? 64 : __builtin_ctzll(~fits), total - r0);  // entries of this round
+          const bool crowded = __builtin_amdgcn_ballot_w64(c > kSlots && wl < taken) != 0;
+          const int at = before & 0xffff;
+          auto term = [&](int q, int j, const float4& p) __attribute__((always_inline)) {
+            const double fx = g64 * ((double)ox - (double)p.x), fy = g64 * ((double)oy - (double)p.y);
+            ww->F[at + q] = j != oi ? make_double2(fx, fy) : make_double2(0.0, 0.0);
+            ww->S[at + q] = make_float2(p.z, p.w);
+            if constexpr (VISITS) ww->vh[at + q] = visit_mix((unsigned)j);
+          };
+          const int mine_np = wl < taken ? np : 0;
+          const bool more2 = __builtin_amdgcn_ballot_w64(mine_np > 2) != 0;
+          if (!src.b.sorted) {  // ids ascending
+            if (more2) {
+#pragma unroll
+              for (int q = 0; q < kSlots; ++q) a[q] = q < np ? a[q] : 0x7fffffff;
+              sort8(a);
+            } else if (np == 2) {
+              const int j0 = min(a[0], a[1]);
+              a[1] = max(a[0], a[1]);
+              a[0] = j0;
+            }
+          }
+          {
+            const float4 p0 = src.pos(mine_np > 0 ? a[0] : 0), p1 = src.pos(mine_np > 1 ? a[1] : 0);
+            if (!more2) {
+              if (mine_np > 0) term(0, a[0], p0);
+              if (mine_np > 1) term(1, a[1], p1);
+            } else {
+              const float4 p2 = src.pos(mine_np > 2 ? a[2] : 0), p3 = src.pos(mine_np > 3 ? a[3] : 0);
+              if (mine_np > 0) term(0, a[0], p0);
+              if (mine_np > 1) term(1, a[1], p1);
+              if (mine_np > 2) term(2, a[2], p2);
+              if (mine_np > 3) term(3, a[3], p3);
+              if (__builtin_amdgcn_ballot_w64(mine_np > 4) != 0) {
+                float4 p[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) p[q] = src.pos(mine_np > 4 + q ? a[4 + q] : 0);
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                  if (mine_np > 4 + q) term(4 + q, a[4 + q], p[q]);
+              }
+            }
+          }
+          ww->pp[wl] = before;
+          if (wl == 63) ww->pp[64] = sum;
+          wave_sync();
+          // the strand's entries of the round
+          const int lo = min(max(first - r0, 0), taken), hi = min(max(last - r0, 0), taken);
+          const int s0 = ww->pp[lo], s1 = ww->pp[hi];
+          auto add = [&](int p) __attribute__((always_inline)) {
+            const double2 f = ww->F[p];
+            const float2 q = ww->S[p];
+            Fx64 += f.x;
+            Fy64 += f.y;
+            Sx += q.x;
+            Sy += q.y;
+            if constexpr (VISITS) vh += ww->vh[p];
+          };
+          if (!crowded) {
+            for (int p = s0 & 0xffff; p < (s1 & 0xffff); ++p) add(p);
+          } else {
+            for (int t = lo; t < hi; ++t) {
+              const int p1 = ww->pp[t + 1] & 0xffff;
+              int p = ww->pp[t] & 0xffff;
+              if (p == p1) {  // crowded, or counted only
+                const int2 e = ww->ent[r0 + t];
+                const int we = e.x & ((1 << kOwnerShift) - 1);
+                const typename Src::Head he = src.head(we);
+                if (he.c > kSlots) {
+                  if (__int_as_float(e.y) <= prm.t_near) visit(we, __int_as_float(e.y), he);
+                  else nb += he.c;
+                }
+              }
+              for (; p < p1; ++p) add(p);
+            }
+          }
+          na += (s1 - s0) & 0xffff;
+          nb += (s1 >> 16) - (s0 >> 16);
+          wave_sync();
+          r0 += taken;
+        }
+      }
     }
   } else {
     // Windows of 32 entries per lane:
@@ -380,7 +633,8 @@ __device__ __forceinline__ StepOut particle_step(const MeshDev& mesh, const Step
 #pragma unroll
         for (int k = 0; k < kScanChunk; ++k) {
           const int e = wbase + (m0 + k) * LANES;
-          ent[k] = e < re ? mesh.nbr[e] : make_int2(0, 0x7f800000);  // +inf ends the walk
+          ent[k] = load_at(mesh.nbr, min(e, re - 1));
+          if (e >= re) ent[k].y = 0x7f800000;  // +inf ends the walk
         }
         bool oc[kScanChunk];
         if constexpr (Src::kOcc) {
@@ -389,10 +643,18 @@ __device__ __forceinline__ StepOut particle_step(const MeshDev& mesh, const Step
 #pragma unroll
           for (int k = 0; k < kScanChunk; ++k) oc[k] = __int_as_float(ent[k].y) <= prm.t_count && src.occupied(ent[k].x);
 #pragma unroll
-          for (int k = 0; k < kScanChunk; ++k) cnt[k] = oc[k] && __int_as_float(ent[k].y) > prm.t_near ? src.count(ent[k].x) : 0;
+          for (int k = 0; k < kScanChunk; ++k) {
+            const bool want = oc[k] && __int_as_float(ent[k].y) > prm.t_near;
+            cnt[k] = src.count(want ? ent[k].x : 0);
+            if (!want) cnt[k] = 0;
+          }
         } else {
 #pragma unroll
-          for (int k = 0; k < kScanChunk; ++k) cnt[k] = __int_as_float(ent[k].y) <= prm.t_count ? src.count(ent[k].x) : 0;
+          for (int k = 0; k < kScanChunk; ++k) {
+            const bool want = __int_as_float(ent[k].y) <= prm.t_count;
+            cnt[k] = src.count(want ? ent[k].x : 0);
+            if (!want) cnt[k] = 0;
+          }
 #pragma unroll
           for (int k = 0; k < kScanChunk; ++k) oc[k] = cnt[k] > 0;
         }
@@ -410,7 +672,7 @@ __device__ __forceinline__ StepOut particle_step(const MeshDev& mesh, const Step
       while (mark) {
         const int m = __builtin_ctz(mark);
         mark &= mark - 1u;
-        const int2 en = mesh.nbr[wbase + m * LANES];
+        const int2 en = load_at(mesh.nbr, wbase + m * LANES);
         visit(en.x, __int_as_float(en.y), src.head(en.x));
       }
     }
@@ -423,6 +685,7 @@ __device__ __forceinline__ StepOut particle_step(const MeshDev& mesh, const Step
   na = group_sum<LANES>(na);
   vh = group_sum<LANES>(vh);
   nb = group_sum<LANES>(nb);
+  if constexpr (Src::kCoop && coop_walk(LANES, P, WAVE)) nb += group_sum<P>(nb_only);
 
   // speed, velocity, Euler step (Locomotion.cpp:71-84)
   const float Fm = sqrtf(Fx * Fx + Fy * Fy);
@@ -449,17 +712,21 @@ __device__ __forceinline__ StepOut particle_step(const MeshDev& mesh, const Step
   if (weak) {
     // the alignment sum again, over the neighbours' headings in FP64
     double Sx64 = 0.0, Sy64 = 0.0;
-    for (int base = rs + lane; base < re; base += kRowChunk * LANES) {
+    for (int base = rs + (lane & (LANES - 1)); base < re; base += kRowChunk * LANES) {
       int2 ent[kRowChunk];
       typename Src::Head head[kRowChunk];
 #pragma unroll
       for (int k = 0; k < kRowChunk; ++k) {
         const int e = base + k * LANES;
-        ent[k] = e < re ? mesh.nbr[e] : make_int2(0, 0x7f800000);
+        ent[k] = load_at(mesh.nbr, min(e, re - 1));
+        if (e >= re) ent[k].y = 0x7f800000;
       }
 #pragma unroll
-      for (int k = 0; k < kRowChunk; ++k)
-        if (__int_as_float(ent[k].y) <= prm.t_near && (!Src::kOcc || src.occupied(ent[k].x))) head[k] = src.head(ent[k].x);
+      for (int k = 0; k < kRowChunk; ++k) {
+        const bool oc = __int_as_float(ent[k].y) <= prm.t_near && (!Src::kOcc || src.occupied(ent[k].x));
+        head[k] = src.head(oc ? ent[k].x : 0);
+        if (!oc) head[k].c = 0;
+      }
       bool stop = false;
 #pragma unroll
       for (int k = 0; k < kRowChunk; ++k) {
@@ -514,7 +781,7 @@ __device__ __forceinline__ StepOut particle_step(const MeshDev& mesh, const Step
     if (__builtin_amdgcn_ballot_w64(loop) != 0) {
       double lx = loop ? px : 0.5, ly = loop ? py : 0.5;
       int q = 0;
-      const bool good = seam_wrap_group<LANES, true>(me.x, me.y, lx, ly, dth, prm.max_crossings, lane, &q);
+      const bool good = seam_wrap_group<P, true>(me.x, me.y, lx, ly, dth, prm.max_crossings, lane, &q);
       if (loop) {
         px = lx;
         py = ly;
@@ -523,7 +790,7 @@ __device__ __forceinline__ StepOut particle_step(const MeshDev& mesh, const Step
       }
     }
   } else if (loop) {
-    if (!seam_wrap_group<LANES, false>(me.x, me.y, px, py, dth, prm.max_crossings, lane, &o.q)) o.fl |= kFlagTiling;
+    if (!seam_wrap_group<P, false>(me.x, me.y, px, py, dth, prm.max_crossings, lane, &o.q)) o.fl |= kFlagTiling;
   }
   if (finite && !folded) thn = wrap_heading(thn + dth);
   if (finite && !inside_unit(px, py)) o.fl |= kFlagLost;
@@ -536,7 +803,7 @@ __device__ __forceinline__ StepOut particle_step(const MeshDev& mesh, const Step
   o.na = na;
   o.vh = vh;
   // UV -> 3D remap of the stored FP32 position (CellHelper.cpp:71-85)
-  o.L = locate<LANES>(mesh, (double)o.xo, (double)o.yo, lane);
+  o.L = locate<P>(mesh, (double)o.xo, (double)o.yo, lane);
   sincosf(o.to, &o.so, &o.co);
   // order parameter (LinearAlgebra.cpp:90-105, z = 0): sign of the cross product's z component
   const double cz = (double)o.xo * (double)vy - (double)o.yo * (double)vx;

@@ -308,7 +308,7 @@ void Engine::rebuild_buckets() {
 void Engine::ensure_tiles(const Shape& s) {
   const auto key = std::make_tuple(s.lanes, s.block, s.xcd);
   if (d_tiles && tiles_key == key) return;
-  const int per = s.block / s.lanes;
+  const int per = s.block / phys_lanes(s);
   std::vector<TileDesc> logical;
   std::vector<int> begin(R + 1, 0);
   for (int r = 0; r < R; ++r) {
@@ -501,7 +501,7 @@ void Engine::enqueue(const Shape& s, int n_steps, const float* nz, size_t stride
         io.visit = d_visit;
         BucketSet out = bs[(bp + 1) % 3];
         if (raw_buckets) out.multi = nullptr;  // no finalize pass reads the sort list
-        HIP_OK(launch_step_tiled(s.lanes, s.block, false, !raw_buckets, md, d_reps, d_tiles, n_phys, bs[bp], out, bs[(bp + 2) % 3],
+        HIP_OK(launch_step_tiled(s.lanes, phys_lanes(s), s.block, false, !raw_buckets, md, d_reps, d_tiles, n_phys, bs[bp], out, bs[(bp + 2) % 3],
                                  io, stream));
         if (rec)
           HIP_OK(launch_record(ntot, d_row0, t, rec->every, rec->depth, io.xycs_out, r3x, r3y, r3z, nbr, rec->d_ring,
@@ -572,7 +572,7 @@ int32_t Engine::run_once(const Shape& s, int n_steps, const float* nz, size_t st
       partial = dalloc<OrderPartial>(need);
       partial_cap = need;
     }
-    const bool occ = stage_occupancy(md.nv, s.block, s.lanes);
+    const bool occ = stage_occupancy(md.nv, s.block, s.lanes, phys_lanes(s));
     if (occ && !occ_kept) buckets_stale = true;  // the sets were filled without the masks this shape reads
     occ_kept = occ;
     if (buckets_stale) rebuild_buckets();

@@ -187,6 +187,7 @@ struct Engine {
   void ensure_tiles(const Shape& s);
   void enqueue(const Shape& s, int n_steps, const float* noise, size_t stride);
   Shape resolve_for(Shape s) const;
+  int phys_lanes(const Shape& s) const { return tissue::phys_lanes(s.lanes, ntot, md.nv, s.block); }
 };
 
 }  // namespace tissue

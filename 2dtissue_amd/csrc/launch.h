@@ -123,8 +123,28 @@ constexpr int kStepMaxBlock = 512;
 // such launches keep the mask up to date: for the others it would be one more memory-side atomic per
 // occupied vertex (63,000 of them in a step of 100,000 particles).
 constexpr int kOccWordsPerParticle = 8;
-inline bool stage_occupancy(int nv, int block, int lanes) {
-  return tdev::occ_words(nv) <= kOccWordsPerParticle * (block / lanes);
+// LDS of one workgroup of the tiled step kernel: the waves' walk areas and the staged mask
+inline size_t step_lds_bytes(int nv, int block, int lanes, int phys, bool crowded, bool occ) {
+  return (tdev::coop_walk(lanes, phys, crowded) ? (size_t)(block / 64) * sizeof(tdev::WaveWalk) : 0) +
+         (occ ? sizeof(unsigned) * (size_t)tdev::occ_words(nv) : 0);
+}
+constexpr size_t kStepMaxLds = 64 * 1024;  // what a launch may ask for without raising the limit
+inline bool stage_occupancy(int nv, int block, int lanes, int phys) {
+  return phys <= lanes && tdev::occ_words(nv) <= kOccWordsPerParticle * (block / phys) &&
+         step_lds_bytes(nv, block, lanes, phys, false, true) <= kStepMaxLds;
+}
+// Physical lanes per particle for sums laid out over `lanes` lanes (the results are the same for any).
+// As many as the layout where the chip is full; more where it is not and a step's longest chain counts
+// (MI355X, us per step): 4 -> 8 at 9,001 particles 25.2 / 22.9, 13,000 in 37 replicas 19.8 / 18.1, 20,000
+// 39.7 / 37.8, 30,000 in 30 replicas 26.5 / 25.1, 40,000 40.5 / 43.3; 8 -> 16 at 5,000 particles
+// 19.2 / 16.7, 8,000 21.2 / 18.1; 2 -> 4 for replicas sparse on a mesh too large for the occupancy mask,
+// 64 x 2,000 (gradients, ms) 30.6 / 29.2, but with the mask 80,000 particles 43.3 / 44.4 and 530,000
+// 163 / 181. Fewer lanes than the layout were slower throughout (530,000 particles, 2 -> 1: 163 / 192).
+inline int phys_lanes(int lanes, int ntot, int nv, int block) {
+  if (lanes == 8 && ntot <= 16384) return 16;
+  if (lanes == 4 && ntot <= 32768) return 8;
+  if (lanes == 2 && ntot <= 163840 && !stage_occupancy(nv, block, 2, 2)) return 4;
+  return lanes;
 }
 constexpr int kResidentMaxBlock = 512;
 
@@ -161,10 +181,11 @@ hipError_t resident_prepare(int nv, int nmax);
 hipError_t launch_resident(int lanes, int block, const tdev::MeshDev& mesh, const ReplicaDesc* reps, int R, int nmax,
                            int steps, const ResidentIO& io, hipStream_t st);
 
-// one step of every replica: n_tiles workgroups of `block` threads, `lanes` lanes per particle;
+// one step of every replica: n_tiles workgroups of `block` threads, `phys` lanes per particle, its
+// sums laid out over `lanes` lanes (phys: phys_lanes);
 // reads bucket set bin, writes bout, clears bclr; tape selects the variant that records the
 // adjoint tape; wave the seam-wrap loop of crowded systems (same results, see seam_wrap_group)
-hipError_t launch_step_tiled(int lanes, int block, bool tape, bool wave, const tdev::MeshDev& mesh, const ReplicaDesc* reps,
+hipError_t launch_step_tiled(int lanes, int phys, int block, bool tape, bool wave, const tdev::MeshDev& mesh, const ReplicaDesc* reps,
                              const TileDesc* tiles, int n_tiles, const BucketSet& bin, const BucketSet& bout,
                              const BucketSet& bclr, const TiledIO& io, hipStream_t st);
 // sort the buckets of set bs that hold two or more particles (over the same tiles as the step);

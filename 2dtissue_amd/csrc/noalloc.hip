@@ -208,7 +208,7 @@ extern "C" int32_t tissue_step_noalloc(const tissue_mesh* mc, const tissue_param
 
     int lanes = 0, block = 0;
     tissue::tiled_default_shape(1, n, &lanes, &block);
-    const int per = block / lanes;
+    const int phys = tissue::phys_lanes(lanes, n, md.nv, block), per = block / phys;
     const int n_tiles = cdiv(n, per);
     if (n_tiles > kMaxTiles) throw ApiError(TISSUE_E_INVALID_ARG, "tissue_step_noalloc: too many tiles");
     const int sorted = tissue::raw_buckets_for(n, md.nv) ? 0 : 1;
@@ -271,7 +271,7 @@ extern "C" int32_t tissue_step_noalloc(const tissue_mesh* mc, const tissue_param
     io.halt_clr = a.rows + 2;
     io.first_bad = a.first_bad;
     io.step = 0;
-    HIP_OK(tissue::launch_step_tiled(lanes, block, false, sorted != 0, md, a.rep, a.tiles, n_tiles, b[0], b[1], b[2], io, st));
+    HIP_OK(tissue::launch_step_tiled(lanes, phys, block, false, sorted != 0, md, a.rep, a.tiles, n_tiles, b[0], b[1], b[2], io, st));
     HIP_OK(tissue::launch_phi_tiles(1, 1, a.tile_begin, n_tiles, tissue::partials_per_tile(block), io.partial, a.rep,
                                     phi, 1, 0, st));
     hipLaunchKernelGGL(k_noalloc_finish, dim3(cdiv(n, 256)), dim3(256), 0, st, n, io.xycs_out, x_out, y_out,

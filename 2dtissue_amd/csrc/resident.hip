@@ -135,7 +135,7 @@ __global__ void __launch_bounds__(kMaxBlock) k_resident(MeshDev mesh, const Repl
     // Jacobi, every particle must read the old state of its neighbours
     for (int i = group; i < n; i += ngroups) {
       const float eta = eta_row ? eta_row[i] : 0.0f;
-      const StepOut o = particle_step<LANES>(mesh, rep.prm, src, i, xycs[i], th[i], vid[i], eta, lane);
+      const StepOut o = particle_step<LANES, LANES>(mesh, rep.prm, src, i, xycs[i], th[i], vid[i], eta, lane);
       if (lane == 0) {
         nxt_xycs[i] = make_float4(o.xo, o.yo, o.co, o.so);
         nxt_th[i] = o.to;

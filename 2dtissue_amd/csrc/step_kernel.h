@@ -1,0 +1,206 @@
+// gfx950 kernel of the tiled per-step update (one launch per step, all replicas at once).
+//
+// k_step_tiled<LANES, P>: each workgroup is a tile of one replica (TileDesc); P lanes of a wave64
+// cooperate on one particle, whose sums are laid out over LANES lanes (particle_step). They stride over the particle's row of the truncated geodesic table
+// (vertices within 2.4 sigma of its vertex, ascending in distance), visit the particles bucketed on
+// those vertices, and reduce force, alignment sum and neighbour count with butterfly shuffles.
+// Every lane then runs the per-particle epilogue (speed, Euler, heading, seam wrap) and the lanes
+// split the point-location candidates of the face bucket. Lane 0 writes the SoA outputs, inserts
+// the particle into next step's vertex buckets and contributes to the tile's order-parameter
+// partials. A single system is the case of one replica.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include <climits>
+
+#include "launch.h"
+
+namespace tissue {
+
+using namespace tdev;
+
+namespace {
+
+template <bool OCC>
+__device__ __forceinline__ void bucket_insert(const BucketsOut& b, int v, int i) {
+  const int old = atomicAdd(&b.count[v], 1);
+  if (OCC && old == 0) atomicOr(&b.occ[v >> 5], 1u << (v & 31));
+  if (old < kSlots) {
+    b.slot[(size_t)v * kSlots + old] = i;
+  } else {
+    const int o = atomicAdd(b.ovf_n, 1);
+    b.ovf[o] = make_int2(v, i);
+  }
+  if (b.multi) b.multi[i] = old == 1 ? v : -1;  // the second arrival has the bucket sorted
+}
+
+__device__ __forceinline__ BucketsOut replica_out(const BucketSet& s, int r, int nv, int off) {
+  return {s.count + (size_t)r * nv, s.slot + (size_t)r * nv * kSlots, s.ovf_n + r, s.ovf + off, s.multi,
+          s.occ + (size_t)r * occ_words(nv)};
+}
+
+}  // namespace
+
+#ifdef TISSUE_STEP_KERNEL  // the kernel itself, for the translation units that instantiate it
+
+namespace {
+
+// the sum over the lanes 0, STRIDE, 2 STRIDE, .. of the wave (integers, so the order is free)
+template <int STRIDE, int OFF = 32, class T>
+__device__ __forceinline__ T strided_wave_sum(T v) {
+  if constexpr (OFF >= STRIDE) {
+    T a, b;
+    butterfly<OFF, 64>(v, a, b);
+    return strided_wave_sum<STRIDE, OFF / 2>(a + b);
+  } else {
+    return v;
+  }
+}
+
+// the wave's sums of (sgn, cs, sn) in fixed point over the first lane of each group, written by its
+// lane 0 to out: each wave keeps its own partial (no workgroup barrier, so a finished wave leaves at
+// once); integer sums make the result independent of their order
+template <int LANES>
+__device__ __forceinline__ void wave_order_partial(int sgn, long long cs, long long sn, OrderPartial* out) {
+  sgn = strided_wave_sum<LANES>(sgn);
+  cs = strided_wave_sum<LANES>(cs);
+  sn = strided_wave_sum<LANES>(sn);
+  if ((threadIdx.x & 63) == 0) *out = OrderPartial{cs, sn, sgn, 0};
+}
+
+template <int LANES, int P, bool TAPE, bool OCC, bool VISITS, bool WAVE>
+__global__ void __launch_bounds__(kStepMaxBlock) k_step_tiled(MeshDev mesh, const ReplicaDesc* __restrict__ reps,
+                                                              const TileDesc* __restrict__ tiles, BucketSet bin, BucketSet bout,
+                                                              BucketSet bclr, TiledIO io) {
+  // the waves' walk areas (whole-wave walk), then with OCC occ_words(nv) words, the input buckets'
+  // occupancy mask
+  extern __shared__ __align__(16) unsigned char smem[];
+  constexpr bool kCoop = coop_walk(LANES, P, WAVE);
+  WaveWalk* ww = kCoop ? reinterpret_cast<WaveWalk*>(smem) + (threadIdx.x >> 6) : nullptr;
+  unsigned* s_occ = reinterpret_cast<unsigned*>(smem + (kCoop ? (blockDim.x >> 6) * sizeof(WaveWalk) : 0));
+  const TileDesc tile = tiles[blockIdx.x];
+  if (tile.r < 0) return;  // idle padding workgroup (whole block)
+  const int r = tile.r;
+  const ReplicaDesc& rep = reps[r];  // uniform: read through the scalar cache where used
+  const int nv = mesh.nv, tid = threadIdx.x, nw = occ_words(nv);
+  const int lane = tid & (P - 1);
+  const int i = tile.first + tid / P;
+  const bool active = i < rep.n;
+  const int g = rep.off + i;
+  // the particle's inputs first: their loads are in flight during the set-up below
+  float4 me = make_float4(0.f, 0.f, 0.f, 0.f);
+  float th = 0.f, eta = 0.f;
+  int v = 0;
+  if (active) {
+    me = io.xycs_in[g];
+    th = io.th_in[g];
+    v = io.vid_in[g];
+    const size_t shift = io.noise_row0 ? (size_t)io.noise_row0[0] * io.noise_stride : 0;
+    eta = io.noise ? io.noise[shift + g] : 0.0f;
+  }
+  if constexpr (OCC) {  // stage this replica's occupancy mask of the input buckets in LDS
+    const unsigned* occ_in = bin.occ + (size_t)r * nw;
+    for (int k = tid; k < nw; k += (int)blockDim.x) s_occ[k] = occ_in[k];
+    __syncthreads();
+  }
+  // a replica flagged before this step passes its state through unchanged (the reference stops
+  // at the first failure); the flag rows rotate like the bucket sets
+  const unsigned halt = io.halt_in[r];
+  if (tile.q == 0 && tid == 0) {
+    bclr.ovf_n[r] = 0;
+    bclr.big_n[r] = 0;
+    io.halt_clr[r] = 0u;
+    if (halt) atomicOr(&io.halt_out[r], halt);
+  }
+  const BucketsOut bo = replica_out(bout, r, nv, rep.off);
+
+  int sgn = 0;
+  long long pcs = 0, psn = 0;
+  if (active || (kCoop && !halt)) {  // a walking wave needs all of its lanes
+    if (halt) {
+      if (lane == 0) {
+        io.xycs_out[g] = me;
+        io.th_out[g] = th;
+        io.vid_out[g] = v;
+        bucket_insert<OCC>(bo, v, g);
+        if constexpr (VISITS) io.visit[g] = make_int2(-1, 0);
+      }
+    } else {
+      const GlobalSource<OCC, WAVE> src{replica_in(bin, r, nv, rep.off), io.xycs_in, io.th_in, s_occ};
+      const StepOut o = particle_step<LANES, P, WAVE, VISITS>(mesh, rep.prm, src, g, me, th, v, eta, lane, active, ww);
+      if (active && lane == 0) {
+        io.xycs_out[g] = make_float4(o.xo, o.yo, o.co, o.so);
+        io.th_out[g] = o.to;
+        io.vid_out[g] = o.L.vid;
+        io.vx[g] = o.vx;
+        io.vy[g] = o.vy;
+        io.r3x[g] = (float)o.L.X;
+        io.r3y[g] = (float)o.L.Y;
+        io.r3z[g] = (float)o.L.Z;
+        io.face[g] = o.L.face;
+        io.nbr[g] = o.nb;  // count_particle_neighbors (2DTissue.cpp:254-268)
+        bucket_insert<OCC>(bo, o.L.vid, g);
+        if (o.fl) {
+          atomicOr(&io.halt_out[r], o.fl);
+          atomicMin(&io.first_bad[r], io.step);
+        }
+        if constexpr (TAPE) {
+          io.tape_fs[g] = make_float4(o.Fx, o.Fy, o.Sx, o.Sy);
+          io.tape_q[g] = o.q;
+        }
+        if constexpr (VISITS) io.visit[g] = make_int2(o.na, (int)o.vh);
+        sgn = o.sgn;
+        pcs = __double2ll_rn((double)o.co * kPhiScale);
+        psn = __double2ll_rn((double)o.so * kPhiScale);
+      }
+    }
+  }
+  // clear this replica's bucket set consumed two steps ago (it is next step's output); last, so that
+  // no load of the step waits behind these stores
+  int* clr = bclr.count + (size_t)r * nv;
+  for (int w = tile.q * (int)blockDim.x + tid; w < nv; w += tile.nq * (int)blockDim.x) clr[w] = 0;
+  if constexpr (OCC) {
+    unsigned* clr_occ = bclr.occ + (size_t)r * nw;
+    for (int k = tile.q * (int)blockDim.x + tid; k < nw; k += tile.nq * (int)blockDim.x) clr_occ[k] = 0u;
+  }
+  const int wpb = (int)blockDim.x >> 6;
+  wave_order_partial<P>(sgn, pcs, psn, io.partial + (size_t)tile.logical * wpb + (tid >> 6));
+}
+
+template <int LANES, int P, bool OCC, bool WAVE>
+void launch_tiled_mode(int block, bool tape, const MeshDev& mesh, const ReplicaDesc* reps, const TileDesc* tiles,
+                       int n_tiles, const BucketSet& bin, const BucketSet& bout, const BucketSet& bclr,
+                       const TiledIO& io, hipStream_t st) {
+  const size_t lds = step_lds_bytes(mesh.nv, block, LANES, P, WAVE, OCC);
+  if (tape)
+    hipLaunchKernelGGL((k_step_tiled<LANES, P, true, OCC, false, WAVE>), dim3(n_tiles), dim3(block), lds, st, mesh, reps,
+                       tiles, bin, bout, bclr, io);
+  else if (io.visit)  // the visit check: the same step, recording each particle's visited set
+    hipLaunchKernelGGL((k_step_tiled<LANES, P, false, OCC, true, WAVE>), dim3(n_tiles), dim3(block), lds, st, mesh, reps,
+                       tiles, bin, bout, bclr, io);
+  else
+    hipLaunchKernelGGL((k_step_tiled<LANES, P, false, OCC, false, WAVE>), dim3(n_tiles), dim3(block), lds, st, mesh, reps,
+                       tiles, bin, bout, bclr, io);
+}
+
+// wave: crowded systems (sorted buckets, the seam-wrap loop of seam_wrap_group), compiled for up to 8
+// lanes of the sums (the shapes such systems run at); wider shapes take the plain kernel (same results)
+template <int LANES, int P, bool OCC>
+void launch_tiled_variant(int block, bool tape, bool wave, const MeshDev& mesh, const ReplicaDesc* reps,
+                          const TileDesc* tiles, int n_tiles, const BucketSet& bin, const BucketSet& bout,
+                          const BucketSet& bclr, const TiledIO& io, hipStream_t st) {
+  if constexpr (LANES <= 8) {
+    if (wave) {
+      launch_tiled_mode<LANES, P, OCC, true>(block, tape, mesh, reps, tiles, n_tiles, bin, bout, bclr, io, st);
+      return;
+    }
+  }
+  (void)wave;
+  launch_tiled_mode<LANES, P, OCC, false>(block, tape, mesh, reps, tiles, n_tiles, bin, bout, bclr, io, st);
+}
+
+}  // namespace
+
+#endif
+
+}  // namespace tissue

@@ -36,3 +36,52 @@ def test_shapes_in_turn(T, n, order):
         assert np.array_equal(sim.get_outputs().nbr, ref.get_outputs().nbr), shape
         ref.close()
     sim.close()
+
+
+def _batch(T, m, sizes, raw, monkeypatch, lanes, x, y, th):
+    monkeypatch.setenv("TISSUE_SORTED_BUCKETS", "0" if raw else "1")
+    b = T.Batch(m, sizes, [T.params(**P.PHYS, sigma=0.1)] * len(sizes))
+    monkeypatch.delenv("TISSUE_SORTED_BUCKETS")
+    b.set_mode(T.MODE_STEP_KERNEL)
+    b.set_launch(lanes, 256)
+    b.set_visit_check()
+    b.set_state(x, y, th)
+    return b
+
+
+@pytest.mark.parametrize("lanes", [1, 2, 4, 8])
+@pytest.mark.parametrize("sizes", [(1, 2, 63), (700, 1, 65), (4000,), (4000,) * 9])
+def test_walk_of_a_whole_wave(T, monkeypatch, lanes, sizes):
+    """The whole-wave walk (raw buckets, and sorted ones with more lanes than the sums' layout) where its
+    lists overflow (4,000 particles on 4,907 vertices: more occupied entries than the list holds, more
+    pairs than a round, crowded buckets) and where waves are nearly empty, on one lane per strand and
+    on several (sizes on either side of phys_lanes): raw and sorted buckets, hence two walks, give the
+    same bits, and each particle's visited set is the one a plain kernel lists."""
+    m, _ = P.mesh_and_tables(22, 0.1)
+    n = sum(sizes)
+    start = [m.random_init_host(40 + r, k) for r, k in enumerate(sizes)]
+    x, y, th = (np.concatenate([s[q] for s in start]) for q in range(3))
+    a, b = (_batch(T, m, sizes, raw, monkeypatch, lanes, x, y, th) for raw in (True, False))
+    noise = np.random.default_rng(1).normal(0, 0.1, (2, n)).astype(np.float32)
+    for q in (a, b):
+        q.stage_noise(noise)
+    for step in range(2):
+        if n <= 4000 and len(sizes) == 1:  # the sets, listed before the step that visits them
+            one = T.Sim(m, T.params(**P.PHYS, sigma=0.1), n)
+            s = a.get_state()
+            one.set_state(s.x, s.y, s.theta, s.vid)
+            lists = one.neighbor_lists()
+            one.close()
+        assert a.run(1, step) == T.OK and b.run(1, step) == T.OK
+        sa, sb = a.get_state(), b.get_state()
+        for k in ("x", "y", "theta", "vid"):
+            assert np.array_equal(getattr(sa, k), getattr(sb, k)), (step, k)
+        oa, ob = a.get_outputs(), b.get_outputs()
+        for k in ("vx", "vy", "r3d", "face", "nbr"):
+            assert np.array_equal(getattr(oa, k), getattr(ob, k)), (step, k)
+        va, vb = a.visits(), b.visits()
+        assert np.array_equal(va[0], vb[0]) and np.array_equal(va[1], vb[1]), step
+        if n <= 4000 and len(sizes) == 1:
+            assert np.array_equal(va[0], [len(q) for q in lists]), step
+    a.close()
+    b.close()
