@@ -4,6 +4,7 @@
 #include <algorithm>
 #include <climits>
 #include <cstdlib>
+#include <cstring>
 #include <mutex>
 #include <numeric>
 #include <thread>
@@ -21,6 +22,7 @@ namespace {
 constexpr int kAutoResidentMax = 256;
 constexpr int kDefaultSpl = 100;          // steps per persistent launch / per phi reduction
 constexpr size_t kMaxGraphs = 32;         // cached graph executables per engine
+constexpr size_t kBackHalfWords = 256 * 1024;  // half of an engine's pinned transfer buffer (1 MiB), at most
 constexpr int kXcds = 8;                  // MI355X: 8 XCDs, workgroups dispatched round-robin
 
 // autotuned shapes, keyed by (replicas, largest replica, particles, mesh vertices)
@@ -99,6 +101,10 @@ Engine::Engine(tissue_mesh* m, int R_, const int* n_, const tissue_params* p_) {
     // the flag rows as a run expects them at its start (each run's end leaves them so again)
     HIP_OK(launch_flags_begin(R, d_halt, d_rows, d_first_bad, stream));
     HIP_OK(hipStreamSynchronize(stream));
+    back_half = std::min<size_t>(((size_t)ntot * 7 + 63) & ~(size_t)63, kBackHalfWords);
+    HIP_OK(hipHostMalloc((void**)&back, 2 * back_half * sizeof(float), hipHostMallocMapped | hipHostMallocCoherent));
+    HIP_OK(hipHostGetDevicePointer((void**)&back_dev, back, 0));
+    for (hipEvent_t& ev : back_ev) HIP_OK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
     hist_ref.resize(R);
     hist_polar.resize(R);
     flags_acc.assign(R, 0u);
@@ -135,6 +141,13 @@ void Engine::release() {
   if (phi) (void)hipHostFree(phi);
   phi = phi_dev = nullptr;
   phi_cap = 0;
+  if (back) (void)hipHostFree(back);
+  back = back_dev = nullptr;
+  back_half = 0;
+  for (hipEvent_t& ev : back_ev) {
+    if (ev) (void)hipEventDestroy(ev);
+    ev = nullptr;
+  }
   if (h_row0) (void)hipHostFree(h_row0);
   h_row0 = nullptr;
   adjoint_release();
@@ -158,29 +171,25 @@ void Engine::set_state(const float* x, const float* y, const float* theta, const
       throw ApiError(TISSUE_E_INVALID_ARG, "position outside the UV square");
     if (vid_in && (vid_in[i] < 0 || vid_in[i] >= md.nv)) throw ApiError(TISSUE_E_INVALID_ARG, "vertex id out of range");
   }
-  float *dx = dalloc<float>(ntot), *dy = dalloc<float>(ntot), *dt = dalloc<float>(ntot);
-  try {
-    HIP_OK(hipMemcpyAsync(dx, x, ntot * sizeof(float), hipMemcpyHostToDevice, stream));
-    HIP_OK(hipMemcpyAsync(dy, y, ntot * sizeof(float), hipMemcpyHostToDevice, stream));
-    HIP_OK(hipMemcpyAsync(dt, theta, ntot * sizeof(float), hipMemcpyHostToDevice, stream));
-    adopt_state(dx, dy, dt, vid_in);
-  } catch (...) {
-    dfree(dx); dfree(dy); dfree(dt);
-    throw;
+  if (3 * (size_t)ntot <= 2 * back_half) {  // read by the kernel from pinned memory
+    std::copy(x, x + ntot, back);
+    std::copy(y, y + ntot, back + ntot);
+    std::copy(theta, theta + ntot, back + 2 * (size_t)ntot);
+    adopt_state(back_dev, back_dev + ntot, back_dev + 2 * (size_t)ntot, vid_in);
+  } else {  // through output buffers that the adoption overwrites
+    HIP_OK(hipMemcpyAsync(vx, x, ntot * sizeof(float), hipMemcpyHostToDevice, stream));
+    HIP_OK(hipMemcpyAsync(vy, y, ntot * sizeof(float), hipMemcpyHostToDevice, stream));
+    HIP_OK(hipMemcpyAsync(r3x, theta, ntot * sizeof(float), hipMemcpyHostToDevice, stream));
+    adopt_state(vx, vy, r3x, vid_in);
   }
-  dfree(dx); dfree(dy); dfree(dt);
 }
 
-// the state from device arrays x, y, theta (and host vertex ids, or located when null)
+// the state from arrays x, y, theta the GPU can read (and host vertex ids, or located when null)
 void Engine::adopt_state(const float* dx, const float* dy, const float* dt, const int32_t* vid_in) {
   const int cur = sphase;
-  HIP_OK(launch_prepare(ntot, dx, dy, dt, xycs[cur], th[cur], stream));
+  HIP_OK(launch_adopt(ntot, dx, dy, dt, xycs[cur], th[cur], vx, vy, nbr, R, d_halt, stream));
   HIP_OK(launch_locate(md, ntot, xycs[cur], vid[cur], face, r3x, r3y, r3z, stream));
   if (vid_in) HIP_OK(hipMemcpyAsync(vid[cur], vid_in, ntot * sizeof(int), hipMemcpyHostToDevice, stream));
-  HIP_OK(hipMemsetAsync(vx, 0, ntot * sizeof(float), stream));
-  HIP_OK(hipMemsetAsync(vy, 0, ntot * sizeof(float), stream));
-  HIP_OK(hipMemsetAsync(nbr, 0, ntot * sizeof(int), stream));
-  HIP_OK(hipMemsetAsync(d_halt, 0, R * sizeof(unsigned), stream));
   HIP_OK(hipStreamSynchronize(stream));
   buckets_stale = true;
   has_state = true;
@@ -190,45 +199,56 @@ void Engine::adopt_state(const float* dx, const float* dy, const float* dt, cons
 void Engine::init_random(const uint64_t* seeds) {
   if (!seeds) throw ApiError(TISSUE_E_INVALID_ARG, "null seeds");
   uint64_t* ds = dalloc<uint64_t>(R);
-  float *dx = dalloc<float>(ntot), *dy = dalloc<float>(ntot), *dt = dalloc<float>(ntot);
   try {
     HIP_OK(hipMemcpyAsync(ds, seeds, R * sizeof(uint64_t), hipMemcpyHostToDevice, stream));
-    HIP_OK(launch_init_random(ntot, d_rid, d_reps, ds, mesh->d_cdf, md, dx, dy, dt, stream));
-    adopt_state(dx, dy, dt, nullptr);
+    HIP_OK(launch_init_random(ntot, d_rid, d_reps, ds, mesh->d_cdf, md, vx, vy, r3x, stream));
+    adopt_state(vx, vy, r3x, nullptr);
   } catch (...) {
-    dfree(ds); dfree(dx); dfree(dy); dfree(dt);
+    dfree(ds);
     throw;
   }
-  dfree(ds); dfree(dx); dfree(dy); dfree(dt);
+  dfree(ds);
+}
+
+// in pieces of half the pinned buffer: a piece is packed while the one before is copied out
+template <class Pack, class Take>
+void Engine::read_back(int words_each, Pack&& pack, Take&& take) {
+  const int per = (int)std::min<size_t>((size_t)ntot, back_half / words_each);
+  for (int first = 0, half = 0; first < ntot + per; first += per, half ^= 1) {
+    if (first < ntot) {
+      pack(first, std::min(per, ntot - first), back_dev + half * back_half);
+      HIP_OK(hipEventRecord(back_ev[half], stream));
+    }
+    if (first >= per) {
+      HIP_OK(hipEventSynchronize(back_ev[half ^ 1]));
+      take(first - per, std::min(per, ntot - (first - per)), back + (half ^ 1) * back_half);
+    }
+  }
 }
 
 void Engine::get_state(float* x, float* y, float* theta, int32_t* vid_out) {
   const int cur = sphase;
-  std::vector<float4> q(ntot);
-  HIP_OK(hipMemcpyAsync(q.data(), xycs[cur], ntot * sizeof(float4), hipMemcpyDeviceToHost, stream));
-  if (theta) HIP_OK(hipMemcpyAsync(theta, th[cur], ntot * sizeof(float), hipMemcpyDeviceToHost, stream));
-  if (vid_out) HIP_OK(hipMemcpyAsync(vid_out, vid[cur], ntot * sizeof(int), hipMemcpyDeviceToHost, stream));
-  HIP_OK(hipStreamSynchronize(stream));
-  for (int i = 0; i < ntot; ++i) {
-    if (x) x[i] = q[i].x;
-    if (y) y[i] = q[i].y;
-  }
+  read_back(4, [&](int first, int n, float* out) {
+    HIP_OK(launch_pack_state(first, n, xycs[cur], th[cur], vid[cur], out, stream));
+  }, [&](int first, int n, const float* w) {
+    if (x) std::copy(w, w + n, x + first);
+    if (y) std::copy(w + n, w + 2 * (size_t)n, y + first);
+    if (theta) std::copy(w + 2 * (size_t)n, w + 3 * (size_t)n, theta + first);
+    if (vid_out) std::memcpy(vid_out + first, w + 3 * (size_t)n, n * sizeof(int32_t));
+  });
 }
 
 void Engine::get_outputs(float* ovx, float* ovy, float* r3d, int32_t* oface, int32_t* onbr) {
-  std::vector<float> a(ntot), b(ntot), c(ntot);
-  if (ovx) HIP_OK(hipMemcpyAsync(ovx, vx, ntot * sizeof(float), hipMemcpyDeviceToHost, stream));
-  if (ovy) HIP_OK(hipMemcpyAsync(ovy, vy, ntot * sizeof(float), hipMemcpyDeviceToHost, stream));
-  if (oface) HIP_OK(hipMemcpyAsync(oface, face, ntot * sizeof(int), hipMemcpyDeviceToHost, stream));
-  if (onbr) HIP_OK(hipMemcpyAsync(onbr, nbr, ntot * sizeof(int), hipMemcpyDeviceToHost, stream));
-  if (r3d) {
-    HIP_OK(hipMemcpyAsync(a.data(), r3x, ntot * sizeof(float), hipMemcpyDeviceToHost, stream));
-    HIP_OK(hipMemcpyAsync(b.data(), r3y, ntot * sizeof(float), hipMemcpyDeviceToHost, stream));
-    HIP_OK(hipMemcpyAsync(c.data(), r3z, ntot * sizeof(float), hipMemcpyDeviceToHost, stream));
-  }
-  HIP_OK(hipStreamSynchronize(stream));
-  if (r3d)
-    for (int i = 0; i < ntot; ++i) { r3d[3 * i] = a[i]; r3d[3 * i + 1] = b[i]; r3d[3 * i + 2] = c[i]; }
+  read_back(7, [&](int first, int n, float* out) {
+    HIP_OK(launch_pack_outputs(first, n, vx, vy, r3x, r3y, r3z, face, nbr, out, stream));
+  }, [&](int first, int n, const float* w) {
+    const size_t k = n;
+    if (ovx) std::copy(w, w + k, ovx + first);
+    if (ovy) std::copy(w + k, w + 2 * k, ovy + first);
+    if (r3d) std::copy(w + 2 * k, w + 5 * k, r3d + 3 * (size_t)first);
+    if (oface) std::memcpy(oface + first, w + 5 * k, k * sizeof(int32_t));
+    if (onbr) std::memcpy(onbr + first, w + 6 * k, k * sizeof(int32_t));
+  });
 }
 
 // ------------------------------------------------------------------ buckets and tiles
@@ -259,10 +279,7 @@ size_t Engine::bucket_set_bytes() const {
 // outside any capture: clear set b (count and list lengths), on stream st (null: the engine's)
 void Engine::clear_bucket_set(BucketSet& b, hipStream_t st) {
   if (!st) st = stream;
-  HIP_OK(hipMemsetAsync(b.count, 0, (size_t)R * md.nv * sizeof(int), st));
-  HIP_OK(hipMemsetAsync(b.occ, 0, (size_t)R * tdev::occ_words(md.nv) * sizeof(unsigned), st));
-  HIP_OK(hipMemsetAsync(b.ovf_n, 0, R * sizeof(int), st));
-  HIP_OK(hipMemsetAsync(b.big_n, 0, R * sizeof(int), st));
+  HIP_OK(launch_clear_sets(R, md.nv, &b, 1, st));
 }
 
 // outside any capture: clear set b, bucket the vertex ids v into it and sort its buckets, on
@@ -289,13 +306,7 @@ void Engine::bucket_state(const int* v, int k) { bucket_state_into(v, bs[k]); }
 // outside any capture: clear every set, bucket the current state into set bphase
 void Engine::rebuild_buckets() {
   ensure_buckets();
-  const size_t cells = (size_t)R * md.nv;
-  for (int k = 0; k < 3; ++k) {
-    HIP_OK(hipMemsetAsync(bs[k].count, 0, cells * sizeof(int), stream));
-    HIP_OK(hipMemsetAsync(bs[k].occ, 0, (size_t)R * tdev::occ_words(md.nv) * sizeof(unsigned), stream));
-    HIP_OK(hipMemsetAsync(bs[k].ovf_n, 0, R * sizeof(int), stream));
-    HIP_OK(hipMemsetAsync(bs[k].big_n, 0, R * sizeof(int), stream));
-  }
+  HIP_OK(launch_clear_sets(R, md.nv, bs, 3, stream));
   bucket_state(vid[sphase], bphase);
   buckets_stale = false;
 }
@@ -403,7 +414,12 @@ const float* Engine::upload_call_noise(const float* h, int n_steps) {
     call_noise = dalloc<float>(need);
     call_noise_cap = need;
   }
-  HIP_OK(hipMemcpyAsync(call_noise, h, need * sizeof(float), hipMemcpyHostToDevice, stream));
+  if (need <= 2 * back_half) {  // (the call's run is waited for, so the pinned words are free by the next use)
+    std::copy(h, h + need, back);
+    HIP_OK(launch_fetch(need, back_dev, call_noise, stream));
+  } else {
+    HIP_OK(hipMemcpyAsync(call_noise, h, need * sizeof(float), hipMemcpyHostToDevice, stream));
+  }
   return call_noise;
 }
 

@@ -31,6 +31,7 @@ struct Engine {
   Engine& operator=(const Engine&) = delete;
 
   // state of all replicas, concatenated (replica r at off[r])
+  // dx, dy may be vx, vy; dt anything but a buffer of the state
   void adopt_state(const float* dx, const float* dy, const float* dt, const int32_t* vid_in);
   void set_state(const float* x, const float* y, const float* theta, const int32_t* vid);
   void init_random(const uint64_t* seeds);
@@ -132,6 +133,16 @@ struct Engine {
   double* phi = nullptr;
   double* phi_dev = nullptr;
   size_t phi_cap = 0;
+  // pinned, mapped host memory through which states and outputs pass (the GPU reads and writes it
+  // directly, the host copies from and to the caller's arrays): two halves of back_half words, used in
+  // turn; back_ev marks a half's last pack
+  float* back = nullptr;
+  float* back_dev = nullptr;
+  size_t back_half = 0;
+  hipEvent_t back_ev[2] = {nullptr, nullptr};
+  // words_each words per particle packed by pack(first, n, device address) and taken by take(first, n, words)
+  template <class Pack, class Take>
+  void read_back(int words_each, Pack&& pack, Take&& take);
   float* noise = nullptr;  // staged rows
   int noise_rows = 0;      // rows of the last staging (the valid ones)
   int noise_cap = 0;       // rows the buffer holds

@@ -229,13 +229,68 @@ __global__ void k_flags_end(int R, const unsigned* last_row, unsigned* halt, int
   first_bad[r] = INT_MAX;
 }
 
-__global__ void k_prepare(int n, const float* x, const float* y, const float* th, float4* xycs, float* th_out) {
+// the state from x, y, theta (device memory, or mapped host memory: each value is read once), with no
+// velocity, neighbour count or flag yet; x, y and theta may be vx, vy and a buffer written later
+__global__ void k_adopt(int n, const float* x, const float* y, const float* th, float4* xycs, float* th_out, float* vx,
+                        float* vy, int* nbr, int R, unsigned* halt) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < R) halt[i] = 0u;  // R <= n: a replica holds a particle at least
+  if (i >= n) return;
+  const float xi = x[i], yi = y[i], ti = th[i];
+  float s, c;
+  sincosf(ti, &s, &c);
+  xycs[i] = make_float4(xi, yi, c, s);
+  th_out[i] = ti;
+  vx[i] = 0.f;
+  vy[i] = 0.f;
+  nbr[i] = 0;
+}
+
+// particles [first, first + n) of the state and of the outputs, laid out as the caller's arrays are, into
+// mapped host memory (consecutive lanes write consecutive words)
+__global__ void k_pack_state(int first, int n, const float4* xycs, const float* th, const int* vid, float* out) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  float s, c;
-  sincosf(th[i], &s, &c);
-  xycs[i] = make_float4(x[i], y[i], c, s);
-  th_out[i] = th[i];
+  const float4 q = xycs[first + i];
+  out[i] = q.x;
+  out[(size_t)n + i] = q.y;
+  out[2 * (size_t)n + i] = th[first + i];
+  reinterpret_cast<int*>(out)[3 * (size_t)n + i] = vid[first + i];
+}
+
+__global__ void k_pack_outputs(int first, int n, const float* vx, const float* vy, const float* r3x, const float* r3y,
+                               const float* r3z, const int* face, const int* nbr, float* out) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;  // a word of r3d [n][3]; the first n also one of each other
+  if (t >= 3 * n) return;
+  const int i = t / 3, c = t - 3 * i;
+  out[2 * (size_t)n + t] = (c == 0 ? r3x : (c == 1 ? r3y : r3z))[first + i];
+  if (t >= n) return;
+  out[t] = vx[first + t];
+  out[(size_t)n + t] = vy[first + t];
+  reinterpret_cast<int*>(out)[5 * (size_t)n + t] = face[first + t];
+  reinterpret_cast<int*>(out)[6 * (size_t)n + t] = nbr[first + t];
+}
+
+// words of mapped host memory into device memory
+__global__ void k_fetch(size_t n, const float* from, float* to) {
+  const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+  if (i < n) to[i] = from[i];
+}
+
+// the counts, masks and list lengths of three bucket sets
+__global__ void k_clear_sets(size_t cells, size_t words, int R, BucketSet a, BucketSet b, BucketSet c, int sets) {
+  const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const BucketSet& s = k == 0 ? a : (k == 1 ? b : c);
+    if (k >= sets) break;
+    if (i < cells) s.count[i] = 0;
+    if (i < words) s.occ[i] = 0u;
+    if (i < (size_t)R) {
+      s.ovf_n[i] = 0;
+      s.big_n[i] = 0;
+    }
+  }
 }
 
 // seam wrap of n moves, LANES lanes per move (the step kernel's lane groups); whole groups only
@@ -383,9 +438,35 @@ hipError_t launch_flags_end(int R, const unsigned* last_row, unsigned* halt, int
   return hipGetLastError();
 }
 
-hipError_t launch_prepare(int n, const float* x, const float* y, const float* th, float4* xycs, float* th_out,
-                          hipStream_t st) {
-  hipLaunchKernelGGL(k_prepare, dim3(cdiv(n, 256)), dim3(256), 0, st, n, x, y, th, xycs, th_out);
+hipError_t launch_adopt(int n, const float* x, const float* y, const float* th, float4* xycs, float* th_out, float* vx,
+                        float* vy, int* nbr, int R, unsigned* halt, hipStream_t st) {
+  hipLaunchKernelGGL(k_adopt, dim3(cdiv(n, 256)), dim3(256), 0, st, n, x, y, th, xycs, th_out, vx, vy, nbr, R, halt);
+  return hipGetLastError();
+}
+
+hipError_t launch_pack_state(int first, int n, const float4* xycs, const float* th, const int* vid, float* out,
+                             hipStream_t st) {
+  hipLaunchKernelGGL(k_pack_state, dim3(cdiv(n, 256)), dim3(256), 0, st, first, n, xycs, th, vid, out);
+  return hipGetLastError();
+}
+
+hipError_t launch_pack_outputs(int first, int n, const float* vx, const float* vy, const float* r3x, const float* r3y,
+                               const float* r3z, const int* face, const int* nbr, float* out, hipStream_t st) {
+  hipLaunchKernelGGL(k_pack_outputs, dim3(cdiv(3l * n, 256)), dim3(256), 0, st, first, n, vx, vy, r3x, r3y, r3z, face,
+                     nbr, out);
+  return hipGetLastError();
+}
+
+hipError_t launch_fetch(size_t n, const float* from, float* to, hipStream_t st) {
+  hipLaunchKernelGGL(k_fetch, dim3(cdiv((long)n, 256)), dim3(256), 0, st, n, from, to);
+  return hipGetLastError();
+}
+
+hipError_t launch_clear_sets(int R, int nv, const BucketSet* sets, int n_sets, hipStream_t st) {
+  const BucketSet &a = sets[0], &b = sets[n_sets > 1 ? 1 : 0], &c = sets[n_sets > 2 ? 2 : 0];
+  hipLaunchKernelGGL(k_clear_sets, dim3(cdiv((long)R * nv, 256)), dim3(256), 0, st, (size_t)R * nv, (size_t)R * occ_words(nv),
+                     R, a, b, c,
+                     n_sets);
   return hipGetLastError();
 }
 

@@ -209,8 +209,20 @@ hipError_t launch_flags_begin(int R, const unsigned* halt, unsigned* rows, int* 
 hipError_t launch_flags_end(int R, const unsigned* last_row, unsigned* halt, int* first_bad, unsigned* tail,
                             unsigned* next_out_row, hipStream_t st);
 
-hipError_t launch_prepare(int n, const float* x, const float* y, const float* th, float4* xycs, float* th_out,
-                          hipStream_t st);
+// the state of n particles from x, y, theta (device or mapped host memory; x, y may be vx, vy), velocities,
+// neighbour counts and the R replicas' halt flags zeroed
+hipError_t launch_adopt(int n, const float* x, const float* y, const float* th, float4* xycs, float* th_out, float* vx,
+                        float* vy, int* nbr, int R, unsigned* halt, hipStream_t st);
+// particles [first, first + n) as consecutive arrays at out (mapped host memory): x, y, theta, vid [n]
+// (16 bytes a particle); vx, vy [n], r3d [n][3], face, nbr [n] (28 bytes)
+hipError_t launch_pack_state(int first, int n, const float4* xycs, const float* th, const int* vid, float* out,
+                             hipStream_t st);
+hipError_t launch_pack_outputs(int first, int n, const float* vx, const float* vy, const float* r3x, const float* r3y,
+                               const float* r3z, const int* face, const int* nbr, float* out, hipStream_t st);
+// n words of mapped host memory into device memory
+hipError_t launch_fetch(size_t n, const float* from, float* to, hipStream_t st);
+// counts, masks and list lengths of n_sets (1 to 3) bucket sets of R replicas zeroed
+hipError_t launch_clear_sets(int R, int nv, const BucketSet* sets, int n_sets, hipStream_t st);
 hipError_t launch_locate(const tdev::MeshDev& mesh, int n, const float4* xycs, int* vid, int* face, float* r3x,
                          float* r3y, float* r3z, hipStream_t st);
 // copy step t's outputs into the per-step output ring (when its global step number, ctl[1] + t + 1,
