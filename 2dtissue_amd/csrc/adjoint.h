@@ -23,21 +23,45 @@ struct LossDev {
 // per replica: out[2r] = phi_T, out[2r+1] = order loss; seeds lr = 0, lt = d loss / d theta_T
 hipError_t launch_adj_seed(int R, const ReplicaDesc* reps, const float4* xycs, const LossDev& L, const unsigned* halt,
                            float2* lr, float* lt, double* out, hipStream_t st);
-// per particle factors of step t's reverse (see adjoint.hip), accumulators acc[kAdjAcc][ntot];
-// the adjoint state of replica r is stored scaled by 2^-E_r: the kernel reads E_r from sexp_in and
-// the max |lambda| of its input from mx_in (the previous gather's), scales its input by a power of
-// two when that max exceeds 2^21, writes the new E_r to sexp_out and clears mx_next
-hipError_t launch_adj_local(const ReplicaDesc* reps, const int* rid, int ntot, const LossDev& L, const unsigned* halt,
-                            const int* sexp_in, int* sexp_out, const unsigned* mx_in, unsigned* mx_next,
-                            const float4* xycs, const float* th, const float4* fs, const int* quarter,
-                            const float2* lr_in, const float* lt_in, float2* gF, float2* gSC, float4* part,
-                            double* acc, hipStream_t st);
-// the transposed neighbour sums over step t's vertex buckets bs; mx_out[r] = max |lambda| of the
-// output of replica r (float bits, combined with atomicMax: clear it before)
-hipError_t launch_adj_gather(int lanes, const tdev::MeshDev& mesh, const ReplicaDesc* reps, const int* rid, int ntot,
-                             const BucketSet& bs, const unsigned* halt, const float4* xycs, const int* vid,
-                             const float2* gF, const float2* gSC, const float4* part, float2* lr_out, float* lt_out,
-                             unsigned* mx_out, hipStream_t st);
+// One launch of the reverse pass (adjoint.hip), by `lanes` (1 to 16) lanes per particle: kFactors: step p's
+// factors from the adjoint (lr_in, lt_in) of the state after it; kGather: the adjoint (lr_out, lt_out)
+// of the state before step q from step q's factors; kBoth: kGather of q, then kFactors of p = q - 1.
+// Accumulators acc[kAdjAcc][ntot]. The adjoint state of replica r is stored scaled by 2^-E_r: the
+// factors' exponent is sexp_in, raised by s_up when the max |lambda| in mx_in (float bits; kFactors: of
+// its input, kBoth: of the step before, from which sup_in has been taken already) exceeds 2^21, and
+// goes with s_up to sexp_out and sup_out; a gather posts its max to mx_out with atomicMax; mx_clear is
+// zeroed for a later launch.
+enum RevPart { kFactors = 0, kGather = 1, kBoth = 2 };
+struct RevStep {
+  BucketSet bs;             // vertex buckets of step q's input state
+  const unsigned* halt;     // [R]
+  int single;               // 1: one replica (rid is not read)
+  int use_occ;              // 1: bs holds its occupancy mask, and few vertices are occupied
+  const float4* xycs_q;     // step q's input state
+  const int* vid_q;
+  const float4* g4_in;      // step q's factors: (lF.x, lF.y, d loss / d sum sin, d loss / d sum cos)
+  const float4* part_in;    // and the particles' own terms (x, y, theta)
+  const float4* xycs_p;     // step p's input state and tape
+  const float* th_p;
+  const float4* fs_p;
+  const int* quarter_p;
+  const float2* lr_in;
+  const float* lt_in;
+  float4* g4_out;
+  float4* part_out;
+  float2* lr_out;
+  float* lt_out;
+  double* acc;
+  const int* sexp_in;
+  const int* sup_in;
+  const unsigned* mx_in;
+  int* sexp_out;
+  int* sup_out;
+  unsigned* mx_out;
+  unsigned* mx_clear;
+};
+hipError_t launch_adj_reverse(int lanes, int part, const tdev::MeshDev& mesh, const ReplicaDesc* reps, const int* rid,
+                              int ntot, const LossDev& L, const RevStep& a, hipStream_t st);
 // out[kAdjAcc r + k] = sum over replica r of acc[k]
 hipError_t launch_adj_reduce(int R, const ReplicaDesc* reps, int ntot, const double* acc, double* out, hipStream_t st);
 

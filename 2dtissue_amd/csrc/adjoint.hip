@@ -13,14 +13,21 @@
 //   lS_i  = rho lt_i C_i / Q_i,  lC_i = -rho lt_i S_i / Q_i,  Q_i = C_i^2 + S_i^2;
 //   lt_i  = (1 - rho) lt_i + s_i lrdot . (-sin, cos) + cos theta_i sum_{j in A_i} lS_j - sin theta_i sum_{j in A_i} lC_j.
 // The neighbour relation is symmetric (the geodesic table is min-symmetrised), so the transposed
-// sums are gathers over the particle's own neighbour set: k_adj_local computes the per-particle
-// factors, k_adj_gather walks the same geodesic rows and vertex buckets as the forward step.
+// sums are gathers over the particle's own neighbour set, along the same geodesic rows and vertex
+// buckets as the forward step. A particle's factors of step t (lF, lS, lC, what its neighbours gather)
+// follow from its own adjoint of the new state alone, so one kernel does the gather of step t and the
+// factors of step t - 1 (k_adj_reverse, kBoth); the first step's factors and the last step's gather
+// run by themselves (kFactors, kGather), and so does every step where a segment's tape is recomputed.
 // The adjoint state of replica r is held as lambda * 2^-E_r (FP32, E_r >= 0 in sexp[r]): the map
 // is linear in lambda, so only the loss sources are scaled by 2^-E_r and the FP64 parameter
-// accumulators by 2^E_r. E_r is raised whenever |lambda| outgrows 2^20: k_adj_gather records each
-// replica's max |lambda| (one atomic per wave), and the next k_adj_local scales its inputs by the
-// matching power of two and carries E_r forward (E and the max alternate between two slots per
-// replica by step parity, so no kernel reads a slot another thread of it writes).
+// accumulators by 2^E_r. E_r is raised whenever |lambda| outgrows 2^20: the gather records each
+// replica's max |lambda| (one atomic per wave), and the next factors are scaled by the matching power
+// of two and carry E_r forward. In kBoth the factors follow in the same kernel, before that max is
+// complete, so they go by the max of the step before, less the scaling it has caused already: one step
+// later than kFactors, |lambda| then reaches 2^20 times one more step's growth, far inside FP32. The
+// scaling is exact either way, so both give the same
+// gradients (but for values 2^-126 below their replica's largest, which underflow in one or the other). (Slots alternate by step, so that no
+// kernel reads one that another thread of it writes.)
 #include <hip/hip_runtime.h>
 
 #include "adjoint.h"
@@ -31,19 +38,28 @@ namespace tissue {
 
 namespace {
 
-__device__ __forceinline__ void field_eval(const LossDev& L, float x, float y, float& ux, float& uy, float& jxx,
-                                           float& jxy, float& jyx, float& jyy) {
-  ux = uy = jxx = jxy = jyx = jyy = 0.f;
+// the target field u and its Jacobian at (x, y), by a group of G lanes: each lane evaluates one mode at a
+// time, and all add the modes in order
+struct Field { float ux, uy, jxx, jxy, jyx, jyy; };
+
+template <int G>
+__device__ __forceinline__ Field field_eval(const LossDev& L, float x, float y, int lane) {
+  Field f{0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  for (int m0 = 0; m0 < L.n_modes; m0 += G) {
+    const int m = min(m0 + lane, L.n_modes - 1);
+    const float kx = L.kx[m], ky = L.ky[m], amp = L.amp[m];
+    float s, c;
+    sincosf(kx * x + ky * y + L.phase[m], &s, &c);
+    const float v = amp * s, d = amp * c, dx = d * kx, dy = d * ky;
 #pragma unroll
-  for (int m = 0; m < kMaxModes; ++m) {
-    if (m < L.n_modes) {
-      float s, c;
-      sincosf(L.kx[m] * x + L.ky[m] * y + L.phase[m], &s, &c);
-      const float v = L.amp[m] * s, d = L.amp[m] * c;
-      if (L.comp[m] == 0) { ux += v; jxx += d * L.kx[m]; jxy += d * L.ky[m]; }
-      else { uy += v; jyx += d * L.kx[m]; jyy += d * L.ky[m]; }
+    for (int l = 0; l < G; ++l) {
+      if (m0 + l >= L.n_modes) break;  // uniform
+      const float vl = G == 1 ? v : __shfl(v, l, G), xl = G == 1 ? dx : __shfl(dx, l, G), yl = G == 1 ? dy : __shfl(dy, l, G);
+      if (L.comp[m0 + l] == 0) { f.ux += vl; f.jxx += xl; f.jxy += yl; }
+      else { f.uy += vl; f.jyx += xl; f.jyy += yl; }
     }
   }
+  return f;
 }
 
 // R_q^T v for a rotation by q counter-clockwise quarter turns
@@ -99,12 +115,12 @@ __global__ void k_adj_seed(const ReplicaDesc* reps, const float4* xycs, LossDev 
   }
 }
 
-// power-of-two exponent that brings a replica's max |lambda| (float bits of a non-negative value)
-// below 2^21; 0 when no rescale is needed or the max is not finite
-__device__ __forceinline__ int rescale_exponent(unsigned mx_bits) {
+// power-of-two exponent that brings a replica's max |lambda| (float bits of a non-negative value),
+// already scaled down by 2^-done, below 2^21; 0 when no rescale is needed or the max is not finite
+__device__ __forceinline__ int rescale_exponent(unsigned mx_bits, int done) {
   const float mx = __uint_as_float(mx_bits);
   if (!(mx > 0.f) || !isfinite(mx)) return 0;
-  const int s = ilogbf(mx) - 20;
+  const int s = ilogbf(mx) - done - 20;
   return s > 0 ? s : 0;
 }
 
@@ -117,23 +133,22 @@ struct AdjLocal {
   float ls, m, ltn, wv, dvx, dvy;
 };
 
-__device__ __forceinline__ AdjLocal adj_local(const StepParams& prm, const LossDev& L, int n_r, float down, float src,
-                                              float4 me, float4 f, int quarter, float2 lr_s, float lt_s) {
+__device__ __forceinline__ AdjLocal adj_local(const StepParams& prm, const LossDev& L, const Field& u, int n_r,
+                                              float down, float src, float4 me, float4 f, int quarter, float2 lr_s,
+                                              float lt_s) {
   AdjLocal o;
   const float2 lp = rot_t(quarter, make_float2(lr_s.x * down, lr_s.y * down));
   o.ltn = lt_s * down;
   o.m = sqrtf(f.x * f.x + f.y * f.y);
   const float s = prm.v0 + prm.mu * o.m;
   const float rdx = me.z * s, rdy = me.w * s;
-  float ux, uy, jxx, jxy, jyx, jyy;
-  field_eval(L, me.x, me.y, ux, uy, jxx, jxy, jyx, jyy);
   o.wv = L.w_velocity / ((float)L.n_steps * (float)n_r);
-  o.dvx = rdx - ux;
-  o.dvy = rdy - uy;
+  o.dvx = rdx - u.ux;
+  o.dvy = rdy - u.uy;
   const float sw = 2.f * o.wv * src;
   const float lrdx = prm.dt * lp.x + sw * o.dvx, lrdy = prm.dt * lp.y + sw * o.dvy;
-  o.lrx = lp.x - sw * (jxx * o.dvx + jyx * o.dvy);
-  o.lry = lp.y - sw * (jxy * o.dvx + jyy * o.dvy);
+  o.lrx = lp.x - sw * (u.jxx * o.dvx + u.jyx * o.dvy);
+  o.lry = lp.y - sw * (u.jxy * o.dvx + u.jyy * o.dvy);
   o.ls = lrdx * me.z + lrdy * me.w;
   const float lm = prm.mu * o.ls;
   o.lF = o.m > 0.f ? make_float2(lm * f.x / o.m, lm * f.y / o.m) : make_float2(0.f, 0.f);
@@ -144,12 +159,17 @@ __device__ __forceinline__ AdjLocal adj_local(const StepParams& prm, const LossD
   return o;
 }
 
-// parameter gradients and the velocity loss of particle g, accumulated in FP64 (true units)
-__device__ __forceinline__ void adj_accumulate(const StepParams& prm, const AdjLocal& o, float4 f, float theta,
-                                               double unscale, double* acc, size_t ntot, int g) {
+// the turn towards the mean heading, wrapped
+__device__ __forceinline__ double mean_turn(float4 f, float theta) {
   double delta = atan2((double)f.w, (double)f.z) - (double)theta;
   if (delta > kPi) delta -= 2.0 * kPi;
   else if (delta <= -kPi) delta += 2.0 * kPi;
+  return delta;
+}
+
+// parameter gradients and the velocity loss of particle g, accumulated in FP64 (true units)
+__device__ __forceinline__ void adj_accumulate(const StepParams& prm, const AdjLocal& o, float4 f, double delta,
+                                               double unscale, double* acc, size_t ntot, int g) {
   const double tau = prm.dt64 / prm.rate64;
   acc[g] += unscale * (double)o.ls;                                            // d v0
   acc[ntot + g] += unscale * (double)o.ls * (double)o.m;                       // d mu
@@ -157,38 +177,6 @@ __device__ __forceinline__ void adj_accumulate(const StepParams& prm, const AdjL
     acc[2 * ntot + g] += unscale * ((double)o.lF.x * f.x + (double)o.lF.y * f.y) / prm.k64;
   acc[3 * ntot + g] += unscale * (double)o.ltn * delta * (-prm.dt64 / (tau * tau));  // d tau
   acc[4 * ntot + g] += (double)o.wv * ((double)o.dvx * o.dvx + (double)o.dvy * o.dvy);  // loss
-}
-
-__global__ void k_adj_local(const ReplicaDesc* reps, const int* rid, int ntot, LossDev L, const unsigned* halt,
-                            const int* sexp_in, int* sexp_out, const unsigned* mx_in, unsigned* mx_next,
-                            const float4* xycs, const float* th, const float4* fs, const int* quarter,
-                            const float2* lr_in, const float* lt_in, float2* gF, float2* gSC, float4* part,
-                            double* acc) {
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= ntot) return;
-  const int r = rid[g];
-  // rescale of the incoming adjoint (exact: a power of two); the replica's first particle carries
-  // the exponent forward and clears the max slot the following gather fills
-  const int s_up = rescale_exponent(mx_in[r]);
-  const int E = sexp_in[r] + s_up;
-  if (g == reps[r].off) {
-    sexp_out[r] = E;
-    mx_next[r] = 0u;
-  }
-  if (halt[r]) {
-    gF[g] = make_float2(0.f, 0.f);
-    gSC[g] = make_float2(0.f, 0.f);
-    part[g] = make_float4(0.f, 0.f, 0.f, 0.f);
-    return;
-  }
-  const StepParams& prm = reps[r].prm;
-  const float4 f = fs[g];  // (Fx, Fy, sum cos, sum sin)
-  const AdjLocal o = adj_local(prm, L, reps[r].n, ldexpf(1.f, -s_up), ldexpf(1.f, -E), xycs[g], f, quarter[g],
-                               lr_in[g], lt_in[g]);
-  gF[g] = o.lF;
-  gSC[g] = o.lsc;
-  part[g] = make_float4(o.lrx, o.lry, o.lth, 0.f);
-  adj_accumulate(prm, o, f, th[g], ldexp(1.0, E), acc, (size_t)ntot, g);
 }
 
 // each replica's max |lambda| over the wave: the wave's particles of one replica occupy a
@@ -209,58 +197,169 @@ __device__ __forceinline__ void post_replica_max(int r, float mx, unsigned* mx_o
   if ((me_lane == 63 || r_next != r) && r >= 0 && mx > 0.f) atomicMax(&mx_out[r], __float_as_uint(mx));
 }
 
-template <int LANES>
-__global__ void __launch_bounds__(256) k_adj_gather(MeshDev mesh, const ReplicaDesc* reps, const int* rid, int ntot,
-                                                   BucketSet bs, const unsigned* halt, const float4* xycs,
-                                                   const int* vid, const float2* gF, const float2* gSC,
-                                                   const float4* part, float2* lr_out, float* lt_out,
-                                                   unsigned* mx_out) {
+// One particle's G lanes. PART: kFactors (step p's factors from lr_in, lt_in), kGather (step q's gather to
+// lr_out, lt_out) or kBoth (step q's gather, then step p = q - 1's factors from it). The gather's sums
+// are laid out over the G lanes like the step's (lane l adds entries l, l + G, .. of the row). A chain
+// of dependent loads (vertex, row, entries, bucket heads, factors) on few waves: entries and heads are
+// loaded side by side from clamped addresses, a neighbour's four factors in one load, and what needs
+// no neighbour (the field, the accumulators' arc tangent) runs between the chain's first loads. With
+// use_occ the occupancy mask, a bit per vertex, is asked first: on a large mesh the counts and slots of
+// the mostly empty rows of sparse replicas are some 500 MB of lines a step (64 x 2,000 particles on
+// 100,265 vertices), the masks stay in the L2s.
+template <int G, int PART>
+__global__ void __launch_bounds__(256) k_adj_reverse(MeshDev mesh, const ReplicaDesc* __restrict__ reps,
+                                                    const int* __restrict__ rid, int ntot, LossDev L, RevStep a) {
   const int tid = blockIdx.x * blockDim.x + threadIdx.x;
-  const int g = tid / LANES, lane = tid & (LANES - 1);
-  const int r = g < ntot ? rid[g] : -1;  // -1: past the end (the lanes stay for the wave reduction)
-  float mx = 0.f;                        // |lambda| of this particle (on lane 0 of its group)
-  if (r >= 0 && halt[r]) {
-    if (lane == 0) { lr_out[g] = make_float2(0.f, 0.f); lt_out[g] = 0.f; }
-  } else if (r >= 0) {
-    const ReplicaDesc& rep = reps[r];
+  const int g = tid / G, lane = tid & (G - 1);
+  const int gc = min(g, ntot - 1);
+  // every load that needs no other first, then the row's bounds
+  int r = a.single ? 0 : rid[gc];
+  int v = 0;
+  float4 mine, me, pt, me_p, f = make_float4(0.f, 0.f, 0.f, 0.f);  // f: step p's (Fx, Fy, sum cos, sum sin)
+  float th_p = 0.f;
+  int quarter = 0;
+  if constexpr (PART != kFactors) {
+    v = a.vid_q[gc];
+    mine = a.g4_in[gc];
+    me = a.xycs_q[gc];
+    pt = a.part_in[gc];
+  }
+  if constexpr (PART != kGather) {
+    me_p = a.xycs_p[gc];
+    f = a.fs_p[gc];
+    th_p = a.th_p[gc];
+    quarter = a.quarter_p[gc];
+  }
+  int rs = 0, re = 0;
+  if constexpr (PART != kFactors) {
+    rs = load_at(mesh.row_ptr, v);
+    re = load_at(mesh.row_ptr, v + 1);
+  }
+  const ReplicaDesc& rep = reps[r];
+  const bool halted = a.halt[r] != 0u;
+  if (g >= ntot) r = -1;  // past the end (the lanes stay for the wave reduction)
+  float mx = 0.f;         // |lambda| of this particle (on lane 0 of its group)
+  if (r >= 0) {
     const StepParams& prm = rep.prm;
-    const int nv = mesh.nv;
-    const BucketsIn b = replica_in(bs, r, nv, rep.off);
-    const float2 mine = gF[g];
-    float ax = 0.f, ay = 0.f, aS = 0.f, aC = 0.f;
-    const int v = vid[g];
-    const int rs = mesh.row_ptr[v], re = mesh.row_ptr[v + 1];
-    for (int e = rs + lane; e < re; e += LANES) {
-      const int2 ent = mesh.nbr[e];
-      const float d = __int_as_float(ent.y);
-      if (d > prm.t_near) break;  // rows ascend in distance
-      const float c = pair_coef(d, prm);
-      for_bucket(b, ent.x, [&](int j) {
-        const float2 oj = gF[j];
-        const float2 sc = gSC[j];
-        if (j != g) {
-          ax += c * (mine.x - oj.x);
-          ay += c * (mine.y - oj.y);
-        }
-        aS += sc.x;
-        aC += sc.y;
-      });
+    // the scaling of this launch's factors; the replica's first particle carries the exponent forward
+    // and clears the max slot of the next launch
+    int s_up = 0, E = 0;
+    if constexpr (PART != kGather) {
+      s_up = rescale_exponent(a.mx_in[r], PART == kBoth ? a.sup_in[r] : 0);
+      E = a.sexp_in[r] + s_up;
+      if (g == rep.off && lane == 0) {
+        a.sexp_out[r] = E;
+        a.sup_out[r] = s_up;
+        a.mx_clear[r] = 0u;
+      }
     }
-    ax = group_sum<LANES>(ax);
-    ay = group_sum<LANES>(ay);
-    aS = group_sum<LANES>(aS);
-    aC = group_sum<LANES>(aC);
-    if (lane == 0) {
-      const float4 pt = part[g];
-      const float4 me = xycs[g];
-      const float2 o = make_float2(pt.x + ax, pt.y + ay);
-      const float ot = pt.z + me.z * aS - me.w * aC;
-      lr_out[g] = o;
-      lt_out[g] = ot;
-      mx = fmaxf(fabsf(o.x), fmaxf(fabsf(o.y), fabsf(ot)));  // fmaxf skips NaN
+    float2 lr = make_float2(0.f, 0.f);
+    float lt = 0.f;
+    Field u{};
+    double delta = 0.0;
+    if constexpr (PART == kFactors) {
+      lr = a.lr_in[g];
+      lt = a.lt_in[g];
+      u = field_eval<G>(L, me_p.x, me_p.y, lane);
+      delta = mean_turn(f, th_p);
+    } else if (!halted) {
+      const int nv = mesh.nv;
+      const BucketsIn b = replica_in(a.bs, r, nv, rep.off);
+      if constexpr (PART == kBoth) u = field_eval<G>(L, me_p.x, me_p.y, lane);
+      float ax = 0.f, ay = 0.f, aS = 0.f, aC = 0.f;
+      auto add = [&](float c, int j, const float4& o) __attribute__((always_inline)) {
+        if (j != g) {
+          ax += c * (mine.x - o.x);
+          ay += c * (mine.y - o.y);
+        }
+        aS += o.z;
+        aC += o.w;
+      };
+      constexpr int kChunk = G >= 8 ? 2 : 4;
+      int2 ent[kChunk];
+      auto load_entries = [&](int base) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < kChunk; ++k) {
+          const int e = base + k * G;
+          ent[k] = load_at(mesh.nbr, min(e, re - 1));
+          if (e >= re) ent[k].y = 0x7f800000;
+        }
+      };
+      int base = rs + lane;
+      load_entries(base);
+      if constexpr (PART == kBoth) delta = mean_turn(f, th_p);
+      for (;;) {
+        int c[kChunk];
+        int2 s[kChunk];
+        bool want[kChunk];
+#pragma unroll
+        for (int k = 0; k < kChunk; ++k) want[k] = __int_as_float(ent[k].y) <= prm.t_near;
+        if (a.use_occ) {  // uniform
+          const unsigned* occ = a.bs.occ + (size_t)r * occ_words(nv);
+          unsigned word[kChunk];
+#pragma unroll
+          for (int k = 0; k < kChunk; ++k) word[k] = load_at(occ, (want[k] ? ent[k].x : 0) >> 5);
+#pragma unroll
+          for (int k = 0; k < kChunk; ++k) want[k] = want[k] && ((word[k] >> (ent[k].x & 31)) & 1u) != 0u;
+        }
+#pragma unroll
+        for (int k = 0; k < kChunk; ++k) {
+          const int w = want[k] ? ent[k].x : 0;
+          c[k] = load_at(b.count, w);
+          s[k] = load_at(reinterpret_cast<const int2*>(b.slot), w * (kSlots / 2));
+        }
+        // the first two particles of every entry, side by side
+        float4 o0[kChunk], o1[kChunk];
+#pragma unroll
+        for (int k = 0; k < kChunk; ++k) {
+          if (!want[k]) c[k] = 0;
+          if (c[k] == 2 && !b.sorted && s[k].x > s[k].y) s[k] = make_int2(s[k].y, s[k].x);
+          o0[k] = load_at(a.g4_in, c[k] == 1 || c[k] == 2 ? s[k].x : 0);
+          o1[k] = load_at(a.g4_in, c[k] == 2 ? s[k].y : 0);
+        }
+#pragma unroll
+        for (int k = 0; k < kChunk; ++k) {
+          if (c[k] == 0) continue;
+          const float co = pair_coef(__int_as_float(ent[k].y), prm);
+          if (c[k] <= 2) {
+            add(co, s[k].x, o0[k]);
+            if (c[k] == 2) add(co, s[k].y, o1[k]);
+          } else {
+            for_bucket(b, ent[k].x, [&](int j) { add(co, j, load_at(a.g4_in, j)); });
+          }
+        }
+        if (__int_as_float(ent[kChunk - 1].y) > prm.t_near) break;  // rows ascend in distance
+        base += kChunk * G;
+        load_entries(base);
+      }
+      ax = group_sum<G>(ax);
+      ay = group_sum<G>(ay);
+      aS = group_sum<G>(aS);
+      aC = group_sum<G>(aC);
+      lr = make_float2(pt.x + ax, pt.y + ay);
+      lt = pt.z + me.z * aS - me.w * aC;
+      if (lane == 0) mx = fmaxf(fabsf(lr.x), fmaxf(fabsf(lr.y), fabsf(lt)));  // fmaxf skips NaN
+    }
+    if constexpr (PART == kGather) {
+      if (lane == 0) {
+        a.lr_out[g] = lr;
+        a.lt_out[g] = lt;
+      }
+    } else if (halted) {
+      if (lane == 0) {
+        a.g4_out[g] = make_float4(0.f, 0.f, 0.f, 0.f);
+        a.part_out[g] = make_float4(0.f, 0.f, 0.f, 0.f);
+      }
+    } else {
+      const AdjLocal o = adj_local(prm, L, u, rep.n, ldexpf(1.f, -s_up), ldexpf(1.f, -E), me_p, f, quarter, lr, lt);
+      if (lane == 0) {
+        a.g4_out[g] = make_float4(o.lF.x, o.lF.y, o.lsc.x, o.lsc.y);
+        a.part_out[g] = make_float4(o.lrx, o.lry, o.lth, 0.f);
+        adj_accumulate(prm, o, f, delta, ldexp(1.0, E), a.acc, (size_t)ntot, g);
+      }
     }
   }
-  post_replica_max(r, mx, mx_out);
+  if constexpr (PART != kFactors) post_replica_max(r, mx, a.mx_out);
 }
 
 // one block per replica: sums of the per-particle accumulators
@@ -286,35 +385,28 @@ hipError_t launch_adj_seed(int R, const ReplicaDesc* reps, const float4* xycs, c
   return hipGetLastError();
 }
 
-hipError_t launch_adj_local(const ReplicaDesc* reps, const int* rid, int ntot, const LossDev& L, const unsigned* halt,
-                            const int* sexp_in, int* sexp_out, const unsigned* mx_in, unsigned* mx_next,
-                            const float4* xycs, const float* th, const float4* fs, const int* quarter,
-                            const float2* lr_in, const float* lt_in, float2* gF, float2* gSC, float4* part,
-                            double* acc, hipStream_t st) {
-  hipLaunchKernelGGL(k_adj_local, dim3(cdiv(ntot, 256)), dim3(256), 0, st, reps, rid, ntot, L, halt, sexp_in, sexp_out,
-                     mx_in, mx_next, xycs, th, fs, quarter, lr_in, lt_in, gF, gSC, part, acc);
-  return hipGetLastError();
-}
-
-hipError_t launch_adj_gather(int lanes, const MeshDev& mesh, const ReplicaDesc* reps, const int* rid, int ntot,
-                             const BucketSet& bs, const unsigned* halt, const float4* xycs, const int* vid,
-                             const float2* gF, const float2* gSC, const float4* part, float2* lr_out, float* lt_out,
-                             unsigned* mx_out, hipStream_t st) {
-  const int blocks = cdiv((long)ntot * lanes, 256);
-#define TISSUE_ADJ_GATHER(L)                                                                                     \
-  hipLaunchKernelGGL(k_adj_gather<L>, dim3(blocks), dim3(256), 0, st, mesh, reps, rid, ntot, bs, halt, xycs, vid, \
-                     gF, gSC, part, lr_out, lt_out, mx_out)
+hipError_t launch_adj_reverse(int lanes, int part, const MeshDev& mesh, const ReplicaDesc* reps, const int* rid, int ntot,
+                              const LossDev& L, const RevStep& a, hipStream_t st) {
+#define TISSUE_ADJ_PART(G, PART)                                                                                    \
+  hipLaunchKernelGGL((k_adj_reverse<G, PART>), dim3(cdiv((long)ntot * G, 256)), dim3(256), 0, st, mesh, reps, rid, ntot, \
+                     L, a)
+#define TISSUE_ADJ_LANES(G)                                                   \
+  case G:                                                                     \
+    if (part == kFactors) TISSUE_ADJ_PART(G, kFactors);                       \
+    else if (part == kGather) TISSUE_ADJ_PART(G, kGather);                    \
+    else if (part == kBoth) TISSUE_ADJ_PART(G, kBoth);                        \
+    else return hipErrorInvalidValue;                                         \
+    break
   switch (lanes) {
-    case 1: TISSUE_ADJ_GATHER(1); break;
-    case 2: TISSUE_ADJ_GATHER(2); break;
-    case 4: TISSUE_ADJ_GATHER(4); break;
-    case 8: TISSUE_ADJ_GATHER(8); break;
-    case 16: TISSUE_ADJ_GATHER(16); break;
-    case 32: TISSUE_ADJ_GATHER(32); break;
-    case 64: TISSUE_ADJ_GATHER(64); break;
+    TISSUE_ADJ_LANES(1);
+    TISSUE_ADJ_LANES(2);
+    TISSUE_ADJ_LANES(4);
+    TISSUE_ADJ_LANES(8);
+    TISSUE_ADJ_LANES(16);
     default: return hipErrorInvalidValue;
   }
-#undef TISSUE_ADJ_GATHER
+#undef TISSUE_ADJ_LANES
+#undef TISSUE_ADJ_PART
   return hipGetLastError();
 }
 

@@ -284,10 +284,13 @@ void Engine::clear_bucket_set(BucketSet& b, hipStream_t st) {
 
 // outside any capture: clear set b, bucket the vertex ids v into it and sort its buckets, on
 // stream st (null: the engine's)
-void Engine::bucket_state_into(const int* v, BucketSet& b, hipStream_t st) {
+void Engine::bucket_state_into(const int* v, BucketSet& b, hipStream_t st, const int* held) {
   if (!st) st = stream;
   if (!d_tiles) ensure_tiles(resolve_tiled());
-  clear_bucket_set(b, st);
+  if (held && 8L * ntot < (long)R * md.nv)  // few particles per vertex: clear where they are
+    HIP_OK(launch_clear_held(ntot, held, d_rid, R, md.nv, b, st));
+  else
+    clear_bucket_set(b, st);
   HIP_OK(launch_insert(ntot, v, d_rid, d_reps, md.nv, b, st));
   if (!raw_buckets)
     HIP_OK(launch_bucket_finalize(std::get<1>(tiles_key), d_reps, d_tiles, n_phys, md.nv, R == 1 ? ntot : 0, b, st));
@@ -470,7 +473,7 @@ Shape Engine::resolve_for(Shape s) const {
   return s;
 }
 
-void Engine::enqueue(const Shape& s, int n_steps, const float* nz, size_t stride) {
+void Engine::enqueue(const Shape& s, int n_steps, const float* nz, size_t stride, Tape* tape) {
   // flag rows rotate by step (t % 3); the first step reads the flags raised before the run from
   // d_halt itself, and finds its output row cleared and first_bad reset by the previous run's end
   // (or the construction)
@@ -515,16 +518,27 @@ void Engine::enqueue(const Shape& s, int n_steps, const float* nz, size_t stride
         io.first_bad = d_first_bad;
         io.step = t;
         io.visit = d_visit;
-        BucketSet out = bs[(bp + 1) % 3];
-        if (raw_buckets) out.multi = nullptr;  // no finalize pass reads the sort list
-        HIP_OK(launch_step_tiled(s.lanes, phys_lanes(s), s.block, false, !raw_buckets, md, d_reps, d_tiles, n_phys, bs[bp], out, bs[(bp + 2) % 3],
-                                 io, stream));
+        if (tape) {
+          const size_t N = ntot;
+          io.xycs_in = tape->xycs + t * N; io.th_in = tape->th + t * N; io.vid_in = tape->vid + t * N;
+          io.xycs_out = tape->xycs + (t + 1) * N; io.th_out = tape->th + (t + 1) * N; io.vid_out = tape->vid + (t + 1) * N;
+          io.tape_fs = tape->fs + t * N;
+          io.tape_q = tape->q + t * N;
+        }
+        // a tape that keeps every state's buckets has a set per step; else three in turn
+        BucketSet* sets = tape ? (adj.keep_sets ? adj.sets.data() + t : nullptr) : nullptr;
+        const int b0 = tape ? t : bp;
+        const BucketSet in = sets ? sets[0] : bs[b0 % 3], clr = sets ? sets[2] : bs[(b0 + 2) % 3],
+                        next = sets ? sets[1] : bs[(b0 + 1) % 3];
+        BucketSet out = next;
+        if (raw_buckets) out.multi = nullptr;  // no finalize pass reads the marks
+        HIP_OK(launch_step_tiled(s.lanes, phys_lanes(s), s.block, tape != nullptr, !raw_buckets, md, d_reps, d_tiles,
+                                 n_phys, in, out, clr, io, stream));
         if (rec)
           HIP_OK(launch_record(ntot, d_row0, t, rec->every, rec->depth, io.xycs_out, r3x, r3y, r3z, nbr, rec->d_ring,
                                rec->d_ring_nbr, stream));
         if (!raw_buckets)
-          HIP_OK(launch_bucket_finalize(s.block, d_reps, d_tiles, n_phys, md.nv, R == 1 ? ntot : 0, bs[(bp + 1) % 3],
-                                        stream));
+          HIP_OK(launch_bucket_finalize(s.block, d_reps, d_tiles, n_phys, md.nv, R == 1 ? ntot : 0, next, stream));
         sp = 1 - sp;
         bp = (bp + 1) % 3;
       }
@@ -561,7 +575,7 @@ int32_t Engine::run_shape(const Shape& s, int n_steps, const float* nz, size_t s
   return status;
 }
 
-int32_t Engine::run_once(const Shape& s, int n_steps, const float* nz, size_t stride, int row0) {
+int32_t Engine::run_once(const Shape& s, int n_steps, const float* nz, size_t stride, int row0, Tape* tape) {
   if (!has_state) throw ApiError(TISSUE_E_INVALID_ARG, "no state: call init_random or set_state first");
   if (n_steps < 0) throw ApiError(TISSUE_E_INVALID_ARG, "negative step count");
   if (n_steps == 0) return TISSUE_OK;
@@ -591,11 +605,11 @@ int32_t Engine::run_once(const Shape& s, int n_steps, const float* nz, size_t st
     const bool occ = stage_occupancy(md.nv, s.block, s.lanes, phys_lanes(s));
     if (occ && !occ_kept) buckets_stale = true;  // the sets were filled without the masks this shape reads
     occ_kept = occ;
-    if (buckets_stale) rebuild_buckets();
+    if (buckets_stale && !tape) rebuild_buckets();
   }
   const auto key = std::make_tuple(n_steps, nz, stride, s.key(), sphase, bphase);
-  auto it = graphs.find(key);
-  if (it == graphs.end()) {
+  auto it = tape ? graphs.end() : graphs.find(key);
+  if (!tape && it == graphs.end()) {
     if (graphs.size() >= kMaxGraphs) {
       HIP_OK(hipStreamSynchronize(stream));
       drop_graphs();
@@ -626,7 +640,10 @@ int32_t Engine::run_once(const Shape& s, int n_steps, const float* nz, size_t st
     row0_known = true;
   }
   HIP_OK(hipEventRecord(ev0, stream));
-  HIP_OK(hipGraphLaunch(it->second, stream));
+  if (tape)  // hundreds of launches that the GPU runs more slowly than the host makes them: no graph to build
+    enqueue(s, n_steps, nz, stride, tape);
+  else
+    HIP_OK(hipGraphLaunch(it->second, stream));
   HIP_OK(hipEventRecord(ev1, stream));
   HIP_OK(hipStreamSynchronize(stream));
   // the history, flags and first failing steps as the run's kernels wrote them

@@ -58,7 +58,9 @@ struct Engine {
   // captured step graphs do not depend on it (it is read from device memory)
   int32_t run(int n_steps, const float* noise, size_t stride, int row0 = 0);
   int32_t run_shape(const Shape& s, int n_steps, const float* noise, size_t stride, int row0 = 0);
-  int32_t run_once(const Shape& s, int n_steps, const float* noise, size_t stride, int row0);
+  // tape: record the run on a whole tape (state 0 and its buckets are in place; direct launches)
+  struct Tape;
+  int32_t run_once(const Shape& s, int n_steps, const float* noise, size_t stride, int row0, Tape* tape = nullptr);
   void record_collect(long base, int n_steps);
   Shape resolve() const;
   // the request resolved for the tiled step kernel (the adjoint records its tape there)
@@ -176,12 +178,25 @@ struct Engine {
     hipStream_t rec_stream[kMaxTapes - 1] = {};
     hipEvent_t ev_fwd = nullptr, ev_ck[kMaxTapes] = {}, ev_rec[kMaxTapes] = {}, ev_rev[kMaxTapes] = {};
     float2* lr[2] = {nullptr, nullptr}; float* lt[2] = {nullptr, nullptr};
-    float2* gF = nullptr; float2* gSC = nullptr; float4* part = nullptr;
+    float4 *g4[2] = {nullptr, nullptr}, *part[2] = {nullptr, nullptr};
+    // the whole tape of a run of whole_T steps: its bucket sets (one allocation) are those of every
+    // state (keep_sets) or two halves of kRingHalf filled ahead of the reverse pass
+    Tape whole;
+    int whole_T = 0;
+    bool keep_sets = false;
+    std::vector<BucketSet> sets;
+    unsigned char* set_slab = nullptr;
     double* acc = nullptr; double* out_seed = nullptr; double* out_red = nullptr;
+    int* sup = nullptr;   // [2][R]: the exponents' last raises
     int* sexp = nullptr;  // [2][R]: the adjoint state is stored scaled by 2^-sexp (slots alternate by step)
-    unsigned* mx = nullptr;  // [2][R]: max |lambda| of the last gather's output (float bits)
+    unsigned* mx = nullptr;  // [3][R]: max |lambda| of the last gathers' outputs (float bits)
   } adj;
   void free_tape(Tape& t);
+  static constexpr int kRingHalf = 4;
+  void alloc_set_slab(std::vector<BucketSet>& sets, int n);
+  bool whole_tape(int T);
+  void free_whole_tape();
+  void adjoint_common();
   void adjoint_buffers(int K, int C);
   void adjoint_release();
 
@@ -190,13 +205,14 @@ struct Engine {
   void ensure_buckets();
   void rebuild_buckets();
   void bucket_state(const int* vid, int set);
-  void bucket_state_into(const int* vid, BucketSet& b, hipStream_t st = nullptr);
+  // held: the vertex ids of the state whose buckets the set holds (null: anything)
+  void bucket_state_into(const int* vid, BucketSet& b, hipStream_t st = nullptr, const int* held = nullptr);
   void alloc_bucket_set(BucketSet& b);
   void free_bucket_set(BucketSet& b);
   void clear_bucket_set(BucketSet& b, hipStream_t st = nullptr);
   size_t bucket_set_bytes() const;
   void ensure_tiles(const Shape& s);
-  void enqueue(const Shape& s, int n_steps, const float* noise, size_t stride);
+  void enqueue(const Shape& s, int n_steps, const float* noise, size_t stride, Tape* tape = nullptr);
   Shape resolve_for(Shape s) const;
   int phys_lanes(const Shape& s) const { return tissue::phys_lanes(s.lanes, ntot, md.nv, s.block); }
 };

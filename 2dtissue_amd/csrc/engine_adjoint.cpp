@@ -1,14 +1,18 @@
 // Adjoint of n_steps of the step (engine side) and its C-ABI entry points.
 //
-// Forward: the tiled step kernel, with the state copied to a checkpoint every ckpt_every steps.
-// Reverse, segment by segment from the last: the segment is recomputed from its checkpoint by
-// the recording variant of the same kernel (bitwise the forward's states), which stores every
-// pre-step state, the force and alignment sums and the seam-wrap turns, and keeps the vertex
-// buckets of every state of the segment (when they fit in about 16 GB; otherwise each reverse
-// step rebuilds its state's buckets from the recorded vertex ids); then, step by step backwards,
-// the two reverse kernels (per-particle factors, then the transposed neighbour gather over the
-// step's buckets) map the adjoint of the new state to the adjoint of the old one. With several
-// tapes the recomputes of the next segments run on their own streams during that reverse pass.
+// Whole tape (the rule when it fits in about 16 GB): the forward pass is the recording variant of the step
+// kernel, which stores every pre-step state, the force and alignment sums and the seam-wrap turns, 44
+// bytes per particle-step; nothing is recomputed. The reverse pass needs the vertex buckets of every
+// state: the forward pass keeps them when they fit too, else they are made again from the recorded
+// vertex ids, a few states ahead of the reverse pass on a stream of their own. Per reverse step one
+// kernel: the transposed neighbour gather and the factors of the step before.
+// Checkpoints (longer runs, and runs that stream or check every step): the tiled step kernel, with the
+// state copied to a checkpoint every ckpt_every steps; in reverse, segment by segment from the last, the
+// segment is recomputed from its checkpoint by the recording variant (bitwise the forward's states),
+// which keeps the vertex buckets of every state of the segment when they fit (otherwise each reverse
+// step rebuilds its state's buckets), and two kernels per step (factors, gather) go backwards through
+// it. With several tapes the recomputes of the next segments run on their own streams meanwhile.
+// Every form gives the same gradients (adjoint.hip).
 #include <hip/hip_runtime.h>
 
 #include <climits>
@@ -64,8 +68,10 @@ void Engine::adjoint_release() {
   dfree(a.ck_xycs); dfree(a.ck_th); dfree(a.ck_vid);
   for (Tape& t : a.tp) free_tape(t);
   for (int k = 0; k < 2; ++k) { dfree(a.lr[k]); dfree(a.lt[k]); }
-  dfree(a.gF); dfree(a.gSC); dfree(a.part); dfree(a.acc); dfree(a.out_seed); dfree(a.out_red);
-  dfree(a.sexp); dfree(a.mx);
+  for (int k = 0; k < 2; ++k) { dfree(a.g4[k]); dfree(a.part[k]); }
+  dfree(a.acc); dfree(a.out_seed); dfree(a.out_red);
+  dfree(a.sexp); dfree(a.sup); dfree(a.mx);
+  free_whole_tape();
   if (a.ev_fwd) (void)hipEventDestroy(a.ev_fwd);
   for (int k = 0; k < kMaxTapes; ++k) {
     if (a.ev_ck[k]) (void)hipEventDestroy(a.ev_ck[k]);
@@ -77,17 +83,87 @@ void Engine::adjoint_release() {
   a = AdjointBuffers{};
 }
 
-void Engine::adjoint_buffers(int K, int C) {
+void Engine::free_whole_tape() {
+  AdjointBuffers& a = adj;
+  free_tape(a.whole);
+  dfree(a.set_slab);
+  a.sets.clear();
+  a.whole_T = 0;
+}
+
+// n bucket sets in one allocation
+void Engine::alloc_set_slab(std::vector<BucketSet>& sets, int n) {
+  const size_t cells = (size_t)R * md.nv, words = (size_t)R * tdev::occ_words(md.nv);
+  size_t o = 0;
+  auto place = [&](size_t bytes) {
+    const size_t at = o;
+    o += (bytes + 255) & ~(size_t)255;
+    return at;
+  };
+  const size_t slot = place(cells * tdev::kSlots * 4), count = place(cells * 4), occ = place(words * 4),
+               ovf = place((size_t)ntot * 8), multi = place((size_t)ntot * 4), big = place((size_t)ntot * 4),
+               ovf_n = place((size_t)R * 4), big_n = place((size_t)R * 4);
+  adj.set_slab = dalloc<unsigned char>(o * n);
+  sets.resize(n);
+  for (int k = 0; k < n; ++k) {
+    unsigned char* p = adj.set_slab + o * k;
+    sets[k] = BucketSet{(unsigned*)(p + occ), (int*)(p + count), (int*)(p + slot), (int*)(p + ovf_n), (int2*)(p + ovf),
+                        (int*)(p + multi), (int*)(p + big_n), (int*)(p + big), raw_buckets ? 0 : 1};
+  }
+}
+
+// the memory the tapes and their bucket sets may take: 16 GB, or TISSUE_ADJOINT_BUCKET_KB kilobytes
+// when that is set (a smaller one selects the other forms, which give the same gradients)
+static size_t adjoint_budget() {
+  size_t budget = size_t(16) << 30;
+  if (const char* e = std::getenv("TISSUE_ADJOINT_BUCKET_KB")) {
+    const long long kb = std::atoll(e);
+    if (kb >= 0) budget = (size_t)kb << 10;
+  }
+  return budget;
+}
+
+// a whole tape of T steps, when it may be used and fits: with the bucket sets of every state, or with
+// two halves of kRingHalf sets
+bool Engine::whole_tape(int T) {
+  AdjointBuffers& a = adj;
+  const size_t N = ntot, budget = adjoint_budget(), bytes = ((size_t)T + 1) * N * 24 + (size_t)T * N * 20;
+  if (rec || d_visit || bytes > budget) return false;
+  const size_t left = (budget - bytes) / (bucket_set_bytes() + 4096);
+  const bool keep = left >= (size_t)T + 2;
+  if (!keep && left < 2 * kRingHalf) return false;
+  const int n_sets = keep ? T + 2 : 2 * kRingHalf;
+  if (T > a.whole_T || keep != a.keep_sets || (int)a.sets.size() < n_sets) {
+    HIP_OK(hipStreamSynchronize(stream));
+    free_whole_tape();
+    for (Tape& t : a.tp) free_tape(t);  // either form's memory, not both
+    a.K = a.ntape = 0;
+    Tape& t = a.whole;
+    t.xycs = dalloc<float4>((size_t)(T + 1) * N);
+    t.th = dalloc<float>((size_t)(T + 1) * N);
+    t.vid = dalloc<int>((size_t)(T + 1) * N);
+    t.fs = dalloc<float4>((size_t)T * N);
+    t.q = dalloc<int>((size_t)T * N);
+    alloc_set_slab(a.sets, n_sets);
+    a.whole_T = T;
+    a.keep_sets = keep;
+  }
+  return true;
+}
+
+// what every form needs
+void Engine::adjoint_common() {
   AdjointBuffers& a = adj;
   const size_t N = ntot;
   if (!a.lr[0]) {
     for (int k = 0; k < 2; ++k) { a.lr[k] = dalloc<float2>(N); a.lt[k] = dalloc<float>(N); }
-    a.gF = dalloc<float2>(N); a.gSC = dalloc<float2>(N); a.part = dalloc<float4>(N);
+    for (int k = 0; k < 2; ++k) { a.g4[k] = dalloc<float4>(N); a.part[k] = dalloc<float4>(N); }
     a.acc = dalloc<double>(kAdjAcc * N);
     a.out_seed = dalloc<double>(2 * (size_t)R);
     a.out_red = dalloc<double>(kAdjAcc * (size_t)R);
     a.sexp = dalloc<int>(2 * (size_t)R);
-    a.mx = dalloc<unsigned>(2 * (size_t)R);
+    a.sup = dalloc<int>(2 * (size_t)R);
+    a.mx = dalloc<unsigned>(3 * (size_t)R);
     for (hipStream_t& st : a.rec_stream) HIP_OK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
     HIP_OK(hipEventCreateWithFlags(&a.ev_fwd, hipEventDisableTiming));
     for (int k = 0; k < kMaxTapes; ++k) {
@@ -96,6 +172,12 @@ void Engine::adjoint_buffers(int K, int C) {
       HIP_OK(hipEventCreateWithFlags(&a.ev_rev[k], hipEventDisableTiming));
     }
   }
+}
+
+void Engine::adjoint_buffers(int K, int C) {
+  AdjointBuffers& a = adj;
+  const size_t N = ntot;
+  free_whole_tape();
   if (C > a.C) {
     dfree(a.ck_xycs); dfree(a.ck_th); dfree(a.ck_vid);
     a.ck_xycs = dalloc<float4>((size_t)C * N); a.ck_th = dalloc<float>((size_t)C * N); a.ck_vid = dalloc<int>((size_t)C * N);
@@ -105,14 +187,7 @@ void Engine::adjoint_buffers(int K, int C) {
   // recomputes of two segments then run side by side while the reverse pass of a third runs;
   // else one tape, with its states' bucket sets when they fit (otherwise each reverse step
   // re-buckets its state), and everything in order on the engine's stream
-  // (the budget is TISSUE_ADJOINT_BUCKET_KB kilobytes when that is set: a smaller one selects the
-  // one-tape and re-bucketing forms, which give the same gradients)
-  const size_t sets = (size_t)K + 2;
-  size_t budget = size_t(16) << 30;
-  if (const char* e = std::getenv("TISSUE_ADJOINT_BUCKET_KB")) {
-    const long long kb = std::atoll(e);
-    if (kb >= 0) budget = (size_t)kb << 10;
-  }
+  const size_t sets = (size_t)K + 2, budget = adjoint_budget();
   int ntape = 1;
   while (ntape < kMaxTapes && (size_t)(ntape + 1) * sets * bucket_set_bytes() <= budget) ++ntape;
   const bool with_sets = sets * bucket_set_bytes() <= budget;
@@ -164,9 +239,92 @@ int32_t Engine::adjoint(int T, const float* nz, size_t stride, int K, const tiss
   const int gather_lanes = std::min(s.lanes, 16);
   ensure_buckets();
   ensure_tiles(s);
-  adjoint_buffers(K, C);
+  adjoint_common();
   AdjointBuffers& a = adj;
   const size_t N = ntot;
+  double fwd_ms = 0.0;
+  int32_t status = TISSUE_OK;
+  float2* lr_end = nullptr;  // the adjoint of the initial state and its exponents
+  float* lt_end = nullptr;
+  int* sexp_end = nullptr;
+  RevStep v{};
+  v.halt = d_halt;
+  v.single = R == 1 ? 1 : 0;
+  v.acc = a.acc;
+  auto begin_reverse = [&] {
+    HIP_OK(hipEventRecord(ev0, stream));
+    HIP_OK(launch_adj_seed(R, d_reps, xycs[sphase], L, d_halt, a.lr[0], a.lt[0], a.out_seed, stream));
+    HIP_OK(hipMemsetAsync(a.acc, 0, kAdjAcc * N * sizeof(double), stream));
+    HIP_OK(hipMemsetAsync(a.sexp, 0, 2 * R * sizeof(int), stream));
+    HIP_OK(hipMemsetAsync(a.sup, 0, 2 * R * sizeof(int), stream));
+    HIP_OK(hipMemsetAsync(a.mx, 0, 3 * R * sizeof(unsigned), stream));
+  };
+  if (whole_tape(T)) {
+    Tape& tp = a.whole;
+    HIP_OK(hipMemcpyAsync(tp.xycs, xycs[sphase], N * sizeof(float4), hipMemcpyDeviceToDevice, stream));
+    HIP_OK(hipMemcpyAsync(tp.th, th[sphase], N * sizeof(float), hipMemcpyDeviceToDevice, stream));
+    HIP_OK(hipMemcpyAsync(tp.vid, vid[sphase], N * sizeof(int), hipMemcpyDeviceToDevice, stream));
+    BucketSet* sets = a.keep_sets ? a.sets.data() : bs;
+    HIP_OK(launch_clear_sets(R, md.nv, sets + 1, 2, stream));
+    bucket_state_into(tp.vid, sets[0]);
+    buckets_stale = true;  // the sets no longer follow the engine's own phase
+    status = run_once(s, T, nz, stride, 0, &tp);
+    fwd_ms = last_ms;
+    HIP_OK(hipMemcpyAsync(xycs[sphase], tp.xycs + T * N, N * sizeof(float4), hipMemcpyDeviceToDevice, stream));
+    HIP_OK(hipMemcpyAsync(th[sphase], tp.th + T * N, N * sizeof(float), hipMemcpyDeviceToDevice, stream));
+    HIP_OK(hipMemcpyAsync(vid[sphase], tp.vid + T * N, N * sizeof(int), hipMemcpyDeviceToDevice, stream));
+    begin_reverse();
+    // half h of the ring: the buckets of the states T - 1 - h kRingHalf .. downwards
+    const int halves = (T + kRingHalf - 1) / kRingHalf;
+    hipStream_t side = a.rec_stream[0];
+    auto ring_set = [&](int q) -> BucketSet& { return a.sets[(T - 1 - q) % (2 * kRingHalf)]; };
+    auto fill = [&](int h) {
+      if (h >= halves) return;
+      if (h >= 2) HIP_OK(hipStreamWaitEvent(side, a.ev_rev[h & 1], 0));
+      for (int q = T - 1 - h * kRingHalf; q >= std::max(0, T - (h + 1) * kRingHalf); --q)
+        bucket_state_into(tp.vid + q * N, ring_set(q), side, h >= 2 ? tp.vid + (q + 2 * kRingHalf) * N : nullptr);
+      HIP_OK(hipEventRecord(a.ev_rec[h & 1], side));
+    };
+    if (!a.keep_sets) {
+      fill(0);
+      fill(1);
+    }
+    // launch j: exponents and maxima from slots that launch j - 1 wrote, to the next ones
+    int j = 0;
+    v.use_occ = !a.keep_sets && 8L * nmax < md.nv ? 1 : 0;
+    auto launch = [&](int part, int q, int p) {
+      v.sexp_in = a.sexp + (j & 1) * R; v.sexp_out = a.sexp + (1 - (j & 1)) * R;
+      v.sup_in = a.sup + (j & 1) * R; v.sup_out = a.sup + (1 - (j & 1)) * R;
+      v.mx_in = a.mx + (j + 2) % 3 * R; v.mx_out = a.mx + j % 3 * R; v.mx_clear = a.mx + (j + 1) % 3 * R;
+      v.g4_in = a.g4[1 - (j & 1)]; v.part_in = a.part[1 - (j & 1)];
+      v.g4_out = a.g4[j & 1]; v.part_out = a.part[j & 1];
+      if (q >= 0) {
+        v.bs = a.keep_sets ? a.sets[q] : ring_set(q);
+        v.xycs_q = tp.xycs + q * N; v.vid_q = tp.vid + q * N;
+      }
+      if (p >= 0) {
+        v.xycs_p = tp.xycs + p * N; v.th_p = tp.th + p * N; v.fs_p = tp.fs + p * N; v.quarter_p = tp.q + p * N;
+      }
+      HIP_OK(launch_adj_reverse(gather_lanes, part, md, d_reps, d_rid, ntot, L, v, stream));
+      ++j;
+    };
+    v.lr_in = a.lr[0]; v.lt_in = a.lt[0];
+    v.lr_out = a.lr[1]; v.lt_out = a.lt[1];
+    launch(kFactors, -1, T - 1);
+    for (int q = T - 1; q >= 0; --q) {
+      const int at = T - 1 - q, h = at / kRingHalf;
+      if (!a.keep_sets && at % kRingHalf == 0) HIP_OK(hipStreamWaitEvent(stream, a.ev_rec[h & 1], 0));
+      launch(q > 0 ? kBoth : kGather, q, q - 1);
+      if (!a.keep_sets && (at % kRingHalf == kRingHalf - 1 || q == 0)) {
+        HIP_OK(hipEventRecord(a.ev_rev[h & 1], stream));
+        fill(h + 2);
+      }
+    }
+    lr_end = a.lr[1];
+    lt_end = a.lt[1];
+    sexp_end = a.sexp + ((j - 1) & 1) * R;
+  } else {
+  adjoint_buffers(K, C);
 
   // recomputes: with nt > 1 tapes, segment c goes to tape c % nt on recompute stream c % (nt - 1),
   // nt - 1 segments ahead of the reverse passes (tapes are handed over by events); with one tape
@@ -229,19 +387,21 @@ int32_t Engine::adjoint(int T, const float* nz, size_t stride, int K, const tiss
     if (overlap) HIP_OK(hipStreamWaitEvent(stream, a.ev_rec[c % nt], 0));
     for (int q = kc - 1; q >= 0; --q) {
       if (!keep) bucket_state_into(tp.vid + q * N, bs[0], stream);
-      HIP_OK(launch_adj_local(d_reps, d_rid, ntot, L, d_halt, a.sexp + cur * R, a.sexp + (1 - cur) * R, a.mx + cur * R,
-                              a.mx + (1 - cur) * R, tp.xycs + q * N, tp.th + q * N, tp.fs + q * N, tp.q + q * N,
-                              a.lr[cur], a.lt[cur], a.gF, a.gSC, a.part, a.acc, stream));
-      HIP_OK(launch_adj_gather(gather_lanes, md, d_reps, d_rid, ntot, keep ? tp.sbs[q] : bs[0], d_halt, tp.xycs + q * N,
-                               tp.vid + q * N, a.gF, a.gSC, a.part, a.lr[1 - cur], a.lt[1 - cur],
-                               a.mx + (1 - cur) * R, stream));
+      v.bs = keep ? tp.sbs[q] : bs[0];
+      v.xycs_q = v.xycs_p = tp.xycs + q * N; v.vid_q = tp.vid + q * N; v.th_p = tp.th + q * N;
+      v.fs_p = tp.fs + q * N; v.quarter_p = tp.q + q * N;
+      v.lr_in = a.lr[cur]; v.lt_in = a.lt[cur]; v.lr_out = a.lr[1 - cur]; v.lt_out = a.lt[1 - cur];
+      v.g4_in = v.g4_out = a.g4[0]; v.part_in = v.part_out = a.part[0];
+      v.sexp_in = a.sexp + cur * R; v.sexp_out = a.sexp + (1 - cur) * R;
+      v.sup_in = a.sup + cur * R; v.sup_out = a.sup + (1 - cur) * R;
+      v.mx_in = a.mx + cur * R; v.mx_out = v.mx_clear = a.mx + (1 - cur) * R;
+      HIP_OK(launch_adj_reverse(gather_lanes, kFactors, md, d_reps, d_rid, ntot, L, v, stream));
+      HIP_OK(launch_adj_reverse(gather_lanes, kGather, md, d_reps, d_rid, ntot, L, v, stream));
       cur = 1 - cur;
     }
     if (overlap) HIP_OK(hipEventRecord(a.ev_rev[c % nt], stream));
   };
   // forward, with a checkpoint at the start of every segment
-  double fwd_ms = 0.0;
-  int32_t status = TISSUE_OK;
   for (int c = 0; c < C; ++c) {
     const int t0 = c * K, kc = std::min(K, T - t0);
     HIP_OK(hipMemcpyAsync(a.ck_xycs + c * N, xycs[sphase], N * sizeof(float4), hipMemcpyDeviceToDevice, stream));
@@ -255,14 +415,8 @@ int32_t Engine::adjoint(int T, const float* nz, size_t stride, int K, const tiss
     fwd_ms += last_ms;
     if (st != TISSUE_OK && status == TISSUE_OK) status = st;
   }
-
-
   // reverse
-  HIP_OK(hipEventRecord(ev0, stream));
-  HIP_OK(launch_adj_seed(R, d_reps, xycs[sphase], L, d_halt, a.lr[0], a.lt[0], a.out_seed, stream));
-  HIP_OK(hipMemsetAsync(a.acc, 0, kAdjAcc * N * sizeof(double), stream));
-  HIP_OK(hipMemsetAsync(a.sexp, 0, 2 * R * sizeof(int), stream));
-  HIP_OK(hipMemsetAsync(a.mx, 0, 2 * R * sizeof(unsigned), stream));
+  begin_reverse();
   if (overlap) {
     HIP_OK(hipEventRecord(a.ev_fwd, stream));  // every checkpoint is written
     for (int c = C - 1; c >= 0; --c) {
@@ -276,6 +430,10 @@ int32_t Engine::adjoint(int T, const float* nz, size_t stride, int K, const tiss
       if (c >= 1) recompute(c - 1, nullptr);
     }
   }
+  lr_end = a.lr[cur];
+  lt_end = a.lt[cur];
+  sexp_end = a.sexp + cur * R;
+  }
   HIP_OK(launch_adj_reduce(R, d_reps, ntot, a.acc, a.out_red, stream));
   HIP_OK(hipEventRecord(ev1, stream));
   std::vector<double> seed(2 * (size_t)R), red(kAdjAcc * (size_t)R);
@@ -284,9 +442,9 @@ int32_t Engine::adjoint(int T, const float* nz, size_t stride, int K, const tiss
   std::vector<int> sexp(R);
   HIP_OK(hipMemcpyAsync(seed.data(), a.out_seed, seed.size() * sizeof(double), hipMemcpyDeviceToHost, stream));
   HIP_OK(hipMemcpyAsync(red.data(), a.out_red, red.size() * sizeof(double), hipMemcpyDeviceToHost, stream));
-  HIP_OK(hipMemcpyAsync(lr.data(), a.lr[cur], N * sizeof(float2), hipMemcpyDeviceToHost, stream));
-  HIP_OK(hipMemcpyAsync(lt.data(), a.lt[cur], N * sizeof(float), hipMemcpyDeviceToHost, stream));
-  HIP_OK(hipMemcpyAsync(sexp.data(), a.sexp + cur * R, R * sizeof(int), hipMemcpyDeviceToHost, stream));
+  HIP_OK(hipMemcpyAsync(lr.data(), lr_end, N * sizeof(float2), hipMemcpyDeviceToHost, stream));
+  HIP_OK(hipMemcpyAsync(lt.data(), lt_end, N * sizeof(float), hipMemcpyDeviceToHost, stream));
+  HIP_OK(hipMemcpyAsync(sexp.data(), sexp_end, R * sizeof(int), hipMemcpyDeviceToHost, stream));
   HIP_OK(hipStreamSynchronize(stream));
   float rev = 0.f;
   HIP_OK(hipEventElapsedTime(&rev, ev0, ev1));

@@ -345,6 +345,20 @@ __global__ void k_record(int ntot, const int* ctl, int t, int every, int depth, 
   ring_nbr[slot * (size_t)ntot + i] = nbr[i];
 }
 
+// the counts, mask words and list lengths of a set that holds the state with vertex ids vid
+__global__ void k_clear_held(int ntot, const int* vid, const int* rid, int R, int nv, BucketSet bs) {
+  const int g = blockIdx.x * blockDim.x + threadIdx.x;
+  if (g >= ntot) return;
+  const int v = vid[g];
+  const size_t r = rid[g];
+  bs.count[r * nv + v] = 0;
+  bs.occ[r * occ_words(nv) + (v >> 5)] = 0u;
+  if (g < R) {
+    bs.ovf_n[g] = 0;
+    bs.big_n[g] = 0;
+  }
+}
+
 __global__ void k_locate(MeshDev mesh, int n, const float4* xycs, int* vid, int* face, float* r3x, float* r3y,
                          float* r3z) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -512,6 +526,12 @@ hipError_t launch_record(int ntot, const int* ctl, int t, int every, int depth, 
                          const float* r3y, const float* r3z, const int* nbr, float* ring, int* ring_nbr, hipStream_t st) {
   hipLaunchKernelGGL(k_record, dim3(cdiv(ntot, 256)), dim3(256), 0, st, ntot, ctl, t, every, depth, xycs, r3x, r3y,
                      r3z, nbr, ring, ring_nbr);
+  return hipGetLastError();
+}
+
+hipError_t launch_clear_held(int ntot, const int* vid, const int* rid, int R, int nv, const BucketSet& bs,
+                             hipStream_t st) {
+  hipLaunchKernelGGL(k_clear_held, dim3(cdiv(ntot, 256)), dim3(256), 0, st, ntot, vid, rid, R, nv, bs);
   return hipGetLastError();
 }
 

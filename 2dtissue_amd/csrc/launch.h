@@ -236,6 +236,8 @@ hipError_t launch_init_random(int ntot, const int* rid, const ReplicaDesc* reps,
 // wave: a wave's last flight is finished by all of its lanes (seam_wrap_group)
 hipError_t launch_seam_wrap(int lanes, int n, const double2* start, double2* end, double* dtheta, int* quarter, int* ok,
                             int max_crossings, int wave, hipStream_t st);
+// clears a bucket set that holds the state with vertex ids vid where that state is
+hipError_t launch_clear_held(int ntot, const int* vid, const int* rid, int R, int nv, const BucketSet& bs, hipStream_t st);
 // bucket every particle of every replica (rid[g] = replica of particle g) into set `bs`
 hipError_t launch_insert(int ntot, const int* vid, const int* rid, const ReplicaDesc* reps, int nv,
                          const BucketSet& bs, hipStream_t st);
