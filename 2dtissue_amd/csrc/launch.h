@@ -146,7 +146,7 @@ inline int phys_lanes(int lanes, int ntot, int nv, int block) {
   if (lanes == 2 && ntot <= 163840 && !stage_occupancy(nv, block, 2, 2)) return 4;
   return lanes;
 }
-constexpr int kResidentMaxBlock = 512;
+constexpr int kResidentMaxBlock = 512;  // of the persistent kernel's shapes; see kFullBlock in resident.hip
 
 // lanes per particle for the persistent kernel when not tuned: wider groups for smaller replicas
 inline int resident_default_lanes(int nmax) { return nmax <= 256 ? 8 : (nmax <= 1024 ? 4 : (nmax <= 2048 ? 2 : 1)); }

@@ -19,20 +19,29 @@ namespace tissue {
 
 namespace {
 
-constexpr int kMaxBlock = kResidentMaxBlock;
+// A shape's largest block, 512, means a full workgroup: 1,024 threads where their reduction words still fit
+// beside the replica in LDS (the capacity is that of 512). A CU holds one such workgroup, and its
+// steps are chains of loads and waits: 16 waves instead of 8 hide them better (MI355X, 100 steps: 256 x
+// 200 particles 3.06 -> 2.27 ms, of which 0.2 ms is the transfer of states and outputs; 100 particles,
+// 50 steps 0.92 -> 0.74 ms). The particles' results do not depend on the number of threads.
+constexpr int kFullBlock = 1024;
+constexpr size_t kLdsBytes = 160 * 1024;
 
 __host__ __device__ inline size_t align16(size_t x) { return (x + 15) & ~(size_t)15; }
 
 struct LdsLayout {
-  size_t begin, xycs, th, vid, sorted, scan, total;
-  __host__ __device__ LdsLayout(int nv, int nmax) {
+  size_t begin, xycs, th, vid, sorted, scan, red_cs, red_sn, red_sg, total;
+  __host__ __device__ LdsLayout(int nv, int nmax, int waves) {
     size_t o = 0;
     begin = o; o = align16(o + 4 * (size_t)(nv + 1));
     xycs = o; o = align16(o + 16 * (size_t)nmax);
     th = o; o = align16(o + 4 * (size_t)nmax);
     vid = o; o = align16(o + 4 * (size_t)nmax);
     sorted = o; o = align16(o + 2 * (size_t)nmax);
-    scan = o; o = align16(o + 4 * (kMaxBlock / 64));
+    scan = o; o = align16(o + 4 * (size_t)waves);
+    red_cs = o; o = align16(o + 8 * (size_t)waves);
+    red_sn = o; o = align16(o + 8 * (size_t)waves);
+    red_sg = o; o = align16(o + 4 * (size_t)waves);
     total = o;
   }
 };
@@ -86,13 +95,14 @@ __device__ void build_buckets(uint32_t* begin, uint16_t* sorted, const int* vid,
 }
 
 template <int LANES>
-__global__ void __launch_bounds__(kMaxBlock) k_resident(MeshDev mesh, const ReplicaDesc* reps, int nmax, int steps,
+__global__ void __launch_bounds__(kFullBlock) k_resident(MeshDev mesh, const ReplicaDesc* __restrict__ reps, int nmax, int steps,
                                                         ResidentIO io) {
   extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ double red_cs[kMaxBlock / 64], red_sn[kMaxBlock / 64];
-  __shared__ int red_sg[kMaxBlock / 64];
   __shared__ unsigned s_flags;
-  const LdsLayout L(mesh.nv, nmax);
+  const LdsLayout L(mesh.nv, nmax, (int)blockDim.x >> 6);
+  double* red_cs = (double*)(smem + L.red_cs);
+  double* red_sn = (double*)(smem + L.red_sn);
+  int* red_sg = (int*)(smem + L.red_sg);
   uint32_t* begin = (uint32_t*)(smem + L.begin);
   float4* xycs = (float4*)(smem + L.xycs);
   float* th = (float*)(smem + L.th);
@@ -101,7 +111,7 @@ __global__ void __launch_bounds__(kMaxBlock) k_resident(MeshDev mesh, const Repl
   uint32_t* scan_tmp = (uint32_t*)(smem + L.scan);
 
   const int r = blockIdx.x;
-  const ReplicaDesc rep = reps[r];
+  const ReplicaDesc& rep = reps[r];
   const int n = rep.n, off = rep.off;
   const int tid = threadIdx.x, nthr = blockDim.x;
   const int lane = tid & (LANES - 1), group = tid / LANES, ngroups = nthr / LANES;
@@ -193,7 +203,7 @@ __global__ void __launch_bounds__(kMaxBlock) k_resident(MeshDev mesh, const Repl
 template <int LANES>
 hipError_t launch_one(int block, const MeshDev& mesh, const ReplicaDesc* reps, int R, int nmax, int steps,
                       const ResidentIO& io, hipStream_t st) {
-  const size_t lds = LdsLayout(mesh.nv, nmax).total;
+  const size_t lds = LdsLayout(mesh.nv, nmax, block / 64).total;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   hipError_t e = hipStreamIsCapturing(st, &cap);
   if (e != hipSuccess) return e;
@@ -208,22 +218,26 @@ hipError_t launch_one(int block, const MeshDev& mesh, const ReplicaDesc* reps, i
 }  // namespace
 
 size_t resident_lds_bytes(int nv, int nmax) {
-  return LdsLayout(nv, nmax).total + sizeof(double) * 2 * (kMaxBlock / 64) + sizeof(int) * (kMaxBlock / 64) + 16;
+  return LdsLayout(nv, nmax, kResidentMaxBlock / 64).total + 16;
+}
+
+// threads of a workgroup for the shape's block
+static int resident_threads(int nv, int nmax, int block) {
+  return block == kResidentMaxBlock && LdsLayout(nv, nmax, kFullBlock / 64).total + 16 <= kLdsBytes ? kFullBlock : block;
 }
 
 int resident_max_particles(int nv) {
-  const size_t cap = 160 * 1024;
   int lo = 0, hi = 65535;
   while (lo < hi) {
     const int mid = (lo + hi + 1) / 2;
-    if (resident_lds_bytes(nv, mid) <= cap) lo = mid;
+    if (resident_lds_bytes(nv, mid) <= kLdsBytes) lo = mid;
     else hi = mid - 1;
   }
   return lo;
 }
 
 hipError_t resident_prepare(int nv, int nmax) {
-  const int lds = (int)LdsLayout(nv, nmax).total;
+  const int lds = (int)LdsLayout(nv, nmax, resident_threads(nv, nmax, kResidentMaxBlock) / 64).total;
   const void* fns[] = {(const void*)k_resident<1>, (const void*)k_resident<2>, (const void*)k_resident<4>,
                        (const void*)k_resident<8>};
   for (const void* f : fns) {
@@ -235,7 +249,8 @@ hipError_t resident_prepare(int nv, int nmax) {
 
 hipError_t launch_resident(int lanes, int block, const MeshDev& mesh, const ReplicaDesc* reps, int R, int nmax,
                            int steps, const ResidentIO& io, hipStream_t st) {
-  if (block < 64 || block > kMaxBlock || block % 64 || nmax > resident_max_particles(mesh.nv)) return hipErrorInvalidValue;
+  if (block < 64 || block > kResidentMaxBlock || block % 64 || nmax > resident_max_particles(mesh.nv)) return hipErrorInvalidValue;
+  block = resident_threads(mesh.nv, nmax, block);
   switch (lanes) {
     case 1: return launch_one<1>(block, mesh, reps, R, nmax, steps, io, st);
     case 2: return launch_one<2>(block, mesh, reps, R, nmax, steps, io, st);

@@ -135,7 +135,8 @@ int32_t tissue_neighbor_lists(tissue_sim* s, int32_t* counts, int32_t* cols, int
  * stopped; steps of the persistent kernel, TISSUE_MODE_RESIDENT, record nothing). */
 int32_t tissue_set_visit_check(tissue_sim* s, int32_t enable);
 int32_t tissue_get_visits(tissue_sim* s, int32_t* na, uint32_t* hash);
-/* launch shape: lanes per particle (1, 2, 4, 8, 16, 32, 64) and threads per block (64..512); 0 = auto */
+/* launch shape: lanes per particle (1, 2, 4, 8, 16, 32, 64) and threads per block (64..512; in the
+ * persistent kernel 512 is a full workgroup, run by 1,024 threads where they fit); 0 = auto */
 int32_t tissue_set_launch(tissue_sim* s, int32_t lanes, int32_t block);
 /* execution mode of tissue_step*: one kernel launch per step over the whole GPU, or the
  * persistent LDS-resident kernel (one workgroup, many steps per launch; needs

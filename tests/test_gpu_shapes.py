@@ -85,3 +85,31 @@ def test_walk_of_a_whole_wave(T, monkeypatch, lanes, sizes):
             assert np.array_equal(va[0], [len(q) for q in lists]), step
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("lanes", [2, 8])
+def test_full_workgroup_of_the_persistent_kernel(T, lanes):
+    """Block 512 runs as 1,024 threads where the reduction words fit beside the replica, as 512 up to the
+    capacity: states and outputs are the step kernel's at the same layout of the sums, bit for bit."""
+    m, _ = P.mesh_and_tables(32, 0.05)
+    cap = T.resident_capacity(m)
+    prm = T.params(**P.PHYS, sigma=0.05)
+    for n in (1, 64, 1025, cap - 24, cap):
+        noise = T.gen_noise(3, 0.1, 2, n)
+        got = []
+        for mode, block in ((T.MODE_RESIDENT, 512), (T.MODE_RESIDENT, 256), (T.MODE_STEP_KERNEL, 256)):
+            s = T.Sim(m, prm, n)
+            s.set_mode(mode)
+            s.set_launch(lanes, block)
+            s.init_random(9)
+            assert s.step(2, noise) == T.OK
+            st, o = s.get_state(), s.get_outputs()
+            got.append([st.x, st.y, st.theta, st.vid, o.vx, o.vy, o.r3d, o.face, o.nbr])
+            phi = s.order()
+            got[-1].append(phi[0])
+            assert np.allclose(phi[1], got[0][10] if len(got) > 1 else phi[1], rtol=0, atol=1e-12)
+            got[-1].append(phi[1])
+            s.close()
+        for other in got[1:]:
+            for a, b in zip(got[0][:10], other[:10]):
+                assert np.array_equal(a, b), n
