@@ -21,7 +21,8 @@ namespace tdev {
 constexpr double kPi = 3.141592653589793;
 constexpr float kLocateMargin = 1e-5f;   // UV units (coordinates in [0, 1])
 constexpr float kVertexMargin = 1e-4f;   // 3-D units, relative to the mesh's extent (|X| <= ~10)
-constexpr int kFaceChunk = 4;            // candidate faces per lane loaded together
+// candidate faces per lane loaded together (3.6 per cell on average)
+constexpr int face_chunk(int lanes) { return lanes >= 8 ? 1 : (lanes >= 4 ? 2 : 4); }
 
 struct MeshDev {
   int32_t nv, nf, grid, pad;
@@ -610,20 +611,20 @@ inline void pack_cell_triangle(const float* uv, const int32_t* faces, int32_t f,
   out[1] = make_float4(uv[2 * c], uv[2 * c + 1], fbits, 0.0f);
 }
 
-// Face record read once the face is chosen: corner ids a, b, c (faces[3f ..]) with their UV and
-// 3-D coordinates, (ua, ub), (uc, a, b), (A, c), (B, 0), (C, 0), ids as float bits; one load level
-// instead of the face's ids and then its corners.
+// Face record read once the face is chosen: corner ids a, b, c (faces[3f ..]) with their 3-D and UV
+// coordinates, (A, a), (B, b), (C, c), (ua, ub), (uc, 0, 0), ids as float bits; one load level instead of the
+// face's ids and then its corners, and a lane can take one corner (float4 k, float2 6 + k).
 inline void pack_face(const float* uv, const float* xyz, const int32_t* faces, int32_t f, float4* out) {
   const int32_t a = faces[3 * f], b = faces[3 * f + 1], c = faces[3 * f + 2];
   float ab, bb, cb;
   __builtin_memcpy(&ab, &a, sizeof a);
   __builtin_memcpy(&bb, &b, sizeof b);
   __builtin_memcpy(&cb, &c, sizeof c);
-  out[0] = make_float4(uv[2 * a], uv[2 * a + 1], uv[2 * b], uv[2 * b + 1]);
-  out[1] = make_float4(uv[2 * c], uv[2 * c + 1], ab, bb);
-  out[2] = make_float4(xyz[3 * a], xyz[3 * a + 1], xyz[3 * a + 2], cb);
-  out[3] = make_float4(xyz[3 * b], xyz[3 * b + 1], xyz[3 * b + 2], 0.0f);
-  out[4] = make_float4(xyz[3 * c], xyz[3 * c + 1], xyz[3 * c + 2], 0.0f);
+  out[0] = make_float4(xyz[3 * a], xyz[3 * a + 1], xyz[3 * a + 2], ab);
+  out[1] = make_float4(xyz[3 * b], xyz[3 * b + 1], xyz[3 * b + 2], bb);
+  out[2] = make_float4(xyz[3 * c], xyz[3 * c + 1], xyz[3 * c + 2], cb);
+  out[3] = make_float4(uv[2 * a], uv[2 * a + 1], uv[2 * b], uv[2 * b + 1]);
+  out[4] = make_float4(uv[2 * c], uv[2 * c + 1], 0.0f, 0.0f);
 }
 
 __host__ __device__ inline int float_bits(float x) {
@@ -781,6 +782,63 @@ __host__ __device__ inline void group_lex_min(double& d, int& f) {
   }
 }
 
+#if defined(__HIP_DEVICE_COMPILE__)
+// lane K of each quad, to all four
+template <int K, class T>
+__device__ inline T quad_lane(T v) {
+  constexpr int W = sizeof(T) / 4;
+  uint32_t w[W];
+  __builtin_memcpy(w, &v, sizeof v);
+#pragma unroll
+  for (int k = 0; k < W; ++k) w[k] = __builtin_amdgcn_update_dpp(w[k], w[k], K * 0x55, 0xf, 0xf, false);
+  __builtin_memcpy(&v, w, sizeof v);
+  return v;
+}
+
+// a + b + c over the quad's first three lanes, added in that order
+template <class T>
+__device__ inline T quad_sum3(T v) { return quad_lane<0>(v) + quad_lane<1>(v) + quad_lane<2>(v); }
+
+// The blend and the nearest vertex within the chosen face (locate), a corner per lane: one of three square
+// roots and divisions each, the same operations in the same order as the plain form.
+__device__ inline void locate_in_face_quad(const float4* fp, int lane, double px, double py, Located& r) {
+  const int q = (lane & 3) < 3 ? lane & 3 : 2;
+  const float4 V = fp[q];
+  const float2 u = reinterpret_cast<const float2*>(fp + 3)[q];
+  const int id = float_bits(V.w);
+  {
+    const float qx = (float)px, qy = (float)py;
+    float w = sqrtf(sqr(qx - u.x) + sqr(qy - u.y));
+    w /= quad_sum3(w);
+    const float X = quad_sum3(w * V.x), Y = quad_sum3(w * V.y), Z = quad_sum3(w * V.z);
+    const float d = sqrtf(sqr(X - V.x) + sqr(Y - V.y) + sqr(Z - V.z));
+    const float da = quad_lane<0>(d), db = quad_lane<1>(d), dc = quad_lane<2>(d);
+    const float mn = fminf(da, fminf(db, dc));
+    const float gap = (da == mn ? fminf(db, dc) : (db == mn ? fminf(da, dc) : fminf(da, db))) - mn;
+    if (gap > kVertexMargin && (da == mn) + (db == mn) + (dc == mn) == 1) {
+      const int ia = quad_lane<0>(id), ib = quad_lane<1>(id), ic = quad_lane<2>(id);
+      r.X = X; r.Y = Y; r.Z = Z;
+      r.vid = da == mn ? ia : (db == mn ? ib : ic);
+      return;
+    }
+  }
+  r.fp64 |= 2;
+  const double Vx = V.x, Vy = V.y, Vz = V.z;
+  double w = sqrt(sqr(px - (double)u.x) + sqr(py - (double)u.y));
+  w /= quad_sum3(w);  // CellHelper::normalize_weights (:224-230)
+  r.X = quad_sum3(w * Vx);
+  r.Y = quad_sum3(w * Vy);
+  r.Z = quad_sum3(w * Vz);
+  const double d = sqrt(sqr(r.X - Vx) + sqr(r.Y - Vy) + sqr(r.Z - Vz));
+  const double da = quad_lane<0>(d), db = quad_lane<1>(d), dc = quad_lane<2>(d);
+  double mn = da;
+  if (db < mn) mn = db;
+  if (dc < mn) mn = dc;
+  const int ia = quad_lane<0>(id), ib = quad_lane<1>(id), ic = quad_lane<2>(id);
+  r.vid = (mn == da) ? ia : ((mn == db) ? ib : ic);
+}
+#endif
+
 // CellHelper::calculate_barycentric_3D_coord (CellHelper.cpp:104-160) with the candidate faces
 // taken from the face bucket of the point's grid cell. Faces containing the point (distance 0
 // up to rounding) always share its cell, so the lexicographic (distance, face) minimum over the
@@ -799,14 +857,15 @@ __host__ __device__ inline Located locate(const MeshDev& m, double px, double py
   const float qx = (float)px, qy = (float)py;
   float b1 = __builtin_inff(), b2 = __builtin_inff();  // squared distances
   int f1 = 0x7fffffff;
-  // candidates in chunks of kFaceChunk per lane, their records loaded together (same visiting
-  // order as one at a time)
+  // candidates in chunks per lane, their records loaded together (same visiting order as one at a time)
+  constexpr int kFaceChunk = face_chunk(LANES);
   for (int q0 = cs + lane; q0 < ce; q0 += kFaceChunk * LANES) {
     float4 e0[kFaceChunk], e1[kFaceChunk];
 #pragma unroll
     for (int k = 0; k < kFaceChunk; ++k) {
-      const int q = q0 + k * LANES;
-      if (q < ce) { e0[k] = m.cell_tri[2 * q]; e1[k] = m.cell_tri[2 * q + 1]; }
+      const int q = q0 + k * LANES < ce ? q0 + k * LANES : q0;
+      e0[k] = m.cell_tri[2 * q];
+      e1[k] = m.cell_tri[2 * q + 1];
     }
 #pragma unroll
     for (int k = 0; k < kFaceChunk; ++k)
@@ -832,12 +891,19 @@ __host__ __device__ inline Located locate(const MeshDev& m, double px, double py
   }
   if (best_f == 0x7fffffff) best_f = 0;  // non-finite point: any valid face keeps indices in range
   const float4* fp = m.face_pack + 5 * (size_t)best_f;
+  r.face = best_f;
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (LANES >= 4) {  // a corner per lane of each quad
+    locate_in_face_quad(fp, lane, px, py, r);
+    return r;
+  }
+#endif
   const float4 p0 = fp[0], p1 = fp[1], p2 = fp[2], p3 = fp[3], p4 = fp[4];
-  const int ia = float_bits(p1.z), ib = float_bits(p1.w), ic = float_bits(p2.w);
-  const float2 ua = make_float2(p0.x, p0.y), ub = make_float2(p0.z, p0.w), uc = make_float2(p1.x, p1.y);
-  const float Ax = p2.x, Ay = p2.y, Az = p2.z;
-  const float Bx = p3.x, By = p3.y, Bz = p3.z;
-  const float Cx = p4.x, Cy = p4.y, Cz = p4.z;
+  const int ia = float_bits(p0.w), ib = float_bits(p1.w), ic = float_bits(p2.w);
+  const float2 ua = make_float2(p3.x, p3.y), ub = make_float2(p3.z, p3.w), uc = make_float2(p4.x, p4.y);
+  const float Ax = p0.x, Ay = p0.y, Az = p0.z;
+  const float Bx = p1.x, By = p1.y, Bz = p1.z;
+  const float Cx = p2.x, Cy = p2.y, Cz = p2.z;
   // FP32 blend and nearest-vertex choice, kept when the choice is clear
   {
     float wa = sqrtf(sqr(qx - ua.x) + sqr(qy - ua.y));
@@ -855,7 +921,6 @@ __host__ __device__ inline Located locate(const MeshDev& m, double px, double py
     if (gap > kVertexMargin && (da == mn) + (db == mn) + (dc == mn) == 1) {
       r.X = X; r.Y = Y; r.Z = Z;
       r.vid = da == mn ? ia : (db == mn ? ib : ic);
-      r.face = best_f;
       return r;
     }
   }
@@ -878,7 +943,6 @@ __host__ __device__ inline Located locate(const MeshDev& m, double px, double py
   if (db < mn) mn = db;
   if (dc < mn) mn = dc;
   r.vid = (mn == da) ? ia : ((mn == db) ? ib : ic);
-  r.face = best_f;
   return r;
 }
 
