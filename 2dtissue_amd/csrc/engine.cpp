@@ -477,6 +477,10 @@ void Engine::enqueue(const Shape& s, int n_steps, const float* nz, size_t stride
   // flag rows rotate by step (t % 3); the first step reads the flags raised before the run from
   // d_halt itself, and finds its output row cleared and first_bad reset by the previous run's end
   // (or the construction)
+  // the flags and first failing steps go right after the run's order history, in the pinned buffer
+  // that run_once reads; the run's last kernel writes them
+  const RunEnd end{d_rows + (size_t)(n_steps % 3) * R, d_halt, d_first_bad,
+                   reinterpret_cast<unsigned*>(phi_dev + 2 * (size_t)R * n_steps), d_rows + R};
   if (s.mode == TISSUE_MODE_RESIDENT) {
     ResidentIO io;
     const int cur = sphase;
@@ -495,6 +499,7 @@ void Engine::enqueue(const Shape& s, int n_steps, const float* nz, size_t stride
       io.t_base = t0;
       io.flags_in = t0 == 0 ? d_halt : d_rows + (size_t)(t0 % 3) * R;
       io.flags_out = d_rows + (size_t)((t0 + k) % 3) * R;
+      io.end = t0 + k == n_steps ? end : RunEnd{};
       HIP_OK(launch_resident(s.lanes, s.block, md, d_reps, R, nmax, k, io, stream));
     }
   } else {
@@ -543,13 +548,9 @@ void Engine::enqueue(const Shape& s, int n_steps, const float* nz, size_t stride
         bp = (bp + 1) % 3;
       }
       HIP_OK(launch_phi_tiles(R, k, d_tile_begin, n_logical, partials_per_tile(s.block), partial, d_reps, phi_dev,
-                              n_steps, t0, stream));
+                              n_steps, t0, t0 + k == n_steps ? end : RunEnd{}, stream));
     }
   }
-  // the flags and first failing steps go right after the run's order history, in the pinned
-  // buffer that run_once reads
-  unsigned* tail = reinterpret_cast<unsigned*>(phi_dev + 2 * (size_t)R * n_steps);
-  HIP_OK(launch_flags_end(R, d_rows + (size_t)(n_steps % 3) * R, d_halt, d_first_bad, tail, d_rows + R, stream));
 }
 
 int32_t Engine::run(int n_steps, const float* nz, size_t stride, int row0) {

@@ -166,42 +166,18 @@ __global__ void __launch_bounds__(kStepMaxBlock) k_bucket_finalize(const Replica
   }
 }
 
-// order parameters of replica r at step s, one workgroup per (r, s): the threads add the
-// replica's wave partials of the step in a strided split, then a wave and a workgroup sum (integer,
-// so the split does not matter)
-constexpr int kPhiBlock = 256;
+// order parameters of replica r at step s, one workgroup per (r, s)
 __global__ void __launch_bounds__(kPhiBlock) k_phi_tiles(int steps, const int* tile_begin, int n_logical, int per_tile,
                                                          const OrderPartial* partial, const ReplicaDesc* reps,
-                                                         double* phi, int phi_stride, int t_base) {
-  __shared__ long long s_cs[kPhiBlock / 64], s_sn[kPhiBlock / 64];
-  __shared__ long s_sg[kPhiBlock / 64];
+                                                         double* phi, int phi_stride, int t_base, int R, RunEnd end) {
+  // the run's last reduction also ends the run, one thread per replica in its first workgroups
+  if (end.halt) {
+    const int e = blockIdx.x * kPhiBlock + (int)threadIdx.x;
+    if (e < R) end_run(end, R, e, end.last_row[e], end.first_bad[e]);
+  }
   const int r = blockIdx.x / steps, s = blockIdx.x % steps;
-  long long cs = 0, sn = 0;
-  long sg = 0;
-  const OrderPartial* row = partial + (size_t)s * n_logical * per_tile;
-  for (int b = tile_begin[r] * per_tile + (int)threadIdx.x; b < tile_begin[r + 1] * per_tile; b += kPhiBlock) {
-    const OrderPartial p = row[b];
-    cs += p.cs;
-    sn += p.sn;
-    sg += p.sgn;
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    cs += __shfl_xor(cs, off, 64);
-    sn += __shfl_xor(sn, off, 64);
-    sg += __shfl_xor(sg, off, 64);
-  }
-  const int wave = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0) { s_cs[wave] = cs; s_sn[wave] = sn; s_sg[wave] = sg; }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < kPhiBlock / 64; ++w) { cs += s_cs[w]; sn += s_sn[w]; sg += s_sg[w]; }
-    const int n = reps[r].n;
-    const double c = (double)cs / kPhiScale, q = (double)sn / kPhiScale;
-    double* out = phi + 2 * ((size_t)r * phi_stride + t_base + s);
-    out[0] = (1.0 / n) * fabs((double)sg);
-    out[1] = sqrt(c * c + q * q) / n;
-  }
+  block_phi(partial + (size_t)s * n_logical * per_tile, tile_begin[r] * per_tile, tile_begin[r + 1] * per_tile, reps[r].n,
+            phi + 2 * ((size_t)r * phi_stride + t_base + s));
 }
 
 __global__ void k_flags_begin(int R, const unsigned* halt, unsigned* rows, int* first_bad) {
@@ -209,23 +185,6 @@ __global__ void k_flags_begin(int R, const unsigned* halt, unsigned* rows, int* 
   if (r >= R) return;
   rows[r] = halt[r];
   rows[R + r] = 0u;
-  first_bad[r] = INT_MAX;
-}
-
-__global__ void k_flags_end(int R, const unsigned* last_row, unsigned* halt, int* first_bad, unsigned* tail,
-                            unsigned* next_out_row) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= R) return;
-  const unsigned f = last_row[r];
-  const int fb = first_bad[r];
-  halt[r] = f;
-  if (tail) {  // the run's flags and first failing steps, beside its order history, for one read-back
-    tail[r] = f;
-    tail[R + r] = (unsigned)fb;
-  }
-  // what k_flags_begin would set for the next run (which reads halt itself at its first step):
-  // the first step's output row cleared, no failure yet
-  next_out_row[r] = 0u;
   first_bad[r] = INT_MAX;
 }
 
@@ -434,21 +393,14 @@ hipError_t launch_bucket_finalize(int block, const ReplicaDesc* reps, const Tile
 
 hipError_t launch_phi_tiles(int R, int steps, const int* tile_begin, int n_logical, int per_tile,
                             const OrderPartial* partial, const ReplicaDesc* reps, double* phi, int phi_stride,
-                            int t_base, hipStream_t st) {
+                            int t_base, const RunEnd& end, hipStream_t st) {
   hipLaunchKernelGGL(k_phi_tiles, dim3(R * steps), dim3(kPhiBlock), 0, st, steps, tile_begin, n_logical, per_tile,
-                     partial, reps, phi, phi_stride, t_base);
+                     partial, reps, phi, phi_stride, t_base, R, end);
   return hipGetLastError();
 }
 
 hipError_t launch_flags_begin(int R, const unsigned* halt, unsigned* rows, int* first_bad, hipStream_t st) {
   hipLaunchKernelGGL(k_flags_begin, dim3(cdiv(R, 64)), dim3(64), 0, st, R, halt, rows, first_bad);
-  return hipGetLastError();
-}
-
-hipError_t launch_flags_end(int R, const unsigned* last_row, unsigned* halt, int* first_bad, unsigned* tail,
-                            unsigned* next_out_row, hipStream_t st) {
-  hipLaunchKernelGGL(k_flags_end, dim3(cdiv(R, 64)), dim3(64), 0, st, R, last_row, halt, first_bad, tail,
-                     next_out_row);
   return hipGetLastError();
 }
 

@@ -86,6 +86,25 @@ struct TiledIO {
                             //   visited (-1, 0 for a replica passed through); null: not recorded
 };
 
+// What a run's last kernel does for every replica r besides its own work: halt = the run's last flags,
+// also to tail[r] and the first failing step to tail[R + r] (the run's read-back words), and for the
+// next run its first step's output row cleared and no failure yet. halt null: not the last kernel.
+struct RunEnd {
+  const unsigned* last_row;  // [R] the run's last flag row (the persistent kernel has them at hand)
+  unsigned* halt;
+  int* first_bad;
+  unsigned* tail;
+  unsigned* next_out_row;
+};
+
+__device__ __forceinline__ void end_run(const RunEnd& e, int R, int r, unsigned flags, int first_bad) {
+  e.halt[r] = flags;
+  e.tail[r] = flags;
+  e.tail[R + r] = (unsigned)first_bad;
+  e.next_out_row[r] = 0u;
+  e.first_bad[r] = 0x7fffffff;
+}
+
 struct ResidentIO {
   float4* xycs;           // batch state, read at launch start and written back at the end
   float* th;
@@ -109,6 +128,7 @@ struct ResidentIO {
   const unsigned* flags_in;  // [R] flags before the launch
   unsigned* flags_out;       // [R] flags after the launch
   int* first_bad;            // [R]
+  RunEnd end;
 };
 
 // largest workgroup of the tiled step kernel and of the persistent kernel (register budget of
@@ -198,17 +218,11 @@ hipError_t launch_bucket_finalize(int block, const ReplicaDesc* reps, const Tile
 // replica r's tiles are tile_begin[r] .. tile_begin[r+1]
 hipError_t launch_phi_tiles(int R, int steps, const int* tile_begin, int n_logical, int per_tile,
                             const OrderPartial* partial, const ReplicaDesc* reps, double* phi, int phi_stride,
-                            int t_base, hipStream_t st);
+                            int t_base, const RunEnd& end, hipStream_t st);
 // order-parameter partials the tiled step kernel writes per tile (one per wave)
 inline int partials_per_tile(int block) { return block / 64; }
-// run start: rows[0] = halt, rows[1] = 0, first_bad = INT_MAX; run end: halt = last row
+// run start: rows[0] = halt, rows[1] = 0, first_bad = INT_MAX
 hipError_t launch_flags_begin(int R, const unsigned* halt, unsigned* rows, int* first_bad, hipStream_t st);
-// halt = the run's last flag row; with tail, also tail[0 .. R) = the flags and tail[R .. 2R) =
-// first_bad (the run's read-back words); then, for the next run, next_out_row (the output row of
-// its first step) = 0 and first_bad = INT_MAX
-hipError_t launch_flags_end(int R, const unsigned* last_row, unsigned* halt, int* first_bad, unsigned* tail,
-                            unsigned* next_out_row, hipStream_t st);
-
 // the state of n particles from x, y, theta (device or mapped host memory; x, y may be vx, vy), velocities,
 // neighbour counts and the R replicas' halt flags zeroed
 hipError_t launch_adopt(int n, const float* x, const float* y, const float* th, float4* xycs, float* th_out, float* vx,

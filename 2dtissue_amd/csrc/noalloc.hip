@@ -6,7 +6,9 @@
 // order-parameter partials and the flag rows) lives in `scratch`, a file-scope device array of
 // kScratchBytes that each GPU the library runs on holds until the process ends. The entry point
 // calls no hipMalloc, hipFree or allocating library routine, and no hipMemsetAsync: buffers that
-// must start at zero are cleared by the set-up kernel. It launches the same step kernel as
+// must start at zero are cleared by the set-up kernel. A call is four kernels (five where buckets are
+// sorted), each some 4 us at these sizes whatever it does: set-up, bucketing of the input state, the
+// step, and one for all that follows it. It launches the same step kernel as
 // tissue_step with the same default launch shape, so its results equal one tissue_step bit for
 // bit. Calls that overlap on one GPU share its scratch and race; the array keeps the last call's
 // contents.
@@ -17,6 +19,7 @@
 #include <mutex>
 
 #include "capi_common.h"
+#include "step_kernel.h"
 
 namespace {
 
@@ -39,7 +42,6 @@ struct Layout {
   static constexpr size_t xycs_in = 0;
   static constexpr size_t xycs_out = xycs_in + al(sizeof(float4) * kMaxParticles);
   static constexpr size_t vid = xycs_out + al(sizeof(float4) * kMaxParticles);
-  static constexpr size_t rid = vid + al(sizeof(int) * kMaxParticles);
   // one bucket set: occupancy mask, count[V], slot[V * kSlots], ovf[N] (int2), multi[N], big[N],
   // counters[2]
   static constexpr size_t set_occ = 0;
@@ -50,14 +52,14 @@ struct Layout {
   static constexpr size_t set_big = set_multi + al(sizeof(int) * kMaxParticles);
   static constexpr size_t set_ctr = set_big + al(sizeof(int) * kMaxParticles);
   static constexpr size_t set_bytes = set_ctr + al(sizeof(int) * 2);
-  static constexpr size_t sets = rid + al(sizeof(int) * kMaxParticles);
+  static constexpr size_t sets = vid + al(sizeof(int) * kMaxParticles);
   static constexpr size_t partial = sets + 3 * set_bytes;
   static constexpr size_t tiles = partial + al(sizeof(OrderPartial) * kMaxTiles * (tissue::kStepMaxBlock / 64));
   static constexpr size_t rep = tiles + al(sizeof(TileDesc) * kMaxTiles);
-  static constexpr size_t tile_begin = rep + al(sizeof(ReplicaDesc));
-  static constexpr size_t rows = tile_begin + al(sizeof(int) * 2);
+  static constexpr size_t rows = rep + al(sizeof(ReplicaDesc));
   static constexpr size_t first_bad = rows + al(sizeof(unsigned) * 3);
-  static constexpr size_t total = first_bad + al(sizeof(int));
+  static constexpr size_t bad = first_bad + al(sizeof(int));  // bad vertex ids of the call, else 0
+  static constexpr size_t total = bad + al(sizeof(unsigned));
 };
 constexpr size_t kScratchBytes = TISSUE_NOALLOC_SCRATCH_BYTES;
 static_assert(Layout::total <= kScratchBytes, "scratch regions exceed the declared scratch size");
@@ -102,75 +104,66 @@ struct SetupArgs {
   const float* x;
   const float* y;
   const float* th;
-  const int* vid_in;
   float4* xycs;
-  int* vid;
-  int* rid;
-  int* counts[3];
-  unsigned* occ[3];
-  int* ctrs[3];
+  BucketSet sets[3];
   TileDesc* tiles;
   ReplicaDesc* rep;
-  int* tile_begin;
   unsigned* rows;
   int* first_bad;
-  unsigned* flags_out;
+  unsigned* bad;
   ReplicaDesc rep_value;
 };
 
-// packs the state (x, y, cos theta, sin theta), copies the vertex ids (an id outside the mesh is
-// replaced by 0 and reported with TISSUE_FLAG_BAD_INPUT, so no later access leaves its table),
-// clears the bucket sets (counts, occupancy masks, list counters) and the flag rows, and writes
-// the tile and replica descriptors
+// packs the state (x, y, cos theta, sin theta), clears the bucket sets (counts, occupancy masks, list
+// lengths) and the flag words, and writes the tile and replica descriptors
 __global__ void k_noalloc_setup(SetupArgs a) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t < a.n) {
     float s, c;
     sincosf(a.th[t], &s, &c);
     a.xycs[t] = make_float4(a.x[t], a.y[t], c, s);
-    const int v = a.vid_in[t];
-    const bool ok = v >= 0 && v < a.nv;
-    a.vid[t] = ok ? v : 0;
-    a.rid[t] = 0;
-    if (!ok) atomicOr(a.flags_out, TISSUE_FLAG_BAD_INPUT);
   }
-  if (t < a.nv) {
-    a.counts[0][t] = 0;
-    a.counts[1][t] = 0;
-    a.counts[2][t] = 0;
-  }
-  if (t < tdev::occ_words(a.nv)) {
-    a.occ[0][t] = 0u;
-    a.occ[1][t] = 0u;
-    a.occ[2][t] = 0u;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    if (t < a.nv) a.sets[k].count[t] = 0;
+    if (t < tdev::occ_words(a.nv)) a.sets[k].occ[t] = 0u;
+    if (t == 0) *a.sets[k].ovf_n = *a.sets[k].big_n = 0;
   }
   if (t < a.n_tiles) a.tiles[t] = TileDesc{0, t * a.per_tile, t, a.n_tiles, t, 0};
-  if (t < 3) {
-    a.ctrs[t][0] = 0;
-    a.ctrs[t][1] = 0;
-    a.rows[t] = 0u;
-  }
+  if (t < 3) a.rows[t] = 0u;
   if (t == 0) {
     *a.rep = a.rep_value;
-    a.tile_begin[0] = 0;
-    a.tile_begin[1] = a.n_tiles;
     *a.first_bad = INT_MAX;
+    *a.bad = 0u;
   }
 }
 
-// flags_out must start at zero before the set-up kernel can report bad vertex ids into it
-__global__ void k_noalloc_clear_flags(unsigned* flags_out) { *flags_out = 0u; }
+// copies the vertex ids (an id outside the mesh is replaced by 0 and reported with TISSUE_FLAG_BAD_INPUT,
+// so no later access leaves its table) and buckets the particles
+__global__ void k_noalloc_insert(int n, int nv, const int* vid_in, int* vid, unsigned* bad, BucketSet set) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n) return;
+  const int v = vid_in[t];
+  const bool ok = v >= 0 && v < nv;
+  vid[t] = ok ? v : 0;
+  if (!ok) atomicOr(bad, TISSUE_FLAG_BAD_INPUT);
+  tissue::bucket_insert<true>(tissue::replica_out(set, 0, nv, 0), ok ? v : 0, t);
+}
 
-// splits the new packed positions into the caller's x and y and reports the step's flags
-__global__ void k_noalloc_finish(int n, const float4* xycs, float* x, float* y, const unsigned* halt_out,
-                                 unsigned* flags_out) {
+// splits the new packed positions into the caller's x and y; workgroup 0 also reduces the order parameters
+// and reports the step's flags
+__global__ void __launch_bounds__(tissue::kPhiBlock) k_noalloc_finish(int n, const float4* xycs, float* x, float* y,
+                                                                     const OrderPartial* partial, int n_partials,
+                                                                     double* phi, const unsigned* halt_out,
+                                                                     const unsigned* bad, unsigned* flags_out) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t < n) {
     const float4 q = xycs[t];
     x[t] = q.x;
     y[t] = q.y;
   }
-  if (t == 0) atomicOr(flags_out, *halt_out);
+  if (t == 0) *flags_out = *bad | *halt_out;
+  if (blockIdx.x == 0) tissue::block_phi(partial, 0, n_partials, n, phi);
 }
 
 inline int cdiv(long a, long b) { return (int)((a + b - 1) / b); }
@@ -222,36 +215,30 @@ extern "C" int32_t tissue_step_noalloc(const tissue_mesh* mc, const tissue_param
     a.x = x_in;
     a.y = y_in;
     a.th = theta_in;
-    a.vid_in = vid_in;
     a.xycs = (float4*)(base + Layout::xycs_in);
-    a.vid = (int*)(base + Layout::vid);
-    a.rid = (int*)(base + Layout::rid);
-    for (int k = 0; k < 3; ++k) {
-      a.counts[k] = b[k].count;
-      a.occ[k] = b[k].occ;
-      a.ctrs[k] = b[k].ovf_n;
-    }
+    int* vid = (int*)(base + Layout::vid);
+    for (int k = 0; k < 3; ++k) a.sets[k] = b[k];
     a.tiles = (TileDesc*)(base + Layout::tiles);
     a.rep = (ReplicaDesc*)(base + Layout::rep);
-    a.tile_begin = (int*)(base + Layout::tile_begin);
     a.rows = (unsigned*)(base + Layout::rows);
     a.first_bad = (int*)(base + Layout::first_bad);
-    a.flags_out = flags;
+    a.bad = (unsigned*)(base + Layout::bad);
     a.rep_value = ReplicaDesc{0, n, make_step_params(*p)};
-    hipLaunchKernelGGL(k_noalloc_clear_flags, dim3(1), dim3(1), 0, st, flags);
-    HIP_OK(hipGetLastError());
     const int span = std::max(std::max(n, md.nv), n_tiles);
     hipLaunchKernelGGL(k_noalloc_setup, dim3(cdiv(span, 256)), dim3(256), 0, st, a);
     HIP_OK(hipGetLastError());
 
     // buckets of the input state (set 0), sorted when the engine's rule sorts them
-    HIP_OK(tissue::launch_insert(n, a.vid, a.rid, a.rep, md.nv, b[0], st));
+    BucketSet in = b[0];
+    if (!sorted) in.multi = nullptr;  // no finalize pass reads the marks
+    hipLaunchKernelGGL(k_noalloc_insert, dim3(cdiv(n, 256)), dim3(256), 0, st, n, md.nv, vid_in, vid, a.bad, in);
+    HIP_OK(hipGetLastError());
     if (sorted) HIP_OK(tissue::launch_bucket_finalize(block, a.rep, a.tiles, n_tiles, md.nv, n, b[0], st));
 
     TiledIO io{};
     io.xycs_in = a.xycs;
     io.th_in = theta_in;
-    io.vid_in = a.vid;
+    io.vid_in = vid;
     io.xycs_out = (float4*)(base + Layout::xycs_out);
     io.th_out = theta_out;
     io.vid_out = vid_out;
@@ -272,10 +259,9 @@ extern "C" int32_t tissue_step_noalloc(const tissue_mesh* mc, const tissue_param
     io.first_bad = a.first_bad;
     io.step = 0;
     HIP_OK(tissue::launch_step_tiled(lanes, phys, block, false, sorted != 0, md, a.rep, a.tiles, n_tiles, b[0], b[1], b[2], io, st));
-    HIP_OK(tissue::launch_phi_tiles(1, 1, a.tile_begin, n_tiles, tissue::partials_per_tile(block), io.partial, a.rep,
-                                    phi, 1, 0, st));
-    hipLaunchKernelGGL(k_noalloc_finish, dim3(cdiv(n, 256)), dim3(256), 0, st, n, io.xycs_out, x_out, y_out,
-                       io.halt_out, flags);
+    hipLaunchKernelGGL(k_noalloc_finish, dim3(cdiv(n, tissue::kPhiBlock)), dim3(tissue::kPhiBlock), 0, st, n, io.xycs_out,
+                       x_out, y_out, io.partial, n_tiles * tissue::partials_per_tile(block), phi, io.halt_out, a.bad,
+                       flags);
     HIP_OK(hipGetLastError());
     return TISSUE_OK;
   });

@@ -197,7 +197,11 @@ __global__ void __launch_bounds__(kFullBlock) k_resident(MeshDev mesh, const Rep
     io.th[off + i] = th[i];
     io.vid[off + i] = vid[i];
   }
-  if (tid == 0) io.flags_out[r] = s_flags;
+  if (tid == 0) {
+    io.flags_out[r] = s_flags;
+    // (first_bad[r] is this workgroup's alone; atomic, as its other threads' updates were)
+    if (io.end.halt) end_run(io.end, (int)gridDim.x, r, s_flags, atomicAdd(&io.first_bad[r], 0));
+  }
 }
 
 template <int LANES>

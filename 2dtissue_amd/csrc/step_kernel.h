@@ -39,6 +39,38 @@ __device__ __forceinline__ BucketsOut replica_out(const BucketSet& s, int r, int
           s.occ + (size_t)r * occ_words(nv)};
 }
 
+// order parameters of one replica and step by one workgroup of kPhiBlock threads: the threads add the wave
+// partials row[first .. last) in a strided split, then a wave and a workgroup sum (integer, so the split
+// does not matter)
+constexpr int kPhiBlock = 256;
+__device__ __forceinline__ void block_phi(const OrderPartial* row, int first, int last, int n, double* out) {
+  __shared__ long long s_cs[kPhiBlock / 64], s_sn[kPhiBlock / 64];
+  __shared__ long s_sg[kPhiBlock / 64];
+  long long cs = 0, sn = 0;
+  long sg = 0;
+  for (int b = first + (int)threadIdx.x; b < last; b += kPhiBlock) {
+    const OrderPartial p = row[b];
+    cs += p.cs;
+    sn += p.sn;
+    sg += p.sgn;
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    cs += __shfl_xor(cs, off, 64);
+    sn += __shfl_xor(sn, off, 64);
+    sg += __shfl_xor(sg, off, 64);
+  }
+  const int wave = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0) { s_cs[wave] = cs; s_sn[wave] = sn; s_sg[wave] = sg; }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kPhiBlock / 64; ++w) { cs += s_cs[w]; sn += s_sn[w]; sg += s_sg[w]; }
+    const double c = (double)cs / kPhiScale, q = (double)sn / kPhiScale;
+    out[0] = (1.0 / n) * fabs((double)sg);
+    out[1] = sqrt(c * c + q * q) / n;
+  }
+}
+
 }  // namespace
 
 #ifdef TISSUE_STEP_KERNEL  // the kernel itself, for the translation units that instantiate it
