@@ -176,12 +176,14 @@ inline int resident_default_lanes(int nmax) { return nmax <= 256 ? 8 : (nmax <= 
 // particles fills few CUs, so more lanes per particle shorten its critical path, and one-wave
 // workgroups let every wave start its walk without waiting for another at the staging barrier
 // (2,000 particles: 32 lanes in 64 threads 18.97 us, 16 in 128 19.30 us, 64 in 64 19.19 us, 8 in
-// 64 20.7 us); a single 100,000-particle system is fastest with 4 (2 lanes 10 % slower), a large
+// 64 20.7 us); beyond, workgroups of 128 leave a shorter last round than 256 (530,000 particles in 256
+// replicas 34.1 -> 33.2 ms per 200 steps, 100,000 8.57 -> 8.41 ms per 100; 64 threads the same or slower
+// again); a single 100,000-particle system is fastest with 4 (2 lanes 10 % slower), a large
 // batch with 2 (autotuned).
 inline void tiled_default_shape(int R, int ntot, int* lanes, int* block) {
   const int big_lanes = R == 1 ? 4 : 2;
   *lanes = ntot <= 4096 ? 32 : (ntot <= 8192 ? 8 : (ntot <= 65536 ? 4 : big_lanes));
-  *block = ntot <= 4096 ? 64 : 256;
+  *block = ntot <= 4096 ? 64 : 128;
 }
 
 // Replicas of a few thousand particles, at most one per two vertices, leave their vertex buckets
