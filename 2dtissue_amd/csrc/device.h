@@ -355,8 +355,9 @@ constexpr int kOwnerShift = 26;  // vertex ids below 2^26 (checked by the launch
 // One particle's update (U1-U6 of the reference step) by a group of P lanes. The sums over the
 // neighbours are laid out over LANES lanes: lane l of LANES adds the entries l, l + LANES, .. of the
 // particle's table row in order, and a butterfly adds the lanes. That layout fixes the results to the
-// bit; P >= LANES, the lanes that do the work, is free (the whole-wave walk): more than LANES where
-// waves are few and the longest chain counts (phys_lanes).
+// bit; P, the lanes that do the work, is free: more than LANES where waves are few and the longest chain
+// counts (the whole-wave walk, phys_lanes), half of 8 where that halves the passes of a workgroup (the
+// persistent kernel).
 //   me = (x, y, cos theta, sin theta) of particle i, th its heading, v its vertex id.
 // Neighbours: particles bucketed on the vertices w of row v of the geodesic table; pair
 // distance d = D[v, w]. Force and alignment for d < 2 sigma (ForceHelper.cpp:34-73,
@@ -373,63 +374,75 @@ template <int LANES, int P, bool WAVE = false, bool VISITS = false, class Src>
 __device__ __forceinline__ StepOut particle_step(const MeshDev& mesh, const StepParams& prm, const Src& src, int i, float4 me,
                                         float th, int v, float eta, int lane, bool active = true,
                                         WaveWalk* ww = nullptr) {
-  // a lane's sums: those of strand lane % LANES of the layout (its copies on the lanes above LANES equal it)
-  float Sx = 0.f, Sy = 0.f;
-  double Fx64 = 0.0, Fy64 = 0.0;  // the force, summed in FP64 (its FP32 rounding drives the FP32 path)
+  // a lane's sums: those of strand lane % LANES of the layout (its copies on the lanes above LANES equal it);
+  // with P = LANES / 2 those of strands lane and lane + P. The force is summed in FP64 (its FP32 rounding
+  // drives the FP32 path).
+  static_assert(P >= LANES || 2 * P == LANES, "one or two strands per lane");
+  constexpr int NS = P < LANES ? 2 : 1, SUMW = P < LANES ? P : LANES;
+  float Sx = 0.f, Sy = 0.f, Sx1 = 0.f, Sy1 = 0.f;  // (the second strand's, unused with one)
+  double Fx64 = 0.0, Fy64 = 0.0, Fx1 = 0.0, Fy1 = 0.0;
   const double kc64 = prm.kc64;
   int na = 0, nb = 0, nb_only = 0;  // nb_only: counted without a pair by the whole-wave scan
   unsigned vh = 0u;
   const int rs = load_at(mesh.row_ptr, v), re = active ? load_at(mesh.row_ptr, v + 1) : rs;
   // pair set-up of a near entry (vertex w at distance d, bucket head h) and its particles
-  auto visit = [&](int w, float d, const typename Src::Head& h) __attribute__((always_inline)) {
+  auto visit_into = [&](double& fx, double& fy, float& sx, float& sy, int w, float d,
+                        const typename Src::Head& h) __attribute__((always_inline)) {
     const double dd = d == 0.0f ? 0.001 : (double)d;
     const double g64 = (kc64 * (dd - prm.two_sigma64)) / dd;
     const bool counted = d != 0.0f;
     src.each_pos(w, h, [&](int j, const float4& q) __attribute__((always_inline)) {
       if (j != i) {
-        Fx64 += g64 * ((double)me.x - (double)q.x);
-        Fy64 += g64 * ((double)me.y - (double)q.y);
+        fx += g64 * ((double)me.x - (double)q.x);
+        fy += g64 * ((double)me.y - (double)q.y);
       }
-      Sx += q.z;
-      Sy += q.w;
+      sx += q.z;
+      sy += q.w;
       ++na;
       vh += visit_mix((unsigned)j);
       if (counted) ++nb;
     });
   };
+  auto visit = [&](int w, float d, const typename Src::Head& h) __attribute__((always_inline)) {
+    visit_into(Fx64, Fy64, Sx, Sy, w, d, h);
+  };
   // Each lane walks its entries rs + lane + m * LANES, m = 0, 1, .., in order.
-  if constexpr (LANES >= kHeadScanLanes && P == LANES) {
+  if constexpr (LANES >= kHeadScanLanes && P <= LANES) {
     // At most a few entries per lane: the scan loads each near entry's bucket head (count and
     // first slots) together with the entries' counts, and the lane visits its occupied entries
     // from registers: table entry -> bucket head -> particles, no reload of marked entries.
-    for (int base = rs + lane; base < re; base += kHeadChunk * LANES) {
-      int2 ent[kHeadChunk];
-      typename Src::Head hd[kHeadChunk];
+    constexpr int kChunk = kHeadChunk * NS;
+    for (int base = rs + lane; base < re; base += kChunk * P) {
+      int2 ent[kChunk];
+      typename Src::Head hd[kChunk];
 #pragma unroll
-      for (int k = 0; k < kHeadChunk; ++k) {
-        const int e = base + k * LANES;
+      for (int k = 0; k < kChunk; ++k) {
+        const int e = base + k * P;
         ent[k] = load_at(mesh.nbr, min(e, re - 1));
         if (e >= re) ent[k].y = 0x7f800000;  // +inf ends the walk
       }
-      bool oc[kHeadChunk];
+      bool oc[kChunk];
 #pragma unroll
-      for (int k = 0; k < kHeadChunk; ++k)
+      for (int k = 0; k < kChunk; ++k)
         oc[k] = __int_as_float(ent[k].y) <= prm.t_count && (!Src::kOcc || src.occupied(ent[k].x));
 #pragma unroll
-      for (int k = 0; k < kHeadChunk; ++k) {
+      for (int k = 0; k < kChunk; ++k) {
         hd[k] = src.head(oc[k] ? ent[k].x : 0);
         if (!oc[k]) hd[k].c = 0;
       }
       bool stop = false;
 #pragma unroll
-      for (int k = 0; k < kHeadChunk; ++k) {
+      for (int k = 0; k < kChunk; ++k) {
         const float d = __int_as_float(ent[k].y);
         if (d > prm.t_count) {  // rows ascend in distance
           stop = true;
           break;
         }
         if (d > prm.t_near) nb += hd[k].c;  // counted only
-        else if (hd[k].c > 0) visit(ent[k].x, d, hd[k]);
+        else if (hd[k].c > 0) {
+          if (k % NS == 0) visit(ent[k].x, d, hd[k]);
+          else visit_into(Fx1, Fy1, Sx1, Sy1, ent[k].x, d, hd[k]);
+        }
       }
       if (stop) break;
     }
@@ -677,14 +690,20 @@ __device__ __forceinline__ StepOut particle_step(const MeshDev& mesh, const Step
       }
     }
   }
-  Fx64 = group_sum<LANES>(Fx64);
-  Fy64 = group_sum<LANES>(Fy64);
+  if constexpr (NS == 2) {  // the butterfly's first level
+    Fx64 += Fx1;
+    Fy64 += Fy1;
+    Sx += Sx1;
+    Sy += Sy1;
+  }
+  Fx64 = group_sum<SUMW>(Fx64);
+  Fy64 = group_sum<SUMW>(Fy64);
   float Fx = (float)Fx64, Fy = (float)Fy64;
-  Sx = group_sum<LANES>(Sx);
-  Sy = group_sum<LANES>(Sy);
-  na = group_sum<LANES>(na);
-  vh = group_sum<LANES>(vh);
-  nb = group_sum<LANES>(nb);
+  Sx = group_sum<SUMW>(Sx);
+  Sy = group_sum<SUMW>(Sy);
+  na = group_sum<SUMW>(na);
+  vh = group_sum<SUMW>(vh);
+  nb = group_sum<SUMW>(nb);
   if constexpr (Src::kCoop && coop_walk(LANES, P, WAVE)) nb += group_sum<P>(nb_only);
 
   // speed, velocity, Euler step (Locomotion.cpp:71-84)
@@ -711,39 +730,50 @@ __device__ __forceinline__ StepOut particle_step(const MeshDev& mesh, const Step
   }
   if (weak) {
     // the alignment sum again, over the neighbours' headings in FP64
+    auto strand = [&](int first, double& sx, double& sy) __attribute__((always_inline)) {
+      for (int base = rs + first; base < re; base += kRowChunk * LANES) {
+        int2 ent[kRowChunk];
+        typename Src::Head head[kRowChunk];
+#pragma unroll
+        for (int k = 0; k < kRowChunk; ++k) {
+          const int e = base + k * LANES;
+          ent[k] = load_at(mesh.nbr, min(e, re - 1));
+          if (e >= re) ent[k].y = 0x7f800000;
+        }
+#pragma unroll
+        for (int k = 0; k < kRowChunk; ++k) {
+          const bool oc = __int_as_float(ent[k].y) <= prm.t_near && (!Src::kOcc || src.occupied(ent[k].x));
+          head[k] = src.head(oc ? ent[k].x : 0);
+          if (!oc) head[k].c = 0;
+        }
+        bool stop = false;
+#pragma unroll
+        for (int k = 0; k < kRowChunk; ++k) {
+          const float d = __int_as_float(ent[k].y);
+          if (d > prm.t_near) { stop = true; break; }
+          src.each(ent[k].x, head[k], [&](int j) {
+            double sj, cj;
+            sincos((double)src.theta(j), &sj, &cj);
+            sx += cj;
+            sy += sj;
+          });
+        }
+        if (stop) break;
+      }
+    };
     double Sx64 = 0.0, Sy64 = 0.0;
-    for (int base = rs + (lane & (LANES - 1)); base < re; base += kRowChunk * LANES) {
-      int2 ent[kRowChunk];
-      typename Src::Head head[kRowChunk];
-#pragma unroll
-      for (int k = 0; k < kRowChunk; ++k) {
-        const int e = base + k * LANES;
-        ent[k] = load_at(mesh.nbr, min(e, re - 1));
-        if (e >= re) ent[k].y = 0x7f800000;
-      }
-#pragma unroll
-      for (int k = 0; k < kRowChunk; ++k) {
-        const bool oc = __int_as_float(ent[k].y) <= prm.t_near && (!Src::kOcc || src.occupied(ent[k].x));
-        head[k] = src.head(oc ? ent[k].x : 0);
-        if (!oc) head[k].c = 0;
-      }
-      bool stop = false;
-#pragma unroll
-      for (int k = 0; k < kRowChunk; ++k) {
-        const float d = __int_as_float(ent[k].y);
-        if (d > prm.t_near) { stop = true; break; }
-        src.each(ent[k].x, head[k], [&](int j) {
-          double sj, cj;
-          sincos((double)src.theta(j), &sj, &cj);
-          Sx64 += cj;
-          Sy64 += sj;
-        });
-      }
-      if (stop) break;
+    if constexpr (NS == 1) {
+      strand(lane & (LANES - 1), Sx64, Sy64);
+    } else {
+      double sx[2] = {0.0, 0.0}, sy[2] = {0.0, 0.0};
+      strand(lane, sx[0], sy[0]);
+      strand(lane + P, sx[1], sy[1]);
+      Sx64 = sx[0] + sx[1];
+      Sy64 = sy[0] + sy[1];
     }
     {
-      Sx64 = group_sum<LANES>(Sx64);
-      Sy64 = group_sum<LANES>(Sy64);
+      Sx64 = group_sum<SUMW>(Sx64);
+      Sy64 = group_sum<SUMW>(Sy64);
       const double mean = atan2(Sy64, Sx64);
       double delta = mean - (double)th;
       if (delta > kPi) delta -= 2.0 * kPi;
