@@ -77,8 +77,6 @@ Engine::Engine(tissue_mesh* m, int R_, const int* n_, const tissue_params* p_) {
     HIP_OK(hipEventCreate(&ev0));
     HIP_OK(hipEventCreate(&ev1));
     d_row0 = dalloc<int>(2);
-    HIP_OK(hipHostMalloc((void**)&h_row0, 2 * sizeof(int), hipHostMallocDefault));
-    h_row0[0] = h_row0[1] = 0;
     if (nmax <= resident_cap) HIP_OK(resident_prepare(md.nv, nmax));
     d_reps = dalloc<ReplicaDesc>(R);
     upload(d_reps, reps.data(), reps.size());
@@ -102,9 +100,10 @@ Engine::Engine(tissue_mesh* m, int R_, const int* n_, const tissue_params* p_) {
     HIP_OK(launch_flags_begin(R, d_halt, d_rows, d_first_bad, stream));
     HIP_OK(hipStreamSynchronize(stream));
     back_half = std::min<size_t>(((size_t)ntot * 7 + 63) & ~(size_t)63, kBackHalfWords);
-    HIP_OK(hipHostMalloc((void**)&back, 2 * back_half * sizeof(float), hipHostMallocMapped | hipHostMallocCoherent));
+    HIP_OK(hipHostMalloc((void**)&back, (2 * back_half + 2) * sizeof(float), hipHostMallocMapped | hipHostMallocCoherent));
     HIP_OK(hipHostGetDevicePointer((void**)&back_dev, back, 0));
-    for (hipEvent_t& ev : back_ev) HIP_OK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    h_row0 = reinterpret_cast<int*>(back + 2 * back_half);
+    h_row0[0] = h_row0[1] = 0;
     hist_ref.resize(R);
     hist_polar.resize(R);
     flags_acc.assign(R, 0u);
@@ -148,7 +147,6 @@ void Engine::release() {
     if (ev) (void)hipEventDestroy(ev);
     ev = nullptr;
   }
-  if (h_row0) (void)hipHostFree(h_row0);
   h_row0 = nullptr;
   adjoint_release();
   if (ev0) (void)hipEventDestroy(ev0);
@@ -214,6 +212,14 @@ void Engine::init_random(const uint64_t* seeds) {
 template <class Pack, class Take>
 void Engine::read_back(int words_each, Pack&& pack, Take&& take) {
   const int per = (int)std::min<size_t>((size_t)ntot, back_half / words_each);
+  if (per == ntot) {
+    pack(0, ntot, back_dev);
+    HIP_OK(hipStreamSynchronize(stream));
+    take(0, ntot, back);
+    return;
+  }
+  for (hipEvent_t& ev : back_ev)
+    if (!ev) HIP_OK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
   for (int first = 0, half = 0; first < ntot + per; first += per, half ^= 1) {
     if (first < ntot) {
       pack(first, std::min(per, ntot - first), back_dev + half * back_half);

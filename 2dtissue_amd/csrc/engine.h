@@ -87,7 +87,8 @@ struct Engine {
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   // control words of the current run, read by its kernels: [0] first noise row, [1] steps done
   // since the output stream's origin (0 when not recording); uploaded from pinned host memory
-  // only when they differ from what the device holds (h_row0 mirrors it once row0_known)
+  // only when they differ from what the device holds (h_row0, behind the transfer buffer, mirrors it
+  // once row0_known)
   int* d_row0 = nullptr;
   int* h_row0 = nullptr;
   bool row0_known = false;
