@@ -350,6 +350,10 @@ struct WaveWalk {
   int pp[64 + 4];               // before each entry of the round: pairs, and << 16 particles counted
   unsigned vh[kWavePairs];      // visit_mix of the pair's particle (visit check only)
 };
+// what particle_step calls with the new vertex id, as soon as that is known
+struct NoPlaced {
+  __device__ void operator()(int) const {}
+};
 constexpr int kOwnerShift = 26;  // vertex ids below 2^26 (checked by the launcher)
 
 // One particle's update (U1-U6 of the reference step) by a group of P lanes. The sums over the
@@ -370,10 +374,10 @@ constexpr int kOwnerShift = 26;  // vertex ids below 2^26 (checked by the launch
 // null). WAVE selects the seam-wrap loop of crowded systems (seam_wrap_group). Always inlined: as an
 // out-of-line call (which the inliner picks once two kernels share an instantiation) its result
 // and live state go through scratch memory.
-template <int LANES, int P, bool WAVE = false, bool VISITS = false, class Src>
+template <int LANES, int P, bool WAVE = false, bool VISITS = false, class Src, class Placed = NoPlaced>
 __device__ __forceinline__ StepOut particle_step(const MeshDev& mesh, const StepParams& prm, const Src& src, int i, float4 me,
                                         float th, int v, float eta, int lane, bool active = true,
-                                        WaveWalk* ww = nullptr) {
+                                        WaveWalk* ww = nullptr, const Placed& placed = {}) {
   // a lane's sums: those of strand lane % LANES of the layout (its copies on the lanes above LANES equal it);
   // with P = LANES / 2 those of strands lane and lane + P. The force is summed in FP64 (its FP32 rounding
   // drives the FP32 path).
@@ -834,6 +838,7 @@ __device__ __forceinline__ StepOut particle_step(const MeshDev& mesh, const Step
   o.vh = vh;
   // UV -> 3D remap of the stored FP32 position (CellHelper.cpp:71-85)
   o.L = locate<P>(mesh, (double)o.xo, (double)o.yo, lane);
+  placed(o.L.vid);
   sincosf(o.to, &o.so, &o.co);
   // order parameter (LinearAlgebra.cpp:90-105, z = 0): sign of the cross product's z component
   const double cz = (double)o.xo * (double)vy - (double)o.yo * (double)vx;

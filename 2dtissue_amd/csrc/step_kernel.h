@@ -21,9 +21,9 @@ using namespace tdev;
 
 namespace {
 
+// particle i into vertex v's bucket as its arrival number old (the value its add to b.count[v] returned)
 template <bool OCC>
-__device__ __forceinline__ void bucket_insert(const BucketsOut& b, int v, int i) {
-  const int old = atomicAdd(&b.count[v], 1);
+__device__ __forceinline__ void bucket_place(const BucketsOut& b, int v, int i, int old) {
   if (OCC && old == 0) atomicOr(&b.occ[v >> 5], 1u << (v & 31));
   if (old < kSlots) {
     b.slot[(size_t)v * kSlots + old] = i;
@@ -32,6 +32,11 @@ __device__ __forceinline__ void bucket_insert(const BucketsOut& b, int v, int i)
     b.ovf[o] = make_int2(v, i);
   }
   if (b.multi) b.multi[i] = old == 1 ? v : -1;  // the second arrival has the bucket sorted
+}
+
+template <bool OCC>
+__device__ __forceinline__ void bucket_insert(const BucketsOut& b, int v, int i) {
+  bucket_place<OCC>(b, v, i, atomicAdd(&b.count[v], 1));
 }
 
 __device__ __forceinline__ BucketsOut replica_out(const BucketSet& s, int r, int nv, int off) {
@@ -159,7 +164,14 @@ __global__ void __launch_bounds__(kStepMaxBlock) k_step_tiled(MeshDev mesh, cons
       }
     } else {
       const GlobalSource<OCC, WAVE> src{replica_in(bin, r, nv, rep.off), io.xycs_in, io.th_in, s_occ};
-      const StepOut o = particle_step<LANES, P, WAVE, VISITS>(mesh, rep.prm, src, g, me, th, v, eta, lane, active, ww);
+      // the arrival counter is asked as soon as the new vertex is known: the answer comes while the heading's
+      // sine and the outputs are written (asked with the rest of the insertion it was the wave's last wait:
+      // 2,000 particles 10.75 -> 10.64 us per step, 525,000 in 256 replicas 151.2 -> 150.0 us)
+      int arrival = 0;
+      const auto arrive = [&](int vnew) __attribute__((always_inline)) {
+        if (active && lane == 0) arrival = atomicAdd(&bo.count[vnew], 1);
+      };
+      const StepOut o = particle_step<LANES, P, WAVE, VISITS>(mesh, rep.prm, src, g, me, th, v, eta, lane, active, ww, arrive);
       if (active && lane == 0) {
         io.xycs_out[g] = make_float4(o.xo, o.yo, o.co, o.so);
         io.th_out[g] = o.to;
@@ -171,7 +183,7 @@ __global__ void __launch_bounds__(kStepMaxBlock) k_step_tiled(MeshDev mesh, cons
         io.r3z[g] = (float)o.L.Z;
         io.face[g] = o.L.face;
         io.nbr[g] = o.nb;  // count_particle_neighbors (2DTissue.cpp:254-268)
-        bucket_insert<OCC>(bo, o.L.vid, g);
+        bucket_place<OCC>(bo, o.L.vid, g, arrival);
         if (o.fl) {
           atomicOr(&io.halt_out[r], o.fl);
           atomicMin(&io.first_bad[r], io.step);
