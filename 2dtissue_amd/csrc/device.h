@@ -335,11 +335,13 @@ __device__ __forceinline__ int wave_scan(int v) {
 // work load a fixed address instead of branching around the load: a load under a branch is waited
 // for before the next is issued. Area per wave:
 constexpr int kWaveEntries = 256;  // entries compacted at a time (more: entry by entry of the lanes)
-constexpr int kWavePairs = 192;    // pairs of a round (a round takes as many entries as fit)
+constexpr int kWavePairs = 184;    // pairs of a round (a round takes as many entries as fit)
 // whether P physical lanes per particle walk this way for sums laid out over LANES lanes (crowded:
 // sorted buckets; with as many lanes as the layout the lane-by-lane walk is 2-3 % faster there, 65,000
 // and 100,000 particles)
 constexpr bool coop_walk(int lanes, int p, bool crowded) { return p != lanes || (lanes <= 4 && !crowded); }
+// whether a wave has an area: for the walk, and for the FP64 headings of wave_heading_sum
+constexpr bool wave_area(int lanes, int p, bool crowded) { return lanes <= 8 || coop_walk(lanes, p, crowded); }
 // table entries per lane taken together, by physical lanes
 constexpr int coop_chunk(int p) { return p >= 16 ? 2 : (p == 8 ? 4 : 8); }
 struct WaveWalk {
@@ -355,6 +357,82 @@ struct NoPlaced {
   __device__ void operator()(int) const {}
 };
 constexpr int kOwnerShift = 26;  // vertex ids below 2^26 (checked by the launcher)
+
+// The alignment sum of one particle over the FP64 cosines and sines of its neighbours' headings, by the
+// whole wave (all lanes present): rs .. re its row. A lane takes one entry and its bucket, then one
+// neighbour and its sine; then every lane adds the terms of strand lane % LANES in the strand's order.
+// The redo of a nearly cancelling sum is rare per particle but not per wave, and walked by the
+// particle's own lanes it was the step's longest chain (up to 18,000 cycles of 38,000 at 9,001 particles,
+// 54,000 of 107,000 at 100,000): four entries a lane at a time, each neighbour's heading and sine behind
+// the one before. 9,001 particles 20.7 -> 18.8 us per step, 100,000 84.1 -> 72.9, 525,000 in 256 replicas
+// 150.4 -> 148.5.
+template <int LANES, class Src>
+__device__ __forceinline__ void wave_heading_sum(const MeshDev& mesh, float t_near, const Src& src, WaveWalk* ww,
+                                                 int rs, int re, double& sx, double& sy) {
+  static_assert(kWavePairs >= 64 && (kWaveEntries + 64) * 2 >= 64 * kSlots, "terms of a round, ids of 64 buckets");
+  const int wl = (int)__lane_id();
+  int* ids = reinterpret_cast<int*>(ww->ent);
+  for (int base = rs; base < re; base += 64) {  // a multiple of LANES: entry base + l is of strand l % LANES
+    int2 ent = load_at(mesh.nbr, min(base + wl, re - 1));
+    if (base + wl >= re) ent.y = 0x7f800000;
+    const bool near = __int_as_float(ent.y) <= t_near && (!Src::kOcc || src.occupied(ent.x));
+    const int count = src.count(near ? ent.x : 0);
+    int a[kSlots];
+    src.slots(near ? ent.x : 0, a);
+    const int c = near ? count : 0;
+    if (!src.b.sorted && __builtin_amdgcn_ballot_w64(c > kSlots) != 0) {  // raw and crowded: rare
+      for (int t = wl & (LANES - 1); t < 64 && base + t < re; t += LANES) {
+        const int2 e = load_at(mesh.nbr, base + t);
+        if (__int_as_float(e.y) > t_near) break;
+        src.each(e.x, src.head(e.x), [&](int j) {
+          double sj, cj;
+          sincos((double)src.theta(j), &sj, &cj);
+          sx += cj;
+          sy += sj;
+        });
+      }
+    } else {
+      if (!src.b.sorted && __builtin_amdgcn_ballot_w64(c > 1) != 0) {  // ids ascending
+#pragma unroll
+        for (int q = 0; q < kSlots; ++q) a[q] = q < c ? a[q] : 0x7fffffff;
+        sort8(a);
+      }
+      const int upto = wave_scan(c), total = __builtin_amdgcn_readlane(upto, 63);
+      ww->pp[wl] = upto - c;
+      if (wl == 63) ww->pp[64] = upto;
+      reinterpret_cast<int4*>(ids)[2 * wl] = make_int4(a[0], a[1], a[2], a[3]);
+      reinterpret_cast<int4*>(ids)[2 * wl + 1] = make_int4(a[4], a[5], a[6], a[7]);
+      constexpr uint64_t kEvery = LANES == 1 ? ~0ull : (LANES == 2 ? 0x5555555555555555ull :
+                                  (LANES == 4 ? 0x1111111111111111ull : 0x0101010101010101ull));
+      static_assert(LANES == 1 || LANES == 2 || LANES == 4 || LANES == 8, "strand mask");
+      const uint64_t strand = __builtin_amdgcn_ballot_w64(c > 0) & (kEvery << (wl & (LANES - 1)));
+      wave_sync();
+      for (int k0 = 0; k0 < total; k0 += 64) {
+        const int k = min(k0 + wl, total - 1);
+        int t = 0;  // the entry that holds neighbour k
+#pragma unroll
+        for (int s = 32; s >= 1; s >>= 1) t += ww->pp[t + s] <= k ? s : 0;
+        const int first = ww->pp[t], held = ww->pp[t + 1] - first;
+        int j = ids[t * kSlots + (held > kSlots ? 0 : k - first)];
+        if (held > kSlots) j = src.b.big[j + k - first];
+        double sj, cj;
+        sincos((double)src.theta(j), &sj, &cj);
+        ww->F[wl] = make_double2(cj, sj);
+        wave_sync();
+        for (uint64_t m = strand; m != 0; m &= m - 1) {
+          const int e = __builtin_ctzll(m), hi = min(ww->pp[e + 1], k0 + 64);
+          for (int p = max(ww->pp[e], k0); p < hi; ++p) {
+            const double2 f = ww->F[p - k0];
+            sx += f.x;
+            sy += f.y;
+          }
+        }
+        wave_sync();
+      }
+    }
+    if (__int_as_float(__builtin_amdgcn_readlane(ent.y, 63)) > t_near) break;  // rows ascend in distance
+  }
+}
 
 // One particle's update (U1-U6 of the reference step) by a group of P lanes. The sums over the
 // neighbours are laid out over LANES lanes: lane l of LANES adds the entries l, l + LANES, .. of the
@@ -732,6 +810,20 @@ __device__ __forceinline__ StepOut particle_step(const MeshDev& mesh, const Step
     vx = (float)vx64;
     vy = (float)vy64;
   }
+  double Sx64 = 0.0, Sy64 = 0.0;
+  constexpr bool kWaveHeadings = Src::kCoop && wave_area(LANES, P, WAVE) && LANES <= 8;
+  if constexpr (kWaveHeadings) {
+    for (uint64_t m = __builtin_amdgcn_ballot_w64(weak && active && lane == 0); m != 0; m &= m - 1) {
+      const int first = __builtin_ctzll(m);
+      double sx = 0.0, sy = 0.0;
+      wave_heading_sum<LANES>(mesh, prm.t_near, src, ww, __builtin_amdgcn_readlane(rs, first),
+                              __builtin_amdgcn_readlane(re, first), sx, sy);
+      if (((int)__lane_id() & ~(P - 1)) == first) {
+        Sx64 = sx;
+        Sy64 = sy;
+      }
+    }
+  }
   if (weak) {
     // the alignment sum again, over the neighbours' headings in FP64
     auto strand = [&](int first, double& sx, double& sy) __attribute__((always_inline)) {
@@ -765,8 +857,8 @@ __device__ __forceinline__ StepOut particle_step(const MeshDev& mesh, const Step
         if (stop) break;
       }
     };
-    double Sx64 = 0.0, Sy64 = 0.0;
-    if constexpr (NS == 1) {
+    if constexpr (kWaveHeadings) {
+    } else if constexpr (NS == 1) {
       strand(lane & (LANES - 1), Sx64, Sy64);
     } else {
       double sx[2] = {0.0, 0.0}, sy[2] = {0.0, 0.0};

@@ -145,10 +145,11 @@ constexpr int kStepMaxBlock = 512;
 constexpr int kOccWordsPerParticle = 8;
 // LDS of one workgroup of the tiled step kernel: the waves' walk areas and the staged mask
 inline size_t step_lds_bytes(int nv, int block, int lanes, int phys, bool crowded, bool occ) {
-  return (tdev::coop_walk(lanes, phys, crowded) ? (size_t)(block / 64) * sizeof(tdev::WaveWalk) : 0) +
+  return (tdev::wave_area(lanes, phys, crowded) ? (size_t)(block / 64) * sizeof(tdev::WaveWalk) : 0) +
          (occ ? sizeof(unsigned) * (size_t)tdev::occ_words(nv) : 0);
 }
 constexpr size_t kStepMaxLds = 64 * 1024;  // what a launch may ask for without raising the limit
+static_assert(kStepMaxBlock / 64 * sizeof(tdev::WaveWalk) <= kStepMaxLds, "the areas of the largest workgroup");
 inline bool stage_occupancy(int nv, int block, int lanes, int phys) {
   return phys <= lanes && tdev::occ_words(nv) <= kOccWordsPerParticle * (block / phys) &&
          step_lds_bytes(nv, block, lanes, phys, false, true) <= kStepMaxLds;

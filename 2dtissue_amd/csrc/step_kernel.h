@@ -112,9 +112,9 @@ __global__ void __launch_bounds__(kStepMaxBlock) k_step_tiled(MeshDev mesh, cons
   // the waves' walk areas (whole-wave walk), then with OCC occ_words(nv) words, the input buckets'
   // occupancy mask
   extern __shared__ __align__(16) unsigned char smem[];
-  constexpr bool kCoop = coop_walk(LANES, P, WAVE);
-  WaveWalk* ww = kCoop ? reinterpret_cast<WaveWalk*>(smem) + (threadIdx.x >> 6) : nullptr;
-  unsigned* s_occ = reinterpret_cast<unsigned*>(smem + (kCoop ? (blockDim.x >> 6) * sizeof(WaveWalk) : 0));
+  constexpr bool kArea = wave_area(LANES, P, WAVE);
+  WaveWalk* ww = kArea ? reinterpret_cast<WaveWalk*>(smem) + (threadIdx.x >> 6) : nullptr;
+  unsigned* s_occ = reinterpret_cast<unsigned*>(smem + (kArea ? (blockDim.x >> 6) * sizeof(WaveWalk) : 0));
   const TileDesc tile = tiles[blockIdx.x];
   if (tile.r < 0) return;  // idle padding workgroup (whole block)
   const int r = tile.r;
@@ -153,7 +153,7 @@ __global__ void __launch_bounds__(kStepMaxBlock) k_step_tiled(MeshDev mesh, cons
 
   int sgn = 0;
   long long pcs = 0, psn = 0;
-  if (active || (kCoop && !halt)) {  // a walking wave needs all of its lanes
+  if (active || (kArea && !halt)) {  // such a wave needs all of its lanes
     if (halt) {
       if (lane == 0) {
         io.xycs_out[g] = me;

@@ -87,6 +87,47 @@ def test_walk_of_a_whole_wave(T, monkeypatch, lanes, sizes):
     b.close()
 
 
+@pytest.mark.parametrize("lanes", [1, 2, 4, 8])
+@pytest.mark.parametrize("raw", [True, False])
+@pytest.mark.parametrize("n,patch", [(1, 1.0), (65, 0.05), (300, 0.02), (1500, 1.0)])
+def test_headings_by_the_whole_wave(T, monkeypatch, lanes, raw, n, patch):
+    """Alignment sums redone in FP64 by the whole wave: random headings with dt / tau = 1, where a sum
+    below 0.6 of its neighbours is redone, for one particle, for a few crowded buckets (300 particles
+    on the vertices of a small patch: more than 8, and more than 64, in one) and for rows over several
+    rounds of entries; raw and sorted buckets. Nothing moves (v0 = mu = 0), so each heading is the mean
+    of its neighbours' in FP64: up to the FP32 rounding of the result where the sum is redone (2.4e-7 at
+    2 pi), up to 1e-6 where it is left in FP32 (three roundings of that size and the sum's 1e-7)."""
+    m, _ = P.mesh_and_tables(22, 0.1)
+    phys = dict(P.PHYS, v0=0.0, mu=0.0, tau=P.PHYS["dt"])
+    rng = np.random.default_rng(n)
+    x, y = (0.5 + patch * (rng.random(n) - 0.5) for _ in range(2))
+    th = rng.random(n) * 2 * np.pi
+    x, y, th = (q.astype(np.float32) for q in (x, y, th))
+    monkeypatch.setenv("TISSUE_SORTED_BUCKETS", "0" if raw else "1")
+    b = T.Batch(m, [n], [T.params(**phys, sigma=0.1)])
+    monkeypatch.delenv("TISSUE_SORTED_BUCKETS")
+    b.set_mode(T.MODE_STEP_KERNEL)
+    b.set_launch(lanes, 128)
+    b.set_state(x, y, th)
+    one = T.Sim(m, T.params(**phys, sigma=0.1), n)
+    one.set_state(x, y, th)
+    th64 = th.astype(np.float64)
+    want = np.empty(n)
+    tol = np.full(n, 1e-6)
+    for i, js in enumerate(one.neighbor_lists()):
+        c, s = np.cos(th64[js]).sum(), np.sin(th64[js]).sum()
+        if np.hypot(c, s) < 0.59 * len(js):
+            tol[i] = 2.5e-7
+        want[i] = th64[i] + (np.arctan2(s, c) - th64[i] + np.pi) % (2 * np.pi) - np.pi
+    assert (tol < 1e-6).sum() > n // 2 or n == 1
+    b.stage_noise(np.zeros((1, n), np.float32))
+    assert b.run(1, 0) == T.OK
+    diff = (b.get_state().theta.astype(np.float64) - want + np.pi) % (2 * np.pi) - np.pi
+    assert (np.abs(diff) <= tol).all(), np.abs(diff).max()
+    one.close()
+    b.close()
+
+
 @pytest.mark.parametrize("lanes", [2, 8])
 def test_full_workgroup_of_the_persistent_kernel(T, lanes):
     """Block 512 runs as 1,024 threads where the reduction words fit beside the replica, as 512 up to the
