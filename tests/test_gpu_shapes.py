@@ -87,6 +87,33 @@ def test_walk_of_a_whole_wave(T, monkeypatch, lanes, sizes):
     b.close()
 
 
+@pytest.mark.parametrize("lanes", [16, 32, 64])
+@pytest.mark.parametrize("n,patch", [(40, 0.04), (300, 0.1), (300, 0.01)])
+def test_piled_particles(T, monkeypatch, lanes, n, patch):
+    """Buckets of three to eight particles, read four states at a time, and fuller ones (a patch of a few
+    vertices), in the shapes that walk lane by lane: raw and sorted buckets give the same bits and each
+    particle's visited set has the size a plain kernel lists."""
+    m, _ = P.mesh_and_tables(22, 0.1)
+    rng = np.random.default_rng(n)
+    x, y, th = ((0.5 + patch * (rng.random(n) - 0.5)).astype(np.float32) for _ in range(3))
+    one = T.Sim(m, T.params(**P.PHYS, sigma=0.1), n)
+    one.set_state(x, y, th)
+    assert max(np.bincount(one.get_state().vid)) > 2
+    sizes = [len(q) for q in one.neighbor_lists()]
+    one.close()
+    got = []
+    for raw in (True, False):
+        b = _batch(T, m, [n], raw, monkeypatch, lanes, x, y, th)
+        b.stage_noise(np.zeros((1, n), np.float32))
+        assert b.run(1, 0) == T.OK
+        assert np.array_equal(b.visits()[0], sizes)
+        got.append((b.get_state(), b.visits()[1]))
+        b.close()
+    for k in ("x", "y", "theta", "vid"):
+        assert np.array_equal(getattr(got[0][0], k), getattr(got[1][0], k)), k
+    assert np.array_equal(got[0][1], got[1][1])
+
+
 @pytest.mark.parametrize("lanes", [1, 2, 4, 8])
 @pytest.mark.parametrize("raw", [True, False])
 @pytest.mark.parametrize("n,patch", [(1, 1.0), (65, 0.05), (300, 0.02), (1500, 1.0)])
