@@ -156,11 +156,12 @@ inline bool stage_occupancy(int nv, int block, int lanes, int phys) {
 }
 // Physical lanes per particle for sums laid out over `lanes` lanes (the results are the same for any).
 // As many as the layout where the chip is full; more where it is not and a step's longest chain counts
-// (MI355X, us per step): 4 -> 8 at 9,001 particles 25.2 / 22.9, 13,000 in 37 replicas 19.8 / 18.1, 20,000
-// 39.7 / 37.8, 30,000 in 30 replicas 26.5 / 25.1, 40,000 40.5 / 43.3; 8 -> 16 at 5,000 particles
-// 19.2 / 16.7, 8,000 21.2 / 18.1; 2 -> 4 for replicas sparse on a mesh too large for the occupancy mask,
-// 64 x 2,000 (gradients, ms) 30.6 / 29.2, but with the mask 80,000 particles 43.3 / 44.4 and 530,000
-// 163 / 181. Fewer lanes than the layout were slower throughout (530,000 particles, 2 -> 1: 163 / 192).
+// (MI355X, us per step): 4 -> 8 at 9,001 particles 23.0 / 18.8, 20,000 32.3 / 26.2, 30,000 in 30 replicas
+// 21.4 / 21.0, but 40,000 33.5 / 37.0 and 100,000 72.6 / 78.2; 8 -> 16 at 5,000 particles 16.7 / 14.1, 8,000
+// 17.9 / 14.6; 2 -> 4 for replicas sparse on a mesh too large for the occupancy mask, 64 x 2,000
+// 57.4 / 55.1, but with the mask 80,000 particles 36.6 / 36.6, 250,000 85.5 / 85.5 and 525,000 159 / 164.
+// Fewer lanes than the layout were slower throughout (525,000 particles, 2 -> 1: 163 / 192, before the
+// figures above).
 inline int phys_lanes(int lanes, int ntot, int nv, int block) {
   if (lanes == 8 && ntot <= 16384) return 16;
   if (lanes == 4 && ntot <= 32768) return 8;
@@ -176,11 +177,11 @@ inline int resident_default_lanes(int nmax) { return nmax <= 256 ? 8 : (nmax <= 
 // R replicas of ntot particles in all. Measured on MI355X: a single system of a few thousand
 // particles fills few CUs, so more lanes per particle shorten its critical path, and one-wave
 // workgroups let every wave start its walk without waiting for another at the staging barrier
-// (2,000 particles: 32 lanes in 64 threads 18.97 us, 16 in 128 19.30 us, 64 in 64 19.19 us, 8 in
-// 64 20.7 us); beyond, workgroups of 128 leave a shorter last round than 256 (530,000 particles in 256
-// replicas 34.1 -> 33.2 ms per 200 steps, 100,000 8.57 -> 8.41 ms per 100; 64 threads the same or slower
-// again); a single 100,000-particle system is fastest with 4 (2 lanes 10 % slower), a large
-// batch with 2 (autotuned).
+// (2,000 particles: 32 lanes in 64 threads 10.08 us, 16 in 64 10.48 us, 16 in 128 10.54 us, 64 in 64
+// 10.19 us, 8 in 64 10.83 us); beyond, workgroups of 128 leave a shorter last round than 256 (525,000
+// particles in 256 replicas 34.1 -> 33.2 ms per 200 steps; 100,000 particles 68.5 -> 67.3 us per step, 64
+// threads 66.6, but slower in the batch); a single 100,000-particle system is fastest with 4 (2 lanes
+// 82.6 us), a large batch with 2 (autotuned).
 inline void tiled_default_shape(int R, int ntot, int* lanes, int* block) {
   const int big_lanes = R == 1 ? 4 : 2;
   *lanes = ntot <= 4096 ? 32 : (ntot <= 8192 ? 8 : (ntot <= 65536 ? 4 : big_lanes));

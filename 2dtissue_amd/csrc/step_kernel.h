@@ -1,9 +1,14 @@
 // gfx950 kernel of the tiled per-step update (one launch per step, all replicas at once).
 //
 // k_step_tiled<LANES, P>: each workgroup is a tile of one replica (TileDesc); P lanes of a wave64
-// cooperate on one particle, whose sums are laid out over LANES lanes (particle_step). They stride over the particle's row of the truncated geodesic table
-// (vertices within 2.4 sigma of its vertex, ascending in distance), visit the particles bucketed on
-// those vertices, and reduce force, alignment sum and neighbour count with butterfly shuffles.
+// cooperate on one particle, whose sums are laid out over LANES lanes (particle_step). They stride over
+// the particle's row of the truncated geodesic table (vertices within 2.4 sigma of its vertex, ascending
+// in distance), visit the particles bucketed on those vertices, and reduce force, alignment sum and
+// neighbour count with butterfly shuffles.
+//
+// The kernel is bound by chains of dependent loads (table row, bucket, particles; cell, candidates, face)
+// and, where the chip is full, by instruction issue; never by bandwidth (2.9 TB/s at most). 2,000 particles
+// 18.7 -> 10.1 us per step, 100,000 274 -> 67, 525,000 in 256 replicas 211 -> 150.
 // Every lane then runs the per-particle epilogue (speed, Euler, heading, seam wrap) and the lanes
 // split the point-location candidates of the face bucket. Lane 0 writes the SoA outputs, inserts
 // the particle into next step's vertex buckets and contributes to the tile's order-parameter

@@ -207,7 +207,8 @@ int32_t tissue_batch_get_visits(tissue_batch* b, int32_t* na, uint32_t* hash);
  * are step t's velocity and pre-step position; u is a smooth field on the UV square, a sum of
  * modes u_c(x, y) += amp sin(kx x + ky y + phase) with c = component (0: x, 1: y).
  * The reverse pass runs through the forward's frozen decisions (neighbour sets, seam-wrap maps,
- * vertex ids), recomputing each segment of ckpt_every steps from a checkpoint. */
+ * vertex ids). They are kept for all steps where they fit in 16 GB (and no recording or visit check is on);
+ * else each segment of ckpt_every steps is recomputed from a checkpoint. The gradients are the same. */
 #define TISSUE_MAX_MODES 16
 typedef struct {
   double target_order;
