@@ -139,12 +139,18 @@ bool Engine::whole_tape(int T) {
     for (Tape& t : a.tp) free_tape(t);  // either form's memory, not both
     a.K = a.ntape = 0;
     Tape& t = a.whole;
-    t.xycs = dalloc<float4>((size_t)(T + 1) * N);
-    t.th = dalloc<float>((size_t)(T + 1) * N);
-    t.vid = dalloc<int>((size_t)(T + 1) * N);
-    t.fs = dalloc<float4>((size_t)T * N);
-    t.q = dalloc<int>((size_t)T * N);
-    alloc_set_slab(a.sets, n_sets);
+    try {
+      t.xycs = dalloc<float4>((size_t)(T + 1) * N);
+      t.th = dalloc<float>((size_t)(T + 1) * N);
+      t.vid = dalloc<int>((size_t)(T + 1) * N);
+      t.fs = dalloc<float4>((size_t)T * N);
+      t.q = dalloc<int>((size_t)T * N);
+      alloc_set_slab(a.sets, n_sets);
+    } catch (const ApiError&) {  // less memory free than that: checkpoints need less
+      (void)hipGetLastError();
+      free_whole_tape();
+      return false;
+    }
     a.whole_T = T;
     a.keep_sets = keep;
   }
