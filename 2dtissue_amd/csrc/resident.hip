@@ -128,8 +128,9 @@ __device__ __forceinline__ double lane_double(double v, int l) {
 // What bounds a step: one workgroup's chain of barriers and dependent loads, the CU's other resources idle.
 // Hence nothing serial stands between two barriers: the new state of a group's last particle stays in
 // registers until the old one has been read (only earlier passes go through global memory), begin is
-// cleared where the state is copied, and the order parameters are added up by the last wave with all its
-// reads in flight (100 particles, 50 steps 0.705 -> 0.677 ms; 256 x 200 particles, 100 steps 1.97 -> 1.87 ms).
+// cleared where the state is copied, and the order parameters are added up by the last wave, with all its
+// reads in flight, and finished by it beside the next step's update (100 particles, 50 steps 0.705 -> 0.660 ms;
+// 256 x 200 particles, 100 steps 1.97 -> 1.83 ms).
 template <int LANES, int P>
 __global__ void __launch_bounds__(kFullBlock) k_resident(MeshDev mesh, const ReplicaDesc* __restrict__ reps, int nmax, int steps,
                                                         ResidentIO io) {
@@ -164,13 +165,25 @@ __global__ void __launch_bounds__(kFullBlock) k_resident(MeshDev mesh, const Rep
   if (tid == 0) s_flags = io.flags_in[r];
   __syncthreads();
 
-  const int wave = tid >> 6, nw = (nthr + 63) >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), nw = (nthr + 63) >> 6;
+  // the sums of the step before (in the last wave, one value a wave), and where its order parameters go
+  double sum_cs = 0.0, sum_sn = 0.0;
+  int sum_sg = 0;
+  double* last_phi = nullptr;
+  auto finish_phi = [&]() __attribute__((always_inline)) {
+    if (last_phi && wave == nw - 1 && (tid & 63) == 0) {
+      last_phi[0] = (1.0 / n) * fabs((double)sum_sg);
+      last_phi[1] = sqrt(sum_cs * sum_cs + sum_sn * sum_sn) / n;
+    }
+    last_phi = nullptr;
+  };
 
   const LdsSource src{begin, sorted, xycs, th};
   for (int s = 0; s < steps; ++s) {
     const int t = io.t_base + s;
     double* phi = io.phi + 2 * ((size_t)r * io.phi_stride + t);
     if (s_flags != 0u) {  // a failed step stops the replica (the reference stops at the first failure)
+      finish_phi();
       if (tid == 0) { phi[0] = 0.0; phi[1] = 0.0; }
       continue;
     }
@@ -180,6 +193,7 @@ __global__ void __launch_bounds__(kFullBlock) k_resident(MeshDev mesh, const Rep
     int sgn = 0;
     double cs = 0.0, sn = 0.0;
     unsigned fl = 0;
+    finish_phi();
     // the update is Jacobi, every particle must read the old state of its neighbours: the new state of a
     // group's last particle is held in registers, that of its earlier ones staged in global memory (this
     // workgroup's slice, L2-resident)
@@ -233,27 +247,24 @@ __global__ void __launch_bounds__(kFullBlock) k_resident(MeshDev mesh, const Rep
       vid[i] = nxt_vid[i];
     }
     for (int v = tid; v <= mesh.nv; v += nthr) begin[v] = 0u;
-    if (wave == nw - 1) {  // the cosines on lane 0, the sines on lane 1, the signs on lane 2
+    if (wave == nw - 1) {  // the waves' sums in order, the cosines on lane 0 and the sines on lane 1
       static_assert(kFullBlock <= 16 * 64, "waves of a workgroup");
-      const int q = in_step(tid) & 63, waves = __builtin_amdgcn_readfirstlane(in_step(nw));
-      const double* part = q == 0 ? red_cs : red_sn;
+      const int l = in_step(tid) & 63, waves = __builtin_amdgcn_readfirstlane(in_step(nw));
+      const double* part = l == 0 ? red_cs : red_sn;
+      const int g = l < waves ? red_sg[l] : 0;
       double v[16], sum = 0.0;
-      int g[16];
 #pragma unroll
-      for (int w = 0; w < 16; ++w) {
-        v[w] = part[w < waves ? w : 0];
-        g[w] = red_sg[w < waves ? w : 0];
-      }
+      for (int w = 0; w < 16; ++w) v[w] = part[w < waves ? w : 0];
 #pragma unroll
-      for (int w = 0; w < 16; ++w) sum += w < waves ? (q < 2 ? v[w] : (double)g[w]) : 0.0;
-      const double C = lane_double(sum, 0), S = lane_double(sum, 1), G = lane_double(sum, 2);
-      if (q == 0) {
-        phi[0] = (1.0 / n) * fabs(G);
-        phi[1] = sqrt(C * C + S * S) / n;
-      }
+      for (int w = 0; w < 16; ++w) sum += w < waves ? v[w] : 0.0;
+      sum_cs = lane_double(sum, 0);
+      sum_sn = lane_double(sum, 1);
+      sum_sg = __builtin_amdgcn_readfirstlane(group_sum<64>(g));
     }
+    last_phi = phi;
     __syncthreads();
   }
+  finish_phi();
 
   for (int i = tid; i < n; i += nthr) {
     io.xycs[off + i] = xycs[i];
