@@ -335,7 +335,8 @@ hipError_t launch_resident(int lanes, int block, const MeshDev& mesh, const Repl
     case 4: return launch_one<4, 4>(block, mesh, reps, R, nmax, steps, io, st);
     case 8:
       // four lanes, two strands each, where eight take more than one pass over the replica (256 replicas
-      // x 100 steps: 200 particles 2.20 -> 1.96 ms, 256 particles 3.03 -> 2.66 ms)
+      // x 100 steps: 200 particles 2.20 -> 1.96 ms, 256 particles 3.03 -> 2.66 ms); where eight fit in one
+      // pass four are slower (100 particles, 100 steps 1.21 -> 1.31 ms, 256 x 100 particles 1.51 -> 1.72 ms)
       if (nmax * 8 > block) return launch_one<8, 4>(block, mesh, reps, R, nmax, steps, io, st);
       return launch_one<8, 8>(block, mesh, reps, R, nmax, steps, io, st);
     default: return hipErrorInvalidValue;
