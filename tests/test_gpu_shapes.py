@@ -181,3 +181,35 @@ def test_full_workgroup_of_the_persistent_kernel(T, lanes):
         for other in got[1:]:
             for a, b in zip(got[0][:10], other[:10]):
                 assert np.array_equal(a, b), n
+
+
+@pytest.mark.parametrize("block", [64, 128, 512])
+@pytest.mark.parametrize("n", [1, 100, 300])
+def test_persistent_kernel_between_its_barriers(T, block, n):
+    """Vertex counts scanned in registers (4,907 vertices: 5 a thread at 1,024 threads) and in LDS (39 and 77
+    a thread), one pass over the replica and several (the last one's states held in registers), one wave and
+    sixteen: states, neighbour counts and order parameters are the step kernel's, states and order parameters
+    also where a step fails (the persistent kernel then writes no outputs of that run)."""
+    m, _ = P.mesh_and_tables(22, 0.1)
+    prm = T.params(**P.PHYS, sigma=0.1)
+    for bad in (None, 2):
+        noise = T.gen_noise(5, 0.1, 4, n)
+        if bad is not None:
+            noise[bad, n - 1] = np.nan
+        got = []
+        for mode, b in ((T.MODE_RESIDENT, block), (T.MODE_STEP_KERNEL, 128)):
+            s = T.Sim(m, prm, n)
+            s.set_mode(mode)
+            s.set_launch(8, b)
+            s.init_random(11)
+            code = s.step(4, noise)
+            st, o, phi = s.get_state(), s.get_outputs(), s.order()
+            got.append((code, [st.x, st.y, st.theta, st.vid] + ([o.nbr] if bad is None else []), phi))
+            s.close()
+        (ca, a, pa), (cb, c, pb) = got
+        assert ca == cb and (ca == T.OK) == (bad is None)
+        for u, v in zip(a, c):
+            assert np.array_equal(u, v, equal_nan=u.dtype.kind == "f"), (bad, n)
+        k = 4 if bad is None else bad
+        assert np.array_equal(pa[0][:k], pb[0][:k])
+        assert np.allclose(pa[1][:k], pb[1][:k], rtol=0, atol=1e-12)
