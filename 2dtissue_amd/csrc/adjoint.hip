@@ -292,7 +292,7 @@ __global__ void __launch_bounds__(256) k_adj_reverse(MeshDev mesh, const Replica
 #pragma unroll
         for (int k = 0; k < kChunk; ++k) {
           const int e = base + k * G;
-          ent[k] = load_at(mesh.nbr, min(e, re - 1));
+          ent[k] = table_entry(mesh.nbr, min(e, re - 1));
           if (e >= re) ent[k].y = 0x7f800000;
         }
       };

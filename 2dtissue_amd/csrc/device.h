@@ -59,8 +59,9 @@ struct BucketsOut { int* count; int* slot; int* ovf_n; int2* ovf; int* multi; un
 __host__ __device__ constexpr int occ_words(int nv) { return (nv + 31) >> 5; }
 
 // base[i] for a uniform base and 0 <= i * sizeof(T) < 2^32: the address is the scalar base plus a
-// 32-bit lane offset, two or three instructions fewer than a 64-bit one (the step's arrays are below
-// 4 GiB each: 2^27 particles, 2^26 vertices, 2^28 table entries)
+// 32-bit lane offset, two or three instructions fewer than a 64-bit one (arrays by particle or by vertex
+// of one replica, below 4 GiB each: 2^27 particles, 2^26 vertices; the geodesic table may be larger and
+// goes through table_entry)
 template <class T>
 __device__ __forceinline__ T load_at(const T* base, int i) {
   return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + (uint32_t)i * (uint32_t)sizeof(T));
@@ -395,7 +396,7 @@ __device__ __forceinline__ void wave_heading_sum(const MeshDev& mesh, float t_ne
   const int wl = (int)__lane_id();
   int* ids = reinterpret_cast<int*>(ww->ent);
   for (int base = rs; base < re; base += 64) {  // a multiple of LANES: entry base + l is of strand l % LANES
-    int2 ent = load_at(mesh.nbr, min(base + wl, re - 1));
+    int2 ent = table_entry(mesh.nbr, min(base + wl, re - 1));
     if (base + wl >= re) ent.y = 0x7f800000;
     const bool near = __int_as_float(ent.y) <= t_near && (!Src::kOcc || src.occupied(ent.x));
     const int count = src.count(near ? ent.x : 0);
@@ -404,7 +405,7 @@ __device__ __forceinline__ void wave_heading_sum(const MeshDev& mesh, float t_ne
     const int c = near ? count : 0;
     if (!src.b.sorted && __builtin_amdgcn_ballot_w64(c > kSlots) != 0) {  // raw and crowded: rare
       for (int t = wl & (LANES - 1); t < 64 && base + t < re; t += LANES) {
-        const int2 e = load_at(mesh.nbr, base + t);
+        const int2 e = table_entry(mesh.nbr, base + t);
         if (__int_as_float(e.y) > t_near) break;
         src.each(e.x, src.head(e.x), [&](int j) {
           double sj, cj;
@@ -522,7 +523,7 @@ __device__ __forceinline__ StepOut particle_step(const MeshDev& mesh, const Step
 #pragma unroll
       for (int k = 0; k < kChunk; ++k) {
         const int e = base + k * P;
-        ent[k] = load_at(mesh.nbr, min(e, re - 1));
+        ent[k] = table_entry(mesh.nbr, min(e, re - 1));
         if (e >= re) ent[k].y = 0x7f800000;  // +inf ends the walk
       }
       bool oc[kChunk];
@@ -564,7 +565,7 @@ __device__ __forceinline__ StepOut particle_step(const MeshDev& mesh, const Step
 #pragma unroll
       for (int k = 0; k < kChunk; ++k) {
         const int e = wbase + k * P;
-        ent[k] = load_at(mesh.nbr, max(min(e, re - 1), 0));
+        ent[k] = table_entry(mesh.nbr, max(min(e, re - 1), 0));
         if (!more || e >= re) ent[k].y = 0x7f800000;
       }
       if constexpr (Src::kOcc) {
@@ -750,7 +751,7 @@ __device__ __forceinline__ StepOut particle_step(const MeshDev& mesh, const Step
 #pragma unroll
         for (int k = 0; k < kScanChunk; ++k) {
           const int e = wbase + (m0 + k) * LANES;
-          ent[k] = load_at(mesh.nbr, min(e, re - 1));
+          ent[k] = table_entry(mesh.nbr, min(e, re - 1));
           if (e >= re) ent[k].y = 0x7f800000;  // +inf ends the walk
         }
         bool oc[kScanChunk];
@@ -789,7 +790,7 @@ __device__ __forceinline__ StepOut particle_step(const MeshDev& mesh, const Step
       while (mark) {
         const int m = __builtin_ctz(mark);
         mark &= mark - 1u;
-        const int2 en = load_at(mesh.nbr, wbase + m * LANES);
+        const int2 en = table_entry(mesh.nbr, wbase + m * LANES);
         visit(en.x, __int_as_float(en.y), src.head(en.x));
       }
     }
@@ -855,7 +856,7 @@ __device__ __forceinline__ StepOut particle_step(const MeshDev& mesh, const Step
 #pragma unroll
         for (int k = 0; k < kRowChunk; ++k) {
           const int e = base + k * LANES;
-          ent[k] = load_at(mesh.nbr, min(e, re - 1));
+          ent[k] = table_entry(mesh.nbr, min(e, re - 1));
           if (e >= re) ent[k].y = 0x7f800000;
         }
 #pragma unroll

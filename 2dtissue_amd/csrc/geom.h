@@ -36,6 +36,10 @@ struct MeshDev {
   const int2* nbr;         // (vertex, float bits of the geodesic distance), rows ascending in distance
 };
 
+// entry e of the geodesic table: the table alone grows with the square of sigma (100,000 vertices pass 2^29
+// entries of 8 bytes at sigma 0.25), so its offsets take 64 bits (load_at's take 32)
+__host__ __device__ inline int2 table_entry(const int2* nbr, int e) { return nbr[(uint32_t)e]; }
+
 // ------------------------------------------------------------------ seam wrap (FP64)
 
 // The predicates below combine their comparisons with & and | rather than && and ||: the

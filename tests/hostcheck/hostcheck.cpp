@@ -109,6 +109,13 @@ void hc_seam_fold_many(int n, const double* a, double* p, double* heading, int m
                      ? 1 : 0;
 }
 
+// entry e of a geodesic table as the kernels address it
+void hc_table_entry(const void* nbr, int e, int* out) {
+  const int2 v = tdev::table_entry((const int2*)nbr, e);
+  out[0] = v.x;
+  out[1] = v.y;
+}
+
 double hc_wrap_heading(double t) { return tdev::wrap_heading(t); }
 
 void hc_seam_wrap_quarter_many(int n, const double* a, const double* p, int max_crossings, int* quarter) {
