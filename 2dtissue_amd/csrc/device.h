@@ -379,7 +379,7 @@ struct WaveWalk {
 struct NoPlaced {
   __device__ void operator()(int) const {}
 };
-constexpr int kOwnerShift = 26;  // vertex ids below 2^26 (checked by the launcher)
+constexpr int kOwnerShift = 26;  // vertex ids below 2^26 (size_error)
 
 // The alignment sum of one particle over the FP64 cosines and sines of its neighbours' headings, by the
 // whole wave (all lanes present): rs .. re its row. A lane takes one entry and its bucket, then one

@@ -61,7 +61,7 @@ Engine::Engine(tissue_mesh* m, int R_, const int* n_, const tissue_params* p_) {
       tot += n_[r];
       nmax = std::max(nmax, n_[r]);
     }
-    if (tot > INT_MAX / 16) throw ApiError(TISSUE_E_INVALID_ARG, "too many particles");
+    if (const char* e = size_error(tot, m->m.nv)) throw ApiError(TISSUE_E_INVALID_ARG, e);
     ntot = (int)tot;
     HIP_OK(hipGetDevice(&device));
     mesh = m;

@@ -374,7 +374,7 @@ TISSUE_STEP_SHAPES(X)
 hipError_t launch_step_tiled(int lanes, int phys, int block, bool tape, bool wave, const MeshDev& mesh,
                              const ReplicaDesc* reps, const TileDesc* tiles, int n_tiles, const BucketSet& bin,
                              const BucketSet& bout, const BucketSet& bclr, const TiledIO& io, hipStream_t st) {
-  if (block < 64 || block > kStepMaxBlock || block % 64 || n_tiles < 1 || mesh.nv >= 1 << kOwnerShift)
+  if (block < 64 || block > kStepMaxBlock || block % 64 || n_tiles < 1 || mesh.nv >= kMaxVertices)
     return hipErrorInvalidValue;
 #define X(L, P)                \
   if (lanes == L && phys == P) \

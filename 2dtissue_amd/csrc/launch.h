@@ -13,6 +13,16 @@ namespace tissue {
 // up to 2^22 particles per replica stay inside int64
 constexpr double kPhiScale = 1099511627776.0;  // 2^40
 
+// what a system may have: particle and vertex numbers that the kernels' 32-bit byte offsets (load_at) and the
+// whole-wave walk's list (kOwnerShift) can hold. Null, or what is too large
+constexpr long kMaxParticlesTotal = 0x7fffffffl / 16;
+constexpr long kMaxVertices = 1l << tdev::kOwnerShift;
+inline const char* size_error(long particles, long vertices) {
+  if (particles > kMaxParticlesTotal) return "too many particles";
+  if (vertices >= kMaxVertices) return "too many UV vertices (at most 2^26 - 1)";
+  return nullptr;
+}
+
 struct OrderPartial {
   long long cs, sn;  // sums of cos / sin of the new headings, fixed point (kPhiScale)
   int sgn, pad;      // sum of sign(x vy - y vx)

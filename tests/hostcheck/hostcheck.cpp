@@ -7,6 +7,7 @@
 
 #include "../../2dtissue_amd/csrc/geodesic.h"
 #include "../../2dtissue_amd/csrc/geom.h"
+#include "../../2dtissue_amd/csrc/launch.h"
 
 extern "C" {
 
@@ -115,6 +116,9 @@ void hc_table_entry(const void* nbr, int e, int* out) {
   out[0] = v.x;
   out[1] = v.y;
 }
+
+// 0: a system of these sizes is taken; 1: refused
+int hc_size_refused(long particles, long vertices) { return tissue::size_error(particles, vertices) ? 1 : 0; }
 
 double hc_wrap_heading(double t) { return tdev::wrap_heading(t); }
 
