@@ -416,6 +416,7 @@ int Engine::checked_first_row(int first_row, int n_steps) const {
 
 const float* Engine::upload_call_noise(const float* h, int n_steps) {
   const size_t need = (size_t)std::max(n_steps, 0) * ntot;
+  if (need == 0) return nullptr;  // no step, no rows (and no launch without a workgroup)
   if (call_noise_cap < need) {
     HIP_OK(hipStreamSynchronize(stream));
     drop_graphs();
