@@ -20,9 +20,10 @@ struct LossDev {
   float target, w_order, w_velocity;
 };
 
-// per replica: out[2r] = phi_T, out[2r+1] = order loss; seeds lr = 0, lt = d loss / d theta_T
+// per replica: out[2r] = phi_T, out[2r+1] = order loss; seeds lr = 0, lt = d loss / d theta_T, mx[r] = max |lt|
+// (float bits)
 hipError_t launch_adj_seed(int R, const ReplicaDesc* reps, const float4* xycs, const LossDev& L, const unsigned* halt,
-                           float2* lr, float* lt, double* out, hipStream_t st);
+                           float2* lr, float* lt, double* out, unsigned* mx, hipStream_t st);
 // One launch of the reverse pass (adjoint.hip), by `lanes` (1 to 16) lanes per particle: kFactors: step p's
 // factors from the adjoint (lr_in, lt_in) of the state after it; kGather: the adjoint (lr_out, lt_out)
 // of the state before step q from step q's factors; kBoth: kGather of q, then kFactors of p = q - 1.

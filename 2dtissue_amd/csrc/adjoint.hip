@@ -22,12 +22,15 @@
 // is linear in lambda, so only the loss sources are scaled by 2^-E_r and the FP64 parameter
 // accumulators by 2^E_r. E_r is raised whenever |lambda| outgrows 2^20: the gather records each
 // replica's max |lambda| (one atomic per wave), and the next factors are scaled by the matching power
-// of two and carry E_r forward. In kBoth the factors follow in the same kernel, before that max is
-// complete, so they go by the max of the step before, less the scaling it has caused already: one step
-// later than kFactors, |lambda| then reaches 2^20 times one more step's growth, far inside FP32. The
-// scaling is exact either way, so both give the same
-// gradients (but for values 2^-126 below their replica's largest, which underflow in one or the other). (Slots alternate by step, so that no
-// kernel reads one that another thread of it writes.)
+// of two and carry E_r forward (the first ones by the seeds' max). In kBoth the factors follow in the same
+// kernel, before that max is complete, so they go by the max of the step before, less the scaling it has
+// caused already: |lambda| then reaches 2^21 times the growth of two steps where by kFactors it reaches 2^21
+// times that of one, so FP32 holds growths below 2^53 a step instead of 2^106 (and large velocity weights,
+// which nothing scales before the first max, times one more step's growth). An adjoint that leaves FP32 stays
+// non-finite back to the initial state, where a particle's own terms carry it; the engine then takes the pass
+// again by kFactors and kGather alone. The scaling is exact either way, so both give the same gradients (but
+// for values 2^-126 below their replica's largest, which underflow in one or the other). (Slots alternate by
+// step, so that no kernel reads one that another thread of it writes.)
 #include <hip/hip_runtime.h>
 
 #include "adjoint.h"
@@ -86,9 +89,12 @@ __device__ double block_sum(double v, double* tmp) {
 }
 
 // one block per replica: polar order of the final state and the seeds of the heading adjoint
+// (mx: their largest, float bits)
 __global__ void k_adj_seed(const ReplicaDesc* reps, const float4* xycs, LossDev L, const unsigned* halt, float2* lr,
-                           float* lt, double* out) {
+                           float* lt, double* out, unsigned* mx) {
   __shared__ double tmp[kAdjBlock / 64];
+  __shared__ unsigned s_mx;
+  if (threadIdx.x == 0) s_mx = 0u;
   const int r = blockIdx.x;
   const int off = reps[r].off, n = reps[r].n;
   double cx = 0.0, cy = 0.0;
@@ -104,12 +110,18 @@ __global__ void k_adj_seed(const ReplicaDesc* reps, const float4* xycs, LossDev 
   const bool ok = halt[r] == 0u;
   // d phi / d theta_i = (-Px sin theta_i + Py cos theta_i) / (n |P|)
   const double coef = (ok && norm > 0.0) ? L.w_order * 2.0 * (phi - L.target) / (n * norm) : 0.0;
+  float largest = 0.f;
   for (int i = threadIdx.x; i < n; i += blockDim.x) {
     const float4 q = xycs[off + i];
+    const float l = (float)(coef * (-Px * (double)q.w + Py * (double)q.z));
     lr[off + i] = make_float2(0.f, 0.f);
-    lt[off + i] = (float)(coef * (-Px * (double)q.w + Py * (double)q.z));
+    lt[off + i] = l;
+    largest = fmaxf(largest, fabsf(l));
   }
+  atomicMax(&s_mx, __float_as_uint(largest));
+  __syncthreads();
   if (threadIdx.x == 0) {
+    mx[r] = s_mx;
     out[2 * r] = phi;
     out[2 * r + 1] = L.w_order * (phi - L.target) * (phi - L.target);
   }
@@ -392,8 +404,8 @@ inline int cdiv(long a, long b) { return (int)((a + b - 1) / b); }
 }  // namespace
 
 hipError_t launch_adj_seed(int R, const ReplicaDesc* reps, const float4* xycs, const LossDev& L, const unsigned* halt,
-                           float2* lr, float* lt, double* out, hipStream_t st) {
-  hipLaunchKernelGGL(k_adj_seed, dim3(R), dim3(kAdjBlock), 0, st, reps, xycs, L, halt, lr, lt, out);
+                           float2* lr, float* lt, double* out, unsigned* mx, hipStream_t st) {
+  hipLaunchKernelGGL(k_adj_seed, dim3(R), dim3(kAdjBlock), 0, st, reps, xycs, L, halt, lr, lt, out, mx);
   return hipGetLastError();
 }
 

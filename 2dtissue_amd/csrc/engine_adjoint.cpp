@@ -18,6 +18,7 @@
 #include <climits>
 #include <cstdlib>
 #include <cmath>
+#include <cstring>
 
 #include "engine.h"
 
@@ -48,6 +49,17 @@ LossDev make_loss(const tissue_loss& l, int n_steps) {
     d.phase[m] = (float)l.phase[m];
   }
   return d;
+}
+
+// n floats at p (a loop without branches)
+bool all_finite(const void* p, size_t n) {
+  uint32_t bad = 0;
+  for (size_t i = 0; i < n; ++i) {
+    uint32_t w;
+    std::memcpy(&w, static_cast<const char*>(p) + 4 * i, 4);
+    bad |= (w & 0x7f800000u) == 0x7f800000u ? 1u : 0u;
+  }
+  return bad == 0;
 }
 
 }  // namespace
@@ -257,13 +269,44 @@ int32_t Engine::adjoint(int T, const float* nz, size_t stride, int K, const tiss
   v.halt = d_halt;
   v.single = R == 1 ? 1 : 0;
   v.acc = a.acc;
-  auto begin_reverse = [&] {
+  std::vector<double> seed, red;
+  std::vector<float2> lr;
+  std::vector<float> lt;
+  std::vector<int> sexp;
+  double rev_ms = 0.0;
+  // mx_slot: the slot of mx that the first factors read
+  auto begin_reverse = [&](int mx_slot) {
     HIP_OK(hipEventRecord(ev0, stream));
-    HIP_OK(launch_adj_seed(R, d_reps, xycs[sphase], L, d_halt, a.lr[0], a.lt[0], a.out_seed, stream));
     HIP_OK(hipMemsetAsync(a.acc, 0, kAdjAcc * N * sizeof(double), stream));
     HIP_OK(hipMemsetAsync(a.sexp, 0, 2 * R * sizeof(int), stream));
     HIP_OK(hipMemsetAsync(a.sup, 0, 2 * R * sizeof(int), stream));
     HIP_OK(hipMemsetAsync(a.mx, 0, 3 * R * sizeof(unsigned), stream));
+    HIP_OK(launch_adj_seed(R, d_reps, xycs[sphase], L, d_halt, a.lr[0], a.lt[0], a.out_seed, a.mx + mx_slot * R, stream));
+  };
+  auto end_reverse = [&] {
+    HIP_OK(launch_adj_reduce(R, d_reps, ntot, a.acc, a.out_red, stream));
+    HIP_OK(hipEventRecord(ev1, stream));
+    seed.resize(2 * (size_t)R);
+    red.resize(kAdjAcc * (size_t)R);
+    lr.resize(N);
+    lt.resize(N);
+    sexp.resize(R);
+    HIP_OK(hipMemcpyAsync(seed.data(), a.out_seed, seed.size() * sizeof(double), hipMemcpyDeviceToHost, stream));
+    HIP_OK(hipMemcpyAsync(red.data(), a.out_red, red.size() * sizeof(double), hipMemcpyDeviceToHost, stream));
+    HIP_OK(hipMemcpyAsync(lr.data(), lr_end, N * sizeof(float2), hipMemcpyDeviceToHost, stream));
+    HIP_OK(hipMemcpyAsync(lt.data(), lt_end, N * sizeof(float), hipMemcpyDeviceToHost, stream));
+    HIP_OK(hipMemcpyAsync(sexp.data(), sexp_end, R * sizeof(int), hipMemcpyDeviceToHost, stream));
+    HIP_OK(hipStreamSynchronize(stream));
+    float ms = 0.f;
+    HIP_OK(hipEventElapsedTime(&ms, ev0, ev1));
+    rev_ms += ms;
+  };
+  // whether the adjoint stayed within FP32 (adjoint.hip); a sum alone may be beyond FP64 of itself
+  auto in_range = [&] {
+    for (int r = 0; r < R; ++r)
+      for (int k = 0; k < kAdjAcc; ++k)
+        if (!std::isfinite(red[kAdjAcc * r + k]) && sexp[r] < 512) return false;
+    return all_finite(lr.data(), 2 * N) && all_finite(lt.data(), N);
   };
   if (whole_tape(T)) {
     Tape& tp = a.whole;
@@ -279,7 +322,6 @@ int32_t Engine::adjoint(int T, const float* nz, size_t stride, int K, const tiss
     HIP_OK(hipMemcpyAsync(xycs[sphase], tp.xycs + T * N, N * sizeof(float4), hipMemcpyDeviceToDevice, stream));
     HIP_OK(hipMemcpyAsync(th[sphase], tp.th + T * N, N * sizeof(float), hipMemcpyDeviceToDevice, stream));
     HIP_OK(hipMemcpyAsync(vid[sphase], tp.vid + T * N, N * sizeof(int), hipMemcpyDeviceToDevice, stream));
-    begin_reverse();
     // half h of the ring: the buckets of the states T - 1 - h kRingHalf .. downwards
     const int halves = (T + kRingHalf - 1) / kRingHalf;
     hipStream_t side = a.rec_stream[0];
@@ -291,44 +333,58 @@ int32_t Engine::adjoint(int T, const float* nz, size_t stride, int K, const tiss
         bucket_state_into(tp.vid + q * N, ring_set(q), side, h >= 2 ? tp.vid + (q + 2 * kRingHalf) * N : nullptr);
       HIP_OK(hipEventRecord(a.ev_rec[h & 1], side));
     };
-    if (!a.keep_sets) {
-      fill(0);
-      fill(1);
-    }
-    // launch j: exponents and maxima from slots that launch j - 1 wrote, to the next ones
-    int j = 0;
     v.use_occ = !a.keep_sets && 8L * nmax < md.nv ? 1 : 0;
-    auto launch = [&](int part, int q, int p) {
-      v.sexp_in = a.sexp + (j & 1) * R; v.sexp_out = a.sexp + (1 - (j & 1)) * R;
-      v.sup_in = a.sup + (j & 1) * R; v.sup_out = a.sup + (1 - (j & 1)) * R;
-      v.mx_in = a.mx + (j + 2) % 3 * R; v.mx_out = a.mx + j % 3 * R; v.mx_clear = a.mx + (j + 1) % 3 * R;
-      v.g4_in = a.g4[1 - (j & 1)]; v.part_in = a.part[1 - (j & 1)];
-      v.g4_out = a.g4[j & 1]; v.part_out = a.part[j & 1];
-      if (q >= 0) {
-        v.bs = a.keep_sets ? a.sets[q] : ring_set(q);
-        v.xycs_q = tp.xycs + q * N; v.vid_q = tp.vid + q * N;
-      }
-      if (p >= 0) {
-        v.xycs_p = tp.xycs + p * N; v.th_p = tp.th + p * N; v.fs_p = tp.fs + p * N; v.quarter_p = tp.q + p * N;
-      }
-      HIP_OK(launch_adj_reverse(gather_lanes, part, md, d_reps, d_rid, ntot, L, v, stream));
-      ++j;
-    };
-    v.lr_in = a.lr[0]; v.lt_in = a.lt[0];
-    v.lr_out = a.lr[1]; v.lt_out = a.lt[1];
-    launch(kFactors, -1, T - 1);
-    for (int q = T - 1; q >= 0; --q) {
-      const int at = T - 1 - q, h = at / kRingHalf;
-      if (!a.keep_sets && at % kRingHalf == 0) HIP_OK(hipStreamWaitEvent(stream, a.ev_rec[h & 1], 0));
-      launch(q > 0 ? kBoth : kGather, q, q - 1);
-      if (!a.keep_sets && (at % kRingHalf == kRingHalf - 1 || q == 0)) {
-        HIP_OK(hipEventRecord(a.ev_rev[h & 1], stream));
-        fill(h + 2);
-      }
-    }
+    v.lt_out = a.lt[1];
+    v.lr_out = a.lr[1];
     lr_end = a.lr[1];
     lt_end = a.lt[1];
-    sexp_end = a.sexp + ((j - 1) & 1) * R;
+    // fused: one launch a step (kBoth); else two, for adjoints that grow faster than FP32 lets it follow
+    auto reverse_whole = [&](bool fused) {
+      begin_reverse(2);
+      if (!a.keep_sets) {
+        fill(0);
+        fill(1);
+      }
+      // launch j: factors and maxima from slots that launch j - 1 wrote, to the next ones; e: the slot of the
+      // exponents, which the launches with factors move on
+      int j = 0, e = 0;
+      v.lr_in = a.lr[0];
+      v.lt_in = a.lt[0];
+      auto launch = [&](int part, int q, int p) {
+        v.sexp_in = a.sexp + e * R; v.sexp_out = a.sexp + (1 - e) * R;
+        v.sup_in = a.sup + e * R; v.sup_out = a.sup + (1 - e) * R;
+        v.mx_in = a.mx + (j + 2) % 3 * R; v.mx_out = a.mx + j % 3 * R; v.mx_clear = a.mx + (j + 1) % 3 * R;
+        v.g4_in = a.g4[1 - (j & 1)]; v.part_in = a.part[1 - (j & 1)];
+        v.g4_out = a.g4[j & 1]; v.part_out = a.part[j & 1];
+        if (q >= 0) {
+          v.bs = a.keep_sets ? a.sets[q] : ring_set(q);
+          v.xycs_q = tp.xycs + q * N; v.vid_q = tp.vid + q * N;
+        }
+        if (p >= 0) {
+          v.xycs_p = tp.xycs + p * N; v.th_p = tp.th + p * N; v.fs_p = tp.fs + p * N; v.quarter_p = tp.q + p * N;
+        }
+        HIP_OK(launch_adj_reverse(gather_lanes, part, md, d_reps, d_rid, ntot, L, v, stream));
+        ++j;
+        if (part != kGather) e = 1 - e;
+      };
+      launch(kFactors, -1, T - 1);
+      v.lr_in = a.lr[1];
+      v.lt_in = a.lt[1];
+      for (int q = T - 1; q >= 0; --q) {
+        const int at = T - 1 - q, h = at / kRingHalf;
+        if (!a.keep_sets && at % kRingHalf == 0) HIP_OK(hipStreamWaitEvent(stream, a.ev_rec[h & 1], 0));
+        launch(fused && q > 0 ? kBoth : kGather, q, q - 1);
+        if (!fused && q > 0) launch(kFactors, -1, q - 1);
+        if (!a.keep_sets && (at % kRingHalf == kRingHalf - 1 || q == 0)) {
+          HIP_OK(hipEventRecord(a.ev_rev[h & 1], stream));
+          fill(h + 2);
+        }
+      }
+      sexp_end = a.sexp + e * R;
+      end_reverse();
+    };
+    reverse_whole(true);
+    if (!in_range()) reverse_whole(false);
   } else {
   adjoint_buffers(K, C);
 
@@ -422,7 +478,7 @@ int32_t Engine::adjoint(int T, const float* nz, size_t stride, int K, const tiss
     if (st != TISSUE_OK && status == TISSUE_OK) status = st;
   }
   // reverse
-  begin_reverse();
+  begin_reverse(0);
   if (overlap) {
     HIP_OK(hipEventRecord(a.ev_fwd, stream));  // every checkpoint is written
     for (int c = C - 1; c >= 0; --c) {
@@ -439,21 +495,8 @@ int32_t Engine::adjoint(int T, const float* nz, size_t stride, int K, const tiss
   lr_end = a.lr[cur];
   lt_end = a.lt[cur];
   sexp_end = a.sexp + cur * R;
+  end_reverse();
   }
-  HIP_OK(launch_adj_reduce(R, d_reps, ntot, a.acc, a.out_red, stream));
-  HIP_OK(hipEventRecord(ev1, stream));
-  std::vector<double> seed(2 * (size_t)R), red(kAdjAcc * (size_t)R);
-  std::vector<float2> lr(N);
-  std::vector<float> lt(N);
-  std::vector<int> sexp(R);
-  HIP_OK(hipMemcpyAsync(seed.data(), a.out_seed, seed.size() * sizeof(double), hipMemcpyDeviceToHost, stream));
-  HIP_OK(hipMemcpyAsync(red.data(), a.out_red, red.size() * sizeof(double), hipMemcpyDeviceToHost, stream));
-  HIP_OK(hipMemcpyAsync(lr.data(), lr_end, N * sizeof(float2), hipMemcpyDeviceToHost, stream));
-  HIP_OK(hipMemcpyAsync(lt.data(), lt_end, N * sizeof(float), hipMemcpyDeviceToHost, stream));
-  HIP_OK(hipMemcpyAsync(sexp.data(), sexp_end, R * sizeof(int), hipMemcpyDeviceToHost, stream));
-  HIP_OK(hipStreamSynchronize(stream));
-  float rev = 0.f;
-  HIP_OK(hipEventElapsedTime(&rev, ev0, ev1));
   buckets_stale = true;  // the reverse pass used the bucket sets
   for (int r = 0; r < R; ++r) {
     tissue_grads& o = g[r];
@@ -466,7 +509,7 @@ int32_t Engine::adjoint(int T, const float* nz, size_t stride, int K, const tiss
     o.d_k = red[kAdjAcc * r + 2];
     o.d_tau = red[kAdjAcc * r + 3];
     o.forward_ms = fwd_ms;
-    o.reverse_ms = rev;
+    o.reverse_ms = rev_ms;
   }
   for (int r = 0; r < R; ++r) {
     const double sc = std::ldexp(1.0, sexp[r]);
@@ -476,7 +519,7 @@ int32_t Engine::adjoint(int T, const float* nz, size_t stride, int K, const tiss
       if (d_y0) d_y0[i] = sc * (double)lr[i].y;
     }
   }
-  last_ms = fwd_ms + rev;
+  last_ms = fwd_ms + rev_ms;
   return status;
 }
 
