@@ -180,8 +180,8 @@ struct Engine {
     hipEvent_t ev_fwd = nullptr, ev_ck[kMaxTapes] = {}, ev_rec[kMaxTapes] = {}, ev_rev[kMaxTapes] = {};
     float2* lr[2] = {nullptr, nullptr}; float* lt[2] = {nullptr, nullptr};
     float4 *g4[2] = {nullptr, nullptr}, *part[2] = {nullptr, nullptr};
-    // the whole tape of a run of whole_T steps: its bucket sets (one allocation) are those of every
-    // state (keep_sets) or two halves of kRingHalf filled ahead of the reverse pass
+    // the whole tape, of up to whole_T steps, and bucket sets (one allocation), which the run at hand uses
+    // for those of every state (keep_sets) or as two halves of kRingHalf filled ahead of the reverse pass
     Tape whole;
     int whole_T = 0;
     bool keep_sets = false;
@@ -195,8 +195,11 @@ struct Engine {
   void free_tape(Tape& t);
   static constexpr int kRingHalf = 4;
   void alloc_set_slab(std::vector<BucketSet>& sets, int n);
+  size_t tape_bytes(int T) const;
   bool whole_tape(int T);
   void free_whole_tape();
+  void free_set_slab();
+  void free_tapes();
   void adjoint_common();
   void adjoint_buffers(int K, int C);
   void adjoint_release();
