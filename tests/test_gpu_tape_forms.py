@@ -1,7 +1,7 @@
 """The whole tape's two forms (engine_adjoint.cpp) really taken, and their gradients those of the checkpointed
 form bit for bit: memory budgets that hold the tape and exactly eight bucket sets (the ring), or every state's.
 The device memory that the calls leave held tells the forms apart: all else is the same in both, so they differ
-by their sets, to the 2 MiB in which memory is given out. Horizons on either side of half a ring, of the
+by their sets, to the 2 MiB blocks in which each call's memory is given out. Horizons on either side of half a ring, of the
 ring and of its second turn; replicas sparse on their mesh (a refilled set is cleared where its old state
 was) and dense (cleared whole); raw buckets and sorted ones (the finalize pass on the side stream)."""
 import ctypes as C
@@ -13,9 +13,9 @@ import parity as P
 
 pytestmark = pytest.mark.gpu
 
-# mesh frequency, sigma, sizes; 16 replicas, so that a bucket set is some megabytes
-SPARSE = (32, 0.05, [60, 1, 77, 250] * 4)
-DENSE = (22, 0.1, [700, 650, 610, 33 + 650] * 4)
+# mesh frequency, sigma, sizes; 64 replicas, so that a bucket set is 24 and 12 MB
+SPARSE = (32, 0.05, [60, 1, 77, 250] * 16)
+DENSE = (22, 0.1, [700, 650, 610, 33 + 650] * 16)
 
 
 def free_bytes(T):
@@ -64,4 +64,4 @@ def test_forms_are_taken_and_agree(T, monkeypatch, steps, system, sorted_buckets
                 assert np.array_equal(a, c), (form, call)
         held[form] = before - free_bytes(T)
         b.close()
-    assert abs(held["kept"] - held["ring"] - (steps + 2 - 8) * set_bytes) <= 2**21 < set_bytes, (held, set_bytes)
+    assert abs(held["kept"] - held["ring"] - (steps + 2 - 8) * set_bytes) <= 2**22 < set_bytes / 2, (held, set_bytes)
