@@ -241,12 +241,15 @@ hipError_t launch_flags_begin(int R, const unsigned* halt, unsigned* rows, int* 
 // neighbour counts and the R replicas' halt flags zeroed
 hipError_t launch_adopt(int n, const float* x, const float* y, const float* th, float4* xycs, float* th_out, float* vx,
                         float* vy, int* nbr, int R, unsigned* halt, hipStream_t st);
-// particles [first, first + n) as consecutive arrays at out (mapped host memory): x, y, theta, vid [n]
-// (16 bytes a particle); vx, vy [n], r3d [n][3], face, nbr [n] (28 bytes)
-hipError_t launch_pack_state(int first, int n, const float4* xycs, const float* th, const int* vid, float* out,
-                             hipStream_t st);
+// particles [first, first + n) as consecutive arrays at out (mapped host memory), those that are asked for:
+// array k (x, y, theta, vid) at out + at[k] n unless at[k] < 0
+struct PackAt { int at[5]; };
+hipError_t launch_pack_state(int first, int n, const float4* xycs, const float* th, const int* vid, const PackAt& where,
+                             float* out, hipStream_t st);
+// the same of vx, vy, r3d ([n][3], so three words of n), face, nbr
 hipError_t launch_pack_outputs(int first, int n, const float* vx, const float* vy, const float* r3x, const float* r3y,
-                               const float* r3z, const int* face, const int* nbr, float* out, hipStream_t st);
+                               const float* r3z, const int* face, const int* nbr, const PackAt& where, float* out,
+                               hipStream_t st);
 // n words of mapped host memory into device memory
 hipError_t launch_fetch(size_t n, const float* from, float* to, hipStream_t st);
 // counts, masks and list lengths of n_sets (1 to 3) bucket sets of R replicas zeroed
