@@ -750,6 +750,9 @@ void build_distance_table(UVMesh& m, double cutoff) {
   // src/simulation/Locomotion.cpp:127-138) and round to FP32: row v gathers its own entries and
   // the transposed entries of the rows that reach v, keeps the minimum per column, and sorts by
   // (FP32 distance, column)
+  int64_t entries = 0;
+  for (const auto& row : rows) entries += (int64_t)row.size();
+  check_table_entries(entries);
   std::vector<int32_t> in_ptr(nv + 1, 0);
   for (int s = 0; s < nv; ++s)
     for (auto [v, t] : rows[s]) ++in_ptr[v + 1];
@@ -786,6 +789,9 @@ void build_distance_table(UVMesh& m, double cutoff) {
     merge();
     for (auto& t : pool) t.join();
   }
+  entries = 0;
+  for (const auto& row : out) entries += (int64_t)row.size();
+  check_table_entries(entries);
   m.cutoff = cutoff;
   m.row_ptr.assign(nv + 1, 0);
   m.col.clear();

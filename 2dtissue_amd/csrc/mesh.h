@@ -11,6 +11,7 @@
 #pragma once
 #include <cstdint>
 #include <functional>
+#include <stdexcept>
 #include <string>
 #include <utility>
 #include <vector>
@@ -81,6 +82,13 @@ UVMesh cut_and_parameterize(const SurfaceMesh& m, int pa = -1, int pm = -1, int 
 
 // ---- acceleration structures ----
 void build_face_buckets(UVMesh& uv, int grid = 0);        // grid <= 0: automatic
+// entries of the geodesic table that 32-bit row numbers can name, with room for the walks, which step up to some
+// thousand entries past the end of a row
+constexpr int64_t kMaxTableEntries = INT32_MAX - (1 << 16);
+inline void check_table_entries(int64_t n) {
+  if (n > kMaxTableEntries)
+    throw std::runtime_error("distance table: more than 2^31 - 2^16 entries (build it for a smaller sigma)");
+}
 // geodesic distance on the open mesh, truncated at cutoff: exact polyhedral distances by window
 // propagation (geodesic.h), one source per task on the host's threads
 void build_distance_table(UVMesh& uv, double cutoff);

@@ -8,6 +8,7 @@
 #include "../../2dtissue_amd/csrc/geodesic.h"
 #include "../../2dtissue_amd/csrc/geom.h"
 #include "../../2dtissue_amd/csrc/launch.h"
+#include "../../2dtissue_amd/csrc/mesh.h"
 
 extern "C" {
 
@@ -119,6 +120,16 @@ void hc_table_entry(const void* nbr, int e, int* out) {
 
 // 0: a system of these sizes is taken; 1: refused
 int hc_size_refused(long particles, long vertices) { return tissue::size_error(particles, vertices) ? 1 : 0; }
+
+// 0: a geodesic table of n entries is built; 1: refused
+int hc_table_refused(int64_t n) {
+  try {
+    tissue::check_table_entries(n);
+    return 0;
+  } catch (const std::runtime_error&) {
+    return 1;
+  }
+}
 
 double hc_wrap_heading(double t) { return tdev::wrap_heading(t); }
 
