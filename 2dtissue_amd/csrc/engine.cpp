@@ -572,6 +572,7 @@ void Engine::enqueue(const Shape& s, int n_steps, const float* nz, size_t stride
         io.halt_clr = d_rows + (size_t)((t + 2) % 3) * R;
         io.first_bad = d_first_bad;
         io.step = t;
+        io.areas = step_areas(nmax, s.block, phys_lanes(s));
         io.visit = d_visit;
         if (tape) {
           const size_t N = ntot;

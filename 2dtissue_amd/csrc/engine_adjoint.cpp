@@ -450,6 +450,7 @@ int32_t Engine::adjoint(int T, const float* nz, size_t stride, int K, const tiss
       io.halt_clr = tp.rows + (size_t)((q + 2) % 3) * R;
       io.first_bad = tp.first_bad;
       io.step = q;
+      io.areas = step_areas(nmax, s.block, phys_lanes(s));
       io.tape_fs = tp.fs + q * N;
       io.tape_q = tp.q + q * N;
       HIP_OK(launch_step_tiled(s.lanes, phys_lanes(s), s.block, true, !raw_buckets, md, d_reps, d_tiles, n_phys, segment_set(tp, kc, q),

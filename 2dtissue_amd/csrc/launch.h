@@ -3,6 +3,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "device.h"
 
 namespace tissue {
@@ -90,6 +92,7 @@ struct TiledIO {
   unsigned* halt_clr;       // [R] the third flag row, cleared for the next step
   int* first_bad;           // [R] first step of the run that raised a flag
   int step;                 // step index within the run
+  int areas;                // waves of a workgroup that can hold particles (step_areas)
   float4* tape_fs;          // adjoint tape of this step, [ntot] (Fx, Fy, Sx, Sy); used by the TAPE variant
   int* tape_q;              // [ntot] quarter turns of the seam wrap
   int2* visit;              // [ntot] (na, vh) of StepOut: the neighbour set the step's own walk
@@ -153,16 +156,22 @@ constexpr int kStepMaxBlock = 512;
 // such launches keep the mask up to date: for the others it would be one more memory-side atomic per
 // occupied vertex (63,000 of them in a step of 100,000 particles).
 constexpr int kOccWordsPerParticle = 8;
+// Waves of a workgroup that can hold particles: of replicas of at most nmax particles, the first so many lanes.
+// Only they have a walk area: areas for the waves past the last particle too, which end at once, kept other
+// workgroups out of the CU's LDS (4,000 replicas of 30 particles in workgroups of 256 99 -> 76 us per step)
+inline int step_areas(int nmax, int block, int phys) {
+  return (int)((std::min<long>(nmax, block / phys) * phys + 63) / 64);
+}
 // LDS of one workgroup of the tiled step kernel: the waves' walk areas and the staged mask
-inline size_t step_lds_bytes(int nv, int block, int lanes, int phys, bool crowded, bool occ) {
-  return (tdev::wave_area(lanes, phys, crowded) ? (size_t)(block / 64) * sizeof(tdev::WaveWalk) : 0) +
+inline size_t step_lds_bytes(int nv, int areas, int lanes, int phys, bool crowded, bool occ) {
+  return (tdev::wave_area(lanes, phys, crowded) ? (size_t)areas * sizeof(tdev::WaveWalk) : 0) +
          (occ ? sizeof(unsigned) * (size_t)tdev::occ_words(nv) : 0);
 }
 constexpr size_t kStepMaxLds = 64 * 1024;  // what a launch may ask for without raising the limit
 static_assert(kStepMaxBlock / 64 * sizeof(tdev::WaveWalk) <= kStepMaxLds, "the areas of the largest workgroup");
 inline bool stage_occupancy(int nv, int block, int lanes, int phys) {
   return phys <= lanes && tdev::occ_words(nv) <= kOccWordsPerParticle * (block / phys) &&
-         step_lds_bytes(nv, block, lanes, phys, false, true) <= kStepMaxLds;
+         step_lds_bytes(nv, block / 64, lanes, phys, false, true) <= kStepMaxLds;
 }
 // Physical lanes per particle for sums laid out over `lanes` lanes (the results are the same for any).
 // As many as the layout where the chip is full; more where it is not and a step's longest chain counts

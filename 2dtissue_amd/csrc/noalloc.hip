@@ -258,6 +258,7 @@ extern "C" int32_t tissue_step_noalloc(const tissue_mesh* mc, const tissue_param
     io.halt_clr = a.rows + 2;
     io.first_bad = a.first_bad;
     io.step = 0;
+    io.areas = tissue::step_areas(n, block, phys);
     HIP_OK(tissue::launch_step_tiled(lanes, phys, block, false, sorted != 0, md, a.rep, a.tiles, n_tiles, b[0], b[1], b[2], io, st));
     hipLaunchKernelGGL(k_noalloc_finish, dim3(cdiv(n, tissue::kPhiBlock)), dim3(tissue::kPhiBlock), 0, st, n, io.xycs_out,
                        x_out, y_out, io.partial, n_tiles * tissue::partials_per_tile(block), phi, io.halt_out, a.bad,

@@ -119,7 +119,7 @@ __global__ void __launch_bounds__(kStepMaxBlock) k_step_tiled(MeshDev mesh, cons
   extern __shared__ __align__(16) unsigned char smem[];
   constexpr bool kArea = wave_area(LANES, P, WAVE);
   WaveWalk* ww = kArea ? reinterpret_cast<WaveWalk*>(smem) + (threadIdx.x >> 6) : nullptr;
-  unsigned* s_occ = reinterpret_cast<unsigned*>(smem + (kArea ? (blockDim.x >> 6) * sizeof(WaveWalk) : 0));
+  unsigned* s_occ = reinterpret_cast<unsigned*>(smem + (kArea ? io.areas * sizeof(WaveWalk) : 0));
   const TileDesc tile = tiles[blockIdx.x];
   if (tile.r < 0) return;  // idle padding workgroup (whole block)
   const int r = tile.r;
@@ -128,6 +128,7 @@ __global__ void __launch_bounds__(kStepMaxBlock) k_step_tiled(MeshDev mesh, cons
   const int lane = tid & (P - 1);
   const int i = tile.first + tid / P;
   const bool active = i < rep.n;
+  const bool wave_holds = __builtin_amdgcn_ballot_w64(active) != 0;  // (by all lanes: not behind a branch on active)
   const int g = rep.off + i;
   // the particle's inputs first: their loads are in flight during the set-up below
   float4 me = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -158,7 +159,9 @@ __global__ void __launch_bounds__(kStepMaxBlock) k_step_tiled(MeshDev mesh, cons
 
   int sgn = 0;
   long long pcs = 0, psn = 0;
-  if (active || (kArea && !halt)) {  // such a wave needs all of its lanes
+  // a wave with an area needs all of its lanes where one holds a particle; waves past the last particle have no
+  // area (step_areas) and do nothing
+  if (active || (kArea && !halt && wave_holds)) {
     if (halt) {
       if (lane == 0) {
         io.xycs_out[g] = me;
@@ -220,7 +223,7 @@ template <int LANES, int P, bool OCC, bool WAVE>
 void launch_tiled_mode(int block, bool tape, const MeshDev& mesh, const ReplicaDesc* reps, const TileDesc* tiles,
                        int n_tiles, const BucketSet& bin, const BucketSet& bout, const BucketSet& bclr,
                        const TiledIO& io, hipStream_t st) {
-  const size_t lds = step_lds_bytes(mesh.nv, block, LANES, P, WAVE, OCC);
+  const size_t lds = step_lds_bytes(mesh.nv, io.areas, LANES, P, WAVE, OCC);
   if (tape)
     hipLaunchKernelGGL((k_step_tiled<LANES, P, true, OCC, false, WAVE>), dim3(n_tiles), dim3(block), lds, st, mesh, reps,
                        tiles, bin, bout, bclr, io);
