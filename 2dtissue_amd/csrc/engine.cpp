@@ -377,7 +377,8 @@ void Engine::ensure_tiles(const Shape& s) {
   for (int r = 0; r < R; ++r) {
     begin[r] = (int)logical.size();
     const int nq = cdiv(n[r], per);
-    for (int q = 0; q < nq; ++q) logical.push_back(TileDesc{r, q * per, q, nq, (int)logical.size(), 0});
+    for (int q = 0; q < nq; ++q)
+      logical.push_back(TileDesc{r, q * per, q, (int)logical.size(), clear_end(md.nv, q - 1, nq), clear_end(md.nv, q, nq)});
   }
   begin[R] = (int)logical.size();
   std::vector<TileDesc> phys;

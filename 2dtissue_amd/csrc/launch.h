@@ -40,11 +40,16 @@ struct ReplicaDesc {
 struct TileDesc {
   int r;        // replica; -1 marks an idle workgroup (padding of the XCD-balanced order)
   int first;    // first particle of the tile, counted within the replica
-  int q, nq;    // tile index within the replica, number of tiles of the replica
+  int q;        // tile index within the replica
   int logical;  // the tile's order-parameter partials start at logical * partials_per_tile(block)
                 // (tiles of a replica are consecutive)
-  int pad;
+  int clr_lo, clr_hi;  // the tile clears these vertices of its replica's oldest bucket set (clear_end)
 };
+// where the share of tile q of nq ends and the next one's begins: whole words of the occupancy mask
+__host__ __device__ inline int clear_end(int nv, long q, long nq) {
+  const long share = ((nv + nq - 1) / nq + 31) & ~31l, end = (q + 1) * share;
+  return (int)(end < nv ? end : nv);
+}
 
 // one vertex-bucket set of all replicas: replica r owns count[r*nv ..], slot[r*nv*kSlots ..],
 // the occupancy mask occ[r*occ_words(nv) ..], the counters ovf_n[r], big_n[r] and

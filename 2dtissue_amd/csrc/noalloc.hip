@@ -129,7 +129,8 @@ __global__ void k_noalloc_setup(SetupArgs a) {
     if (t < tdev::occ_words(a.nv)) a.sets[k].occ[t] = 0u;
     if (t == 0) *a.sets[k].ovf_n = *a.sets[k].big_n = 0;
   }
-  if (t < a.n_tiles) a.tiles[t] = TileDesc{0, t * a.per_tile, t, a.n_tiles, t, 0};
+  if (t < a.n_tiles) a.tiles[t] = TileDesc{0, t * a.per_tile, t, t, tissue::clear_end(a.nv, t - 1, a.n_tiles),
+                                            tissue::clear_end(a.nv, t, a.n_tiles)};
   if (t < 3) a.rows[t] = 0u;
   if (t == 0) {
     *a.rep = a.rep_value;
