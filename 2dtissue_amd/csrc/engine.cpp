@@ -515,7 +515,7 @@ Shape Engine::resolve_for(Shape s) const {
     s.xcd = 0;
   } else {
     int lanes = 0, block = 0;
-    tiled_default_shape(R, ntot, &lanes, &block);
+    tiled_default_shape(R, ntot, nmax, md.nv, &lanes, &block);
     s.lanes = s.lanes > 0 ? s.lanes : lanes;
     s.block = s.block > 0 ? s.block : block;
     s.spl = s.spl > 0 ? s.spl : kDefaultSpl;

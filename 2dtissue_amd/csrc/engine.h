@@ -218,7 +218,7 @@ struct Engine {
   void ensure_tiles(const Shape& s);
   void enqueue(const Shape& s, int n_steps, const float* noise, size_t stride, Tape* tape = nullptr);
   Shape resolve_for(Shape s) const;
-  int phys_lanes(const Shape& s) const { return tissue::phys_lanes(s.lanes, ntot, md.nv, s.block); }
+  int phys_lanes(const Shape& s) const { return tissue::phys_lanes(s.lanes, ntot, nmax, md.nv, s.block); }
 };
 
 }  // namespace tissue

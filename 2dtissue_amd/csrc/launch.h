@@ -183,12 +183,14 @@ inline bool stage_occupancy(int nv, int block, int lanes, int phys) {
 // (MI355X, us per step): 4 -> 8 at 9,001 particles 23.0 / 18.8, 20,000 32.3 / 26.2, 30,000 in 30 replicas
 // 21.4 / 21.0, but 40,000 33.5 / 37.0 and 100,000 72.6 / 78.2; 8 -> 16 at 5,000 particles 16.7 / 14.1, 8,000
 // 17.9 / 14.6; 2 -> 4 for replicas sparse on a mesh too large for the occupancy mask, 64 x 2,000
-// 57.4 / 55.1, but with the mask 80,000 particles 36.6 / 36.6, 250,000 85.5 / 85.5 and 525,000 159 / 164.
+// 57.4 / 55.1, but with the mask 80,000 particles 36.6 / 36.6, 250,000 85.5 / 85.5 and 525,000 159 / 164. Replicas
+// of at most 64 particles keep 4 earlier, as their tiles at 8 are many and half empty: 909 replicas of 33 particles
+// 25.5 / 29.6, 600 of 50 23.1 / 26.7, but 449 of 55 20.4 / 19.9.
 // Fewer lanes than the layout were slower throughout (525,000 particles, 2 -> 1: 163 / 192, before the
 // figures above).
-inline int phys_lanes(int lanes, int ntot, int nv, int block) {
+inline int phys_lanes(int lanes, int ntot, int nmax, int nv, int block) {
   if (lanes == 8 && ntot <= 16384) return 16;
-  if (lanes == 4 && ntot <= 32768) return 8;
+  if (lanes == 4 && ntot <= (nmax <= 64 ? 24576 : 32768)) return 8;
   if (lanes == 2 && ntot <= 163840 && !stage_occupancy(nv, block, 2, 2)) return 4;
   return lanes;
 }
@@ -198,18 +200,22 @@ constexpr int kResidentMaxBlock = 512;  // of the persistent kernel's shapes; se
 inline int resident_default_lanes(int nmax) { return nmax <= 256 ? 8 : (nmax <= 1024 ? 4 : (nmax <= 2048 ? 2 : 1)); }
 
 // Default launch shape of the tiled step kernel (lanes per particle, threads per workgroup) for
-// R replicas of ntot particles in all. Measured on MI355X: a single system of a few thousand
-// particles fills few CUs, so more lanes per particle shorten its critical path, and one-wave
+// R replicas of ntot particles in all, the largest of nmax, on nv vertices. Measured on MI355X: a single system
+// of a few thousand particles fills few CUs, so more lanes per particle shorten its critical path, and one-wave
 // workgroups let every wave start its walk without waiting for another at the staging barrier
 // (2,000 particles: 32 lanes in 64 threads 10.08 us, 16 in 64 10.48 us, 16 in 128 10.54 us, 64 in 64
 // 10.19 us, 8 in 64 10.83 us); beyond, workgroups of 128 leave a shorter last round than 256 (525,000
 // particles in 256 replicas 34.1 -> 33.2 ms per 200 steps; 100,000 particles 68.5 -> 67.3 us per step, 64
-// threads 66.6, but slower in the batch); a single 100,000-particle system is fastest with 4 (2 lanes
-// 82.6 us), a large batch with 2 (autotuned).
-inline void tiled_default_shape(int R, int ntot, int* lanes, int* block) {
+// threads 66.6, but slower in the batch), but replicas that fit in one workgroup of 256 and not in one of 128
+// take that (1,000 replicas of 100 particles 41.7 us against 45.1 in twos of 128, 1,538 of 65 54.5 against 61.8);
+// a single 100,000-particle system is fastest with 4 (2 lanes 82.6 us), a large batch with 2 (autotuned).
+inline void tiled_default_shape(int R, int ntot, int nmax, int nv, int* lanes, int* block) {
   const int big_lanes = R == 1 ? 4 : 2;
   *lanes = ntot <= 4096 ? 32 : (ntot <= 8192 ? 8 : (ntot <= 65536 ? 4 : big_lanes));
   *block = ntot <= 4096 ? 64 : 128;
+  if (*block == 128 && R > 1 && nmax > 128 / phys_lanes(*lanes, ntot, nmax, nv, 128) &&
+      nmax <= 256 / phys_lanes(*lanes, ntot, nmax, nv, 256))
+    *block = 256;
 }
 
 // Replicas of a few thousand particles, at most one per two vertices, leave their vertex buckets

@@ -201,8 +201,8 @@ extern "C" int32_t tissue_step_noalloc(const tissue_mesh* mc, const tissue_param
     auto st = (hipStream_t)stream;
 
     int lanes = 0, block = 0;
-    tissue::tiled_default_shape(1, n, &lanes, &block);
-    const int phys = tissue::phys_lanes(lanes, n, md.nv, block), per = block / phys;
+    tissue::tiled_default_shape(1, n, n, md.nv, &lanes, &block);
+    const int phys = tissue::phys_lanes(lanes, n, n, md.nv, block), per = block / phys;
     const int n_tiles = cdiv(n, per);
     if (n_tiles > kMaxTiles) throw ApiError(TISSUE_E_INVALID_ARG, "tissue_step_noalloc: too many tiles");
     const int sorted = tissue::raw_buckets_for(n, md.nv) ? 0 : 1;

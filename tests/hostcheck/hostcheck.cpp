@@ -121,6 +121,14 @@ void hc_table_entry(const void* nbr, int e, int* out) {
 // 0: a system of these sizes is taken; 1: refused
 int hc_size_refused(long particles, long vertices) { return tissue::size_error(particles, vertices) ? 1 : 0; }
 
+// the default launch shape of the step kernel: lanes, threads per workgroup, physical lanes, LDS bytes at most
+void hc_default_shape(int R, int ntot, int nmax, int nv, int* out) {
+  tissue::tiled_default_shape(R, ntot, nmax, nv, &out[0], &out[1]);
+  out[2] = tissue::phys_lanes(out[0], ntot, nmax, nv, out[1]);
+  out[3] = (int)tissue::step_lds_bytes(nv, tissue::step_areas(nmax, out[1], out[2]), out[0], out[2], false,
+                                       tissue::stage_occupancy(nv, out[1], out[0], out[2]));
+}
+
 // 0: a geodesic table of n entries is built; 1: refused
 int hc_table_refused(int64_t n) {
   try {
