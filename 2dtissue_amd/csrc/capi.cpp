@@ -240,6 +240,7 @@ int32_t tissue_seam_wrap(int32_t n, const double* start_xy, double* end_xy, doub
     b.d = dalloc<double>(n);
     b.q = dalloc<int>(n);
     b.ok = dalloc<int>(n);
+    std::lock_guard<std::mutex> lk(tissue::g_capture_mu);
     HIP_OK(hipMemcpy(b.s, start_xy, 2 * sizeof(double) * (size_t)n, hipMemcpyHostToDevice));
     HIP_OK(hipMemcpy(b.e, end_xy, 2 * sizeof(double) * (size_t)n, hipMemcpyHostToDevice));
     const int mc = max_crossings > 0 ? max_crossings : kDefaultMaxCrossings;

@@ -62,7 +62,9 @@ void dfree(T*& p) {
 
 template <class T>
 void upload(T* dst, const T* src, size_t n) {
-  if (n) HIP_OK(hipMemcpy(dst, src, n * sizeof(T), hipMemcpyHostToDevice));
+  if (n == 0) return;
+  std::lock_guard<std::mutex> lk(tissue::g_capture_mu);
+  HIP_OK(hipMemcpy(dst, src, n * sizeof(T), hipMemcpyHostToDevice));
 }
 
 // largest float f with (double)f < T (strict) or <= T: FP32 thresholds that reproduce the

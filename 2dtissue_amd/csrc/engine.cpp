@@ -668,6 +668,7 @@ int32_t Engine::run_once(const Shape& s, int n_steps, const float* nz, size_t st
       drop_graphs();
     }
     hipGraph_t g = nullptr;
+    std::lock_guard<std::mutex> lk(g_capture_mu);
     HIP_OK(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
     try {
       enqueue(s, n_steps, nz, stride);

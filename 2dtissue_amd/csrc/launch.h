@@ -4,10 +4,15 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <mutex>
 
 #include "device.h"
 
 namespace tissue {
+
+// Held while a graph is captured and around every use of the legacy stream (synchronous copies): the runtime
+// refuses such a use while a stream of any thread is being captured, and ends the capture
+inline std::mutex g_capture_mu;
 
 // fixed-point scale of the order-parameter sums: cos and sin of the headings are summed as
 // integers llrint(value * 2^40), which is exact and associative, so the sums do not depend on the

@@ -14,6 +14,7 @@
 #include <string>
 #include <vector>
 
+#include "launch.h"
 #include "mesh.h"
 #include "uvsolve.h"
 
@@ -219,9 +220,12 @@ bool uv_solve_gpu(const UvSystem& s, std::vector<double>* sol) {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   check(hipStreamSynchronize(st), "sync");
-  check(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal), "capture");
-  enqueue(kBatch);
-  check(hipStreamEndCapture(st, &graph), "capture");
+  {
+    std::lock_guard<std::mutex> lk(g_capture_mu);
+    check(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal), "capture");
+    enqueue(kBatch);
+    check(hipStreamEndCapture(st, &graph), "capture");
+  }
   const hipError_t ie = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
   (void)hipGraphDestroy(graph);
   check(ie, "graph");
