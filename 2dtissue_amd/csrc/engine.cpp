@@ -633,7 +633,7 @@ int32_t Engine::run_once(const Shape& s, int n_steps, const float* nz, size_t st
   if (n_steps < 0) throw ApiError(TISSUE_E_INVALID_ARG, "negative step count");
   if (n_steps == 0) return TISSUE_OK;
   const size_t need_phi = 2 * (size_t)R * n_steps;
-  const size_t need_back = need_phi + (size_t)R;  // + the flag words (2R of 4 bytes) written by flags_end
+  const size_t need_back = need_phi + (size_t)R;  // + the flag words (2R of 4 bytes) written by the run's last kernel
   if (phi_cap < need_back) {
     HIP_OK(hipStreamSynchronize(stream));
     drop_graphs();

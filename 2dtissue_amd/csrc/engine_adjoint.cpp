@@ -5,7 +5,8 @@
 // bytes per particle-step; nothing is recomputed. The reverse pass needs the vertex buckets of every
 // state: the forward pass keeps them when they fit too, else they are made again from the recorded
 // vertex ids, a few states ahead of the reverse pass on a stream of their own. Per reverse step one
-// kernel: the transposed neighbour gather and the factors of the step before.
+// kernel: the transposed neighbour gather and the factors of the step before; two, in a second pass, where the
+// adjoint grows too fast for that (adjoint.hip).
 // Checkpoints (longer runs, and runs that stream or check every step): the tiled step kernel, with the
 // state copied to a checkpoint every ckpt_every steps; in reverse, segment by segment from the last, the
 // segment is recomputed from its checkpoint by the recording variant (bitwise the forward's states),

@@ -3,10 +3,12 @@
 // Per workgroup the replica's state (x, y, cos, sin, theta, vertex id) and the step's vertex
 // buckets live in LDS. Each step:
 //   1. counting sort of the particles by vertex id into a CSR (LDS atomics + block scan);
-//   2. every LANES-lane group updates its particles with the shared particle_step (the
-//      geodesic-table rows and the mesh stay in L2) and stages the new state in a global slice;
-//   3. barrier, then the staged state is copied back to LDS (the update is Jacobi: every
-//      particle reads the old state) and the order parameters are reduced and written.
+//   2. every group of P lanes updates its particles with the shared particle_step (sums laid out over LANES
+//      lanes; the geodesic-table rows and the mesh stay in L2). The update is Jacobi, every particle reads
+//      the old state: the new one of a group's last particle stays in registers, that of its earlier ones
+//      is staged in a global slice;
+//   3. barrier, then the new states go to LDS and the last wave adds up the order parameters, which it
+//      finishes beside the next step's update.
 // Per step only the noise row is read from HBM and the order parameters written; the staged
 // state stays in L2; the state goes back to its HBM home once per launch.
 #include <hip/hip_runtime.h>

@@ -7,8 +7,9 @@
 // neighbour count with butterfly shuffles.
 //
 // The kernel is bound by chains of dependent loads (table row, bucket, particles; cell, candidates, face)
-// and, where the chip is full, by instruction issue; never by bandwidth (2.9 TB/s at most). 2,000 particles
-// 18.7 -> 10.1 us per step, 100,000 274 -> 67, 525,000 in 256 replicas 211 -> 150.
+// and, where the chip is full, by instruction issue; never by bandwidth (2.9 TB/s at most), but for replicas with
+// some 100 vertices per particle and more, where clearing the bucket sets is most of it. 2,000 particles 18.7 -> 10.1 us
+// per step, 100,000 274 -> 66 (the first 50 steps of a run), 525,000 in 256 replicas 211 -> 150.
 // Every lane then runs the per-particle epilogue (speed, Euler, heading, seam wrap) and the lanes
 // split the point-location candidates of the face bucket. Lane 0 writes the SoA outputs, inserts
 // the particle into next step's vertex buckets and contributes to the tile's order-parameter

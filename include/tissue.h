@@ -98,7 +98,8 @@ int32_t tissue_mesh_export(const tissue_mesh* m, double* uv /* nv*2 */, double* 
 int32_t tissue_mesh_save_off(const tissue_mesh* m, const char* path_3d, const char* path_uv);
 
 /* ---- one simulation on the current GPU ---- */
-/* replaces _2DTissue::_2DTissue (2DTissue.cpp:20-111) for the per-step state */
+/* replaces _2DTissue::_2DTissue (2DTissue.cpp:20-111) for the per-step state; up to 2^27 - 1 particles, on a
+ * mesh of fewer than 2^26 UV vertices */
 int32_t tissue_create(const tissue_mesh* m, const tissue_params* p, int32_t n, tissue_sim** out);
 void tissue_destroy(tissue_sim* s);
 /* replaces _2DTissue::start (2DTissue.cpp:117-134): positions uniform by area, headings uniform
@@ -106,6 +107,7 @@ void tissue_destroy(tissue_sim* s);
 int32_t tissue_init_random(tissue_sim* s, uint64_t seed);
 /* state upload; vid == NULL computes vertex ids with the remap, as start() does */
 int32_t tissue_set_state(tissue_sim* s, const float* x, const float* y, const float* theta, const int32_t* vid);
+/* arrays that are NULL are left out, here and below, and not transferred */
 int32_t tissue_get_state(tissue_sim* s, float* x, float* y, float* theta, int32_t* vid);
 /* per-particle outputs of the last step (System/Particle, Struct.h:9-29; 2DTissue.cpp:148-166) */
 int32_t tissue_get_outputs(tissue_sim* s, float* vx, float* vy, float* r3d, int32_t* face, int32_t* nbr);
@@ -222,7 +224,7 @@ typedef struct {
 typedef struct {
   double loss, loss_order, loss_velocity, phi_final;
   double d_tau, d_mu, d_v0, d_k;  /* dloss / d parameter */
-  double forward_ms, reverse_ms;  /* GPU time of the checkpointed forward and of the reverse pass */
+  double forward_ms, reverse_ms;  /* GPU time of the forward and of the reverse pass */
 } tissue_grads;
 /* runs n_steps from the current state (noise from staged row first_row, < 0: none), leaves the
  * final state, and returns the gradients; d_theta0 / d_x0 / d_y0 [n] (may be NULL) are dloss with
