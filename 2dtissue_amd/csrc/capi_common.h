@@ -28,7 +28,10 @@ struct ApiError : std::runtime_error {
 #define HIP_OK(expr)                                                                                  \
   do {                                                                                                \
     hipError_t e_ = (expr);                                                                           \
-    if (e_ != hipSuccess) throw ApiError(TISSUE_E_HIP, std::string(#expr ": ") + hipGetErrorString(e_)); \
+    if (e_ != hipSuccess) {                                                                           \
+      (void)hipGetLastError(); /* reported here, not by the next launch */                            \
+      throw ApiError(TISSUE_E_HIP, std::string(#expr ": ") + hipGetErrorString(e_));                  \
+    }                                                                                                 \
   } while (0)
 
 template <class F>
@@ -58,6 +61,16 @@ template <class T>
 void dfree(T*& p) {
   if (p) (void)hipFree((void*)p);
   p = nullptr;
+}
+
+// p anew for n elements; cap, what it holds, is 0 meanwhile: without the memory p stays empty and is
+// allocated again by the next caller
+template <class T, class C>
+void regrow(T*& p, C& cap, size_t n) {
+  dfree(p);
+  cap = 0;
+  p = dalloc<T>(n);
+  cap = (C)n;
 }
 
 template <class T>

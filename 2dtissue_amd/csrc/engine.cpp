@@ -405,10 +405,10 @@ void Engine::ensure_tiles(const Shape& s) {
   drop_graphs();
   dfree(d_tiles);
   dfree(d_tile_begin);
-  d_tiles = dalloc<TileDesc>(phys.size());
-  upload(d_tiles, phys.data(), phys.size());
   d_tile_begin = dalloc<int>(begin.size());
   upload(d_tile_begin, begin.data(), begin.size());
+  d_tiles = dalloc<TileDesc>(phys.size());  // last: with it the tiles count as there
+  upload(d_tiles, phys.data(), phys.size());
   n_phys = (int)phys.size();
   n_logical = (int)logical.size();
   tiles_key = key;
@@ -422,7 +422,7 @@ void Engine::stage_noise(const float* h, int rows) {
     HIP_OK(hipStreamSynchronize(stream));
     drop_graphs();
     dfree(noise);
-    noise_rows = 0;
+    noise_rows = noise_cap = 0;
     noise = dalloc<float>((size_t)rows * ntot);
     noise_cap = rows;
   }
@@ -464,9 +464,7 @@ const float* Engine::upload_call_noise(const float* h, int n_steps) {
   if (call_noise_cap < need) {
     HIP_OK(hipStreamSynchronize(stream));
     drop_graphs();
-    dfree(call_noise);
-    call_noise = dalloc<float>(need);
-    call_noise_cap = need;
+    regrow(call_noise, call_noise_cap, need);
   }
   if (need <= 2 * back_half) {  // (the call's run is waited for, so the pinned words are free by the next use)
     std::copy(h, h + need, back);
@@ -651,9 +649,7 @@ int32_t Engine::run_once(const Shape& s, int n_steps, const float* nz, size_t st
     if (partial_cap < need) {
       HIP_OK(hipStreamSynchronize(stream));
       drop_graphs();
-      dfree(partial);
-      partial = dalloc<OrderPartial>(need);
-      partial_cap = need;
+      regrow(partial, partial_cap, need);
     }
     const bool occ = stage_occupancy(md.nv, s.block, s.lanes, phys_lanes(s));
     if (occ && !occ_kept) buckets_stale = true;  // the sets were filled without the masks this shape reads

@@ -178,7 +178,6 @@ bool Engine::whole_tape(int T) {
     }
     if (new_sets) alloc_set_slab(a.sets, (int)n_sets);
   } catch (const ApiError&) {  // less memory free than that: checkpoints need less
-    (void)hipGetLastError();
     free_whole_tape();
     return false;
   }
@@ -195,7 +194,8 @@ void Engine::free_tapes() {
 void Engine::adjoint_common() {
   AdjointBuffers& a = adj;
   const size_t N = ntot;
-  if (!a.lr[0]) {
+  if (a.lr[0]) return;
+  try {
     for (int k = 0; k < 2; ++k) { a.lr[k] = dalloc<float2>(N); a.lt[k] = dalloc<float>(N); }
     for (int k = 0; k < 2; ++k) { a.g4[k] = dalloc<float4>(N); a.part[k] = dalloc<float4>(N); }
     a.acc = dalloc<double>(kAdjAcc * N);
@@ -211,6 +211,9 @@ void Engine::adjoint_common() {
       HIP_OK(hipEventCreateWithFlags(&a.ev_rec[k], hipEventDisableTiming));
       HIP_OK(hipEventCreateWithFlags(&a.ev_rev[k], hipEventDisableTiming));
     }
+  } catch (...) {  // all of them or none
+    adjoint_release();
+    throw;
   }
 }
 
@@ -220,6 +223,7 @@ void Engine::adjoint_buffers(int K, int C) {
   free_whole_tape();
   if (C > a.C) {
     dfree(a.ck_xycs); dfree(a.ck_th); dfree(a.ck_vid);
+    a.C = 0;
     a.ck_xycs = dalloc<float4>((size_t)C * N); a.ck_th = dalloc<float>((size_t)C * N); a.ck_vid = dalloc<int>((size_t)C * N);
     a.C = C;
   }
@@ -257,9 +261,7 @@ void Engine::adjoint_buffers(int K, int C) {
     Tape& t = a.tp[k];
     const int np = n_logical * partials_per_tile(kStepMaxBlock);  // written, not read: sized for any shape
     if (t.partial_n < np) {
-      dfree(t.partial);
-      t.partial = dalloc<OrderPartial>(np);
-      t.partial_n = np;
+      regrow(t.partial, t.partial_n, np);
     }
   }
 }
