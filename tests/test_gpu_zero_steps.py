@@ -1,5 +1,5 @@
-"""A call of no steps, with and without noise rows: OK, and state, outputs and order history as they were (a
-driver's empty remainder chunk)."""
+"""A call of no steps, with and without noise rows: OK, and state, outputs and order history as they were (the
+empty remainder of a run in chunks)."""
 import numpy as np
 import pytest
 
